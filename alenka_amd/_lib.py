@@ -143,6 +143,8 @@ SIGNATURES = {
     "aln_eval": (C.c_int, [P, C.POINTER(Col), C.c_int, U32, C.POINTER(Insn), C.c_int, P, U64, P]),
     "aln_apply_perm": (C.c_int, [P, P, P, U64, P]),
     "aln_hash_join": (C.c_int, [P, P, U64, P, U64, P, P, U64, PU64]),
+    "aln_hash_join_count": (C.c_int, [P, P, U64, P, U64, PU64]),
+    "aln_hash_join_pairs": (C.c_int, [P, P, P, U64, PU64]),
     "aln_join_rows": (C.c_int, [P, P, U64, U64, C.c_int, P, U64, PU64]),
     "aln_dict_lookup": (C.c_int, [P, P, U64, P, U64, P]),
     "aln_like_dict": (C.c_int, [P, P, U64, C.c_uint32, C.c_char_p, P]),

@@ -74,6 +74,15 @@ struct aln_ctx {
     uint32_t nsegs[3];
     int64_t mn[3], mx[3];
   } star_rng;
+  // a join counted but not yet written (aln_hash_join_count): arrays in the workspace, so
+  // the next ws_reset ends it
+  struct JoinMatch {
+    bool valid = false;
+    uint64_t np, ntiles, total;
+    const uint32_t *match, *rowid, *srow;
+    const void *runs;
+    const uint64_t *toff;
+  } join;
 };
 
 namespace aln {

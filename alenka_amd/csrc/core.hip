@@ -63,6 +63,7 @@ int ws_alloc(aln_ctx *c, size_t bytes, void **out) {
 }
 
 void ws_reset(aln_ctx *c) {
+  c->join.valid = false;
   c->cur = 0;
   c->off = 0;
 }

@@ -8,10 +8,10 @@
 //   * unique build keys whose range is at most 64 per build row (the primary-key case): a
 //     table with one 8-byte entry per 32 keys (bits present, rank base) and the build rows
 //     in key order;
-//   * other unique keys: an open-addressing table keyed by MurmurHash64A (linear probing), a
-//     slot holding the build row;
-//   * duplicate build keys: the build side is radix-sorted by key (stable, so equal keys
-//     keep ascending row order) and a slot holds a run of equal keys.
+//   * other keys: an open-addressing table keyed by MurmurHash64A (linear probing) of 16-byte
+//     entries, so that a probe step is one load: the key and the build row, or, when build
+//     keys repeat, the bounds of the key's run in the build rows sorted by table slot (a
+//     stable sort, so equal keys keep ascending row order).
 // Pairs come out in probe-row order and, for one probe row, in ascending build-row order;
 // the count pass records each probe row's match so the write pass does not probe again.
 #include <string.h>
@@ -26,144 +26,212 @@ constexpr int J_BLOCK = 256;
 constexpr int J_ITEMS = 8;
 constexpr int J_TILE = J_BLOCK * J_ITEMS;
 
-// Build: slot value = index into `keys` (a build row, or a run of equal keys).
+// ---- hash table ------------------------------------------------------------------------------
+// One entry per distinct build key: x, y = the key, z, w = its build row (unique keys) or the
+// bounds [z, w) of its run in the sorted build rows.  A free entry holds J_NOKEY; a build key
+// of that value has the extra entry at index cap, marked taken by key 0.
+constexpr int64_t J_NOKEY = (int64_t)0x9A7C0F53D1B24E86ull;
+
+__device__ __forceinline__ int64_t je_key(uint4 e) { return (int64_t)((uint64_t)e.y << 32 | e.x); }
+
+// The entry a key's probing starts at, and the key as it is stored.
+__device__ __forceinline__ uint64_t je_start(int64_t key, uint64_t mask, int64_t *stored) {
+  *stored = key == J_NOKEY ? 0 : key;
+  return key == J_NOKEY ? mask + 1 : murmur64a_u64((uint64_t)key, J_SEED) & mask;
+}
+
+__global__ void __launch_bounds__(256) k_join_clear(uint4 *__restrict__ ent, uint64_t n) {
+  const uint4 e = make_uint4((uint32_t)(uint64_t)J_NOKEY, (uint32_t)((uint64_t)J_NOKEY >> 32), 0u, 0u);
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) ent[i] = e;
+}
+
+// Each build row's entry index into sid, its row into the entry it takes; *dup is set when a
+// key comes twice.  Bound by the random entry reads and one CAS per distinct key (24 G/s);
+// the flag is written once per wave and only while it reads as clear (a million atomics on
+// its one address took 6.5 ms for 2M rows, against 0.11 ms for the whole kernel now).
 __global__ void __launch_bounds__(256) k_join_insert(const int64_t *__restrict__ keys, uint64_t n,
-                                                     uint32_t *slot, int64_t *tk, uint64_t cap,
+                                                     uint4 *ent, uint64_t cap, uint64_t *__restrict__ sid,
                                                      uint32_t *dup) {
   const uint64_t mask = cap - 1;
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * 256) {
-    int64_t key = keys[i];
-    uint32_t id = (uint32_t)i;
-    uint64_t h = murmur64a_u64((uint64_t)key, J_SEED) & mask;
+    int64_t st;
+    uint64_t h = je_start(keys[i], mask, &st);
+    bool lost = false;
     for (uint64_t probes = 0; probes <= cap; ++probes) {
-      uint32_t cur = slot[h];
-      if (cur == J_EMPTY) {
-        cur = atomicCAS(&slot[h], J_EMPTY, id);
-        if (cur == J_EMPTY) {
-          tk[h] = key;
+      unsigned long long *slot = reinterpret_cast<unsigned long long *>(ent + h);
+      int64_t cur = (int64_t)__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (cur == J_NOKEY) {
+        cur = (int64_t)atomicCAS(slot, (unsigned long long)J_NOKEY, (unsigned long long)st);
+        if (cur == J_NOKEY) {
+          reinterpret_cast<uint32_t *>(ent + h)[2] = (uint32_t)i;
           break;
         }
       }
-      // occupied: compare with the key of the row (or run) that owns it
-      int64_t other = keys[cur];
-      if (other == key) {
-        atomicExch(dup, 1u);
+      if (cur == st) {
+        lost = true;
         break;
       }
       h = (h + 1) & mask;
     }
+    sid[i] = h;
+    const uint64_t any = __builtin_amdgcn_ballot_w64(lost);
+    if (any && lost && below_count(any) == 0 &&
+        __hip_atomic_load(dup, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+      __hip_atomic_store(dup, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
-__device__ __forceinline__ uint32_t join_find(const uint32_t *__restrict__ slot,
-                                              const int64_t *__restrict__ tk, uint64_t mask,
-                                              int64_t key) {
-  uint64_t h = murmur64a_u64((uint64_t)key, J_SEED) & mask;
-  for (uint64_t probes = 0; probes <= mask; ++probes) {
-    uint32_t s = slot[h];
-    if (s == J_EMPTY) return J_EMPTY;
-    if (tk[h] == key) return s;
-    h = (h + 1) & mask;
-  }
-  return J_EMPTY;
-}
-
-// PASS 0: per probe row, the matching slot value and per-tile pair counts.
-__global__ void __launch_bounds__(J_BLOCK) k_join_probe_count(
-    const int64_t *__restrict__ pk, uint64_t np, const uint32_t *__restrict__ slot,
-    const int64_t *__restrict__ tk, uint64_t mask, const uint32_t *__restrict__ rlen,
-    uint32_t *__restrict__ match, uint32_t *__restrict__ tcount) {
-  uint64_t base = (uint64_t)blockIdx.x * J_TILE;
-  uint32_t s = 0;
-  for (int j = 0; j < J_ITEMS; ++j) {
-    uint64_t p = base + (uint64_t)j * J_BLOCK + threadIdx.x;
-    if (p < np) {
-      uint32_t m = join_find(slot, tk, mask, pk[p]);
-      match[p] = m;
-      if (m != J_EMPTY) s += rlen ? rlen[m] : 1;
-    }
-  }
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
-  __shared__ uint32_t wsum[J_BLOCK / 64];
-  if (__lane_id() == 0) wsum[threadIdx.x / 64] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t t = 0;
-    for (int w = 0; w < J_BLOCK / 64; ++w) t += wsum[w];
-    tcount[blockIdx.x] = t;
+// Repeated keys: the rows sorted by entry (sid ascending); each run's bounds into its entry.
+__global__ void __launch_bounds__(256) k_join_runs(const uint64_t *__restrict__ sid, uint64_t n,
+                                                   uint4 *__restrict__ ent) {
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256) {
+    const uint64_t h = sid[i];
+    uint32_t *e = reinterpret_cast<uint32_t *>(ent + h);
+    if (i == 0 || sid[i - 1] != h) e[2] = (uint32_t)i;
+    if (i + 1 == n || sid[i + 1] != h) e[3] = (uint32_t)(i + 1);
   }
 }
 
-__global__ void __launch_bounds__(J_BLOCK) k_join_probe_write(
-    uint64_t np, const uint32_t *__restrict__ match, const uint32_t *__restrict__ rstart,
-    const uint32_t *__restrict__ rlen, const uint32_t *__restrict__ srow,
-    const uint64_t *__restrict__ toff, uint32_t *__restrict__ out_p, uint32_t *__restrict__ out_b) {
+// Pass 0: each probe row's match (its build row, or J_EMPTY; RUNS: its run's start and
+// length) and the tile's pair count.  The entries of all of a thread's rows are loaded
+// together, round by round, so a wave waits one trip to memory per probe step and not one
+// per row and step.
+template <bool RUNS>
+__global__ void __launch_bounds__(J_BLOCK) k_join_probe(const int64_t *__restrict__ pk, uint64_t np,
+                                                        const uint4 *__restrict__ ent, uint64_t mask,
+                                                        uint32_t *__restrict__ match, uint2 *__restrict__ runs,
+                                                        uint32_t *__restrict__ tcount,
+                                                        uint64_t *__restrict__ tcount64) {
   __shared__ uint64_t wsum[J_BLOCK / 64];
-  // blocked: thread t owns probe rows base + t*ITEMS .. +ITEMS-1 (keeps probe-row order)
-  uint64_t base = (uint64_t)blockIdx.x * J_TILE + (uint64_t)threadIdx.x * J_ITEMS;
-  uint32_t cnt[J_ITEMS], m[J_ITEMS];
-  uint64_t s = 0;
+  const uint64_t base = (uint64_t)blockIdx.x * J_TILE + threadIdx.x;
+  int64_t st[J_ITEMS];
+  uint64_t h[J_ITEMS];
+  uint4 e[J_ITEMS];
+  uint32_t todo = 0;
+#pragma unroll
   for (int j = 0; j < J_ITEMS; ++j) {
-    uint64_t p = base + j;
-    m[j] = p < np ? match[p] : J_EMPTY;
-    cnt[j] = m[j] == J_EMPTY ? 0 : (rlen ? rlen[m[j]] : 1);
-    s += cnt[j];
+    const uint64_t p = base + (uint64_t)j * J_BLOCK;
+    st[j] = p < np ? __builtin_nontemporal_load(pk + p) : 0;
+    if (p < np) todo |= 1u << j;
   }
-  unsigned lane = __lane_id(), wid = threadIdx.x / 64;
-  uint64_t x = s;
-  for (int o = 1; o < 64; o <<= 1) {
-    uint64_t y = __shfl_up(x, o, 64);
-    if (lane >= (unsigned)o) x += y;
-  }
-  if (lane == 63) wsum[wid] = x;
-  __syncthreads();
-  uint64_t before = 0;
-  for (int w = 0; w < (int)wid; ++w) before += wsum[w];
-  uint64_t pos = toff[blockIdx.x] + before + x - s;
-  for (int j = 0; j < J_ITEMS; ++j) {
-    if (!cnt[j]) continue;
-    uint32_t p = (uint32_t)(base + j);
-    if (!rlen) {
-      out_p[pos] = p;
-      out_b[pos] = m[j];
-      ++pos;
-    } else {
-      uint32_t st = rstart[m[j]];
-      for (uint32_t t = 0; t < cnt[j]; ++t, ++pos) {
-        out_p[pos] = p;
-        out_b[pos] = srow[st + t];
+#pragma unroll
+  for (int j = 0; j < J_ITEMS; ++j) h[j] = je_start(st[j], mask, &st[j]);
+  const uint32_t mine = todo;
+  uint32_t hit = 0;
+  while (todo) {  // the table is at most half full: every chain of entries ends in a free one
+#pragma unroll
+    for (int j = 0; j < J_ITEMS; ++j)
+      if (todo >> j & 1) e[j] = ent[h[j]];
+#pragma unroll
+    for (int j = 0; j < J_ITEMS; ++j) {
+      if (!(todo >> j & 1)) continue;
+      const int64_t k = je_key(e[j]);
+      if (k == J_NOKEY || k == st[j]) {
+        todo &= ~(1u << j);
+        if (k == st[j]) hit |= 1u << j;
+      } else {
+        h[j] = (h[j] + 1) & mask;
       }
     }
   }
-}
-
-// Runs mode helpers
-__global__ void k_join_codes(const int64_t *k, uint64_t n, int64_t kmin, uint64_t *code,
-                             uint32_t *row) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256) {
-    code[i] = (uint64_t)k[i] - (uint64_t)kmin;
-    row[i] = (uint32_t)i;
+  uint64_t n = 0;
+#pragma unroll
+  for (int j = 0; j < J_ITEMS; ++j) {
+    if (!(mine >> j & 1)) continue;
+    const uint64_t p = base + (uint64_t)j * J_BLOCK;
+    const bool f = hit >> j & 1;
+    if (RUNS) {
+      const uint32_t len = f ? e[j].w - e[j].z : 0u;
+      runs[p] = make_uint2(f ? e[j].z : 0u, len);
+      n += len;
+    } else {
+      match[p] = f ? e[j].z : J_EMPTY;
+      n += f;
+    }
+  }
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o, 64);
+  if (__lane_id() == 0) wsum[threadIdx.x / 64] = n;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t t = 0;
+    for (int w = 0; w < J_BLOCK / 64; ++w) t += wsum[w];
+    if (RUNS)
+      tcount64[blockIdx.x] = t;
+    else
+      tcount[blockIdx.x] = (uint32_t)t;
   }
 }
-__global__ void k_join_heads(const uint64_t *code, uint64_t n, uint32_t *head) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256)
-    head[i] = i == 0 || code[i] != code[i - 1];
-}
-__global__ void k_join_runs(const uint64_t *code, const uint32_t *head, const uint64_t *pos,
-                            uint64_t n, int64_t kmin, uint32_t *rstart, uint32_t *rlen,
-                            int64_t *rkey) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256) {
-    if (!head[i]) continue;
-    uint64_t r = pos[i];
-    uint64_t e = i + 1;
-    while (e < n && !head[e]) ++e;
-    rstart[r] = (uint32_t)i;
-    rlen[r] = (uint32_t)(e - i);
-    rkey[r] = (int64_t)((uint64_t)kmin + code[i]);
+
+// Pass 1 of repeated keys: a tile's pairs.  The probe rows' first pair numbers stand in LDS;
+// each thread takes pairs by number and finds its probe row by a binary search there, so the
+// stores to the output are whole lines and a long run is spread over the block (a thread per
+// probe row, storing its own pairs one by one, took 371 us for 9.6M pairs).
+__global__ void __launch_bounds__(J_BLOCK) k_join_expand(const uint2 *__restrict__ runs, uint64_t np,
+                                                         const uint32_t *__restrict__ srow,
+                                                         const uint64_t *__restrict__ toff,
+                                                         uint32_t *__restrict__ out_p, uint32_t *__restrict__ out_b) {
+  __shared__ uint64_t off[J_TILE];
+  __shared__ uint32_t start[J_TILE];
+  __shared__ uint64_t wsum[J_BLOCK / 64];
+  const uint64_t t0 = (uint64_t)blockIdx.x * J_TILE;
+  const unsigned lane = __lane_id(), wid = threadIdx.x / 64;
+  // wave w holds the tile's rows w * 512 .. + 511, a row of 64 per load
+  uint2 r[J_ITEMS];
+#pragma unroll
+  for (int j = 0; j < J_ITEMS; ++j) {
+    const uint64_t p = t0 + (uint64_t)wid * (64 * J_ITEMS) + (uint64_t)j * 64 + lane;
+    r[j] = p < np ? runs[p] : make_uint2(0u, 0u);
+  }
+  uint64_t carry = 0, ex[J_ITEMS];
+#pragma unroll
+  for (int j = 0; j < J_ITEMS; ++j) {
+    uint64_t x = r[j].y;
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint64_t y = __shfl_up(x, o, 64);
+      if (lane >= (unsigned)o) x += y;
+    }
+    ex[j] = carry + x - r[j].y;
+    carry += __shfl(x, 63, 64);
+  }
+  if (lane == 0) wsum[wid] = carry;
+  __syncthreads();
+  uint64_t before = 0, total = 0;
+  for (int w = 0; w < J_BLOCK / 64; ++w) {
+    before += w < (int)wid ? wsum[w] : 0;
+    total += wsum[w];
+  }
+#pragma unroll
+  for (int j = 0; j < J_ITEMS; ++j) {
+    const uint32_t i = wid * (64 * J_ITEMS) + j * 64 + lane;
+    off[i] = before + ex[j];
+    start[i] = r[j].x;
+  }
+  __syncthreads();
+  const uint64_t o0 = toff[blockIdx.x];
+  constexpr int U = 4;
+  for (uint64_t q0 = threadIdx.x; q0 < total; q0 += (uint64_t)U * J_BLOCK) {
+    uint32_t i[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // the last row whose first pair number is <= q
+      const uint64_t q = q0 + (uint64_t)u * J_BLOCK;
+      i[u] = 0;
+#pragma unroll
+      for (uint32_t s = J_TILE / 2; s > 0; s >>= 1)
+        if (off[i[u] + s] <= q) i[u] += s;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t q = q0 + (uint64_t)u * J_BLOCK;
+      b[u] = q < total ? srow[start[i[u]] + (uint32_t)(q - off[i[u]])] : 0u;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint64_t q = q0 + (uint64_t)u * J_BLOCK;
+      if (q >= total) continue;
+      out_p[o0 + q] = (uint32_t)(t0 + i[u]);
+      out_b[o0 + q] = b[u];
+    }
   }
 }
 
@@ -373,23 +441,40 @@ __global__ void __launch_bounds__(J_BLOCK) k_jd_write(const uint32_t *__restrict
   }
 }
 
-// The pairs from each probe row's build row (match) and the tiles' pair counts.
-// rowid: as for k_jd_write.
-static int join_write_pairs(aln_ctx *c, const uint32_t *match, const uint32_t *rowid, uint64_t np,
-                            const uint32_t *tcount, uint64_t *toff, uint64_t ntiles, uint32_t *d_probe_idx,
-                            uint32_t *d_build_idx, uint64_t cap, uint64_t *h_npairs) {
-  uint64_t total = 0;
-  ALN_TRY(exclusive_scan_u32(c, tcount, ntiles, toff, &total));
+// The counted join waits in the context for its pairs to be written (join_pairs).
+static int join_counted(aln_ctx *c, uint64_t np, uint64_t ntiles, const uint32_t *match, const uint32_t *rowid,
+                        const uint2 *runs, const uint32_t *srow, const uint64_t *toff, uint64_t total,
+                        uint64_t *h_npairs) {
+  aln_ctx::JoinMatch &m = c->join;
+  m.valid = true;
+  m.np = np;
+  m.ntiles = ntiles;
+  m.total = total;
+  m.match = match;
+  m.rowid = rowid;
+  m.runs = runs;
+  m.srow = srow;
+  m.toff = toff;
   *h_npairs = total;
-  if (total > cap)
-    return set_error(ALN_E_CAPACITY, "aln_hash_join: %llu pairs, capacity %llu", (unsigned long long)total,
+  return ALN_OK;
+}
+
+static int join_pairs(aln_ctx *c, uint32_t *d_probe_idx, uint32_t *d_build_idx, uint64_t cap, uint64_t *h_npairs) {
+  const aln_ctx::JoinMatch &m = c->join;
+  *h_npairs = m.total;
+  if (m.total > cap)
+    return set_error(ALN_E_CAPACITY, "aln_hash_join: %llu pairs, capacity %llu", (unsigned long long)m.total,
                      (unsigned long long)cap);
-  if (total == 0) return ALN_OK;
+  if (m.total == 0) return ALN_OK;
   ALN_REQUIRE(d_probe_idx && d_build_idx, "aln_hash_join: no output buffers");
   {
     ProfScope p(c, "join_write");
-    hipLaunchKernelGGL(k_jd_write, dim3((unsigned)ntiles), dim3(J_BLOCK), 0, c->stream, match, np, rowid,
-                       (const uint64_t *)toff, d_probe_idx, d_build_idx);
+    if (m.runs)
+      hipLaunchKernelGGL(k_join_expand, dim3((unsigned)m.ntiles), dim3(J_BLOCK), 0, c->stream,
+                         static_cast<const uint2 *>(m.runs), m.np, m.srow, m.toff, d_probe_idx, d_build_idx);
+    else
+      hipLaunchKernelGGL(k_jd_write, dim3((unsigned)m.ntiles), dim3(J_BLOCK), 0, c->stream, m.match, m.np, m.rowid,
+                         m.toff, d_probe_idx, d_build_idx);
   }
   ALN_TRY(check_launch("join_write"));
   ALN_HIP(hipStreamSynchronize(c->stream));
@@ -398,8 +483,7 @@ static int join_write_pairs(aln_ctx *c, const uint32_t *match, const uint32_t *r
 
 // The dense path; *taken = false (and nothing else done) when the build keys repeat.
 static int join_dense(aln_ctx *c, const int64_t *bk, uint64_t nb, const int64_t *pk, uint64_t np, int64_t kmin,
-                      uint64_t range, uint32_t *d_probe_idx, uint32_t *d_build_idx, uint64_t cap,
-                      uint64_t *h_npairs, bool *taken) {
+                      uint64_t range, uint64_t *h_npairs, bool *taken) {
   *taken = false;
   const uint64_t ntiles = (np + J_TILE - 1) / J_TILE;
   uint32_t *match, *tcount;
@@ -443,119 +527,113 @@ static int join_dense(aln_ctx *c, const int64_t *bk, uint64_t nb, const int64_t 
                        kmin, range, match, tcount);
   }
   ALN_TRY(check_launch("join_dense_match"));
-  return join_write_pairs(c, match, rowid, np, tcount, toff, ntiles, d_probe_idx, d_build_idx, cap, h_npairs);
+  uint64_t total = 0;
+  ALN_TRY(exclusive_scan_u32(c, tcount, ntiles, toff, &total));
+  return join_counted(c, np, ntiles, match, rowid, nullptr, nullptr, toff, total, h_npairs);
 }
 
-}  // namespace aln
-
-using namespace aln;
-
-extern "C" int aln_hash_join(aln_ctx *c, const int64_t *d_build_keys, uint64_t nbuild,
-                             const int64_t *d_probe_keys, uint64_t nprobe, uint32_t *d_probe_idx,
-                             uint32_t *d_build_idx, uint64_t cap, uint64_t *h_npairs) {
-  ALN_REQUIRE(c && h_npairs, "aln_hash_join: bad arguments");
-  ALN_REQUIRE(nbuild < 0xFFFFFFFFull && nprobe < 0xFFFFFFFFull, "aln_hash_join: more than 2^32-1 rows");
-  ALN_REQUIRE((nbuild == 0 || d_build_keys) && (nprobe == 0 || d_probe_keys),
-              "aln_hash_join: NULL keys");
+// Every probe row's match and the number of pairs, left in the context's workspace.
+static int join_count(aln_ctx *c, const int64_t *d_build_keys, uint64_t nbuild, const int64_t *d_probe_keys,
+                      uint64_t nprobe, uint64_t *h_npairs) {
   ws_reset(c);
   *h_npairs = 0;
-  if (nbuild == 0 || nprobe == 0) return ALN_OK;
+  if (nbuild == 0 || nprobe == 0)
+    return join_counted(c, nprobe, 0, nullptr, nullptr, nullptr, nullptr, nullptr, 0, h_npairs);
   // dense unique build keys: the bitmap + rank index
   int64_t bmin, bmax;
   ALN_TRY(minmax_i64(c, d_build_keys, nbuild, &bmin, &bmax));
   const uint64_t brange = (uint64_t)bmax - (uint64_t)bmin + 1;
   if (brange != 0 && brange <= (1ull << 31) && brange <= JD_DENSITY * nbuild) {
     bool taken = false;
-    ALN_TRY(join_dense(c, d_build_keys, nbuild, d_probe_keys, nprobe, bmin, brange, d_probe_idx, d_build_idx,
-                       cap, h_npairs, &taken));
+    ALN_TRY(join_dense(c, d_build_keys, nbuild, d_probe_keys, nprobe, bmin, brange, h_npairs, &taken));
     if (taken) return ALN_OK;
     ws_reset(c);
   }
-  uint64_t tcap = next_pow2(2 * nbuild < 1024 ? 1024 : 2 * nbuild);
-  uint32_t *slot, *dup;
-  int64_t *tk;
-  ALN_TRY(ws(c, tcap, &slot));
-  ALN_TRY(ws(c, tcap, &tk));
+  const uint64_t tcap = next_pow2(2 * nbuild < 1024 ? 1024 : 2 * nbuild);
+  uint32_t *dup, *srow = nullptr;
+  uint4 *ent;
+  uint64_t *sid;
+  ALN_TRY(ws(c, tcap + 1, &ent));
+  ALN_TRY(ws(c, nbuild, &sid));
   ALN_TRY(ws(c, 1, &dup));
-  ALN_TRY(fill_u32(c, slot, tcap, J_EMPTY));
+  hipLaunchKernelGGL(k_join_clear, dim3(grid_for(tcap + 1, 1024, 65536)), dim3(256), 0, c->stream, ent, tcap + 1);
+  ALN_TRY(check_launch("join_clear"));
   ALN_TRY(fill_u32(c, dup, 1, 0));
   {
     ProfScope p(c, "join_build");
     hipLaunchKernelGGL(k_join_insert, dim3(grid_for(nbuild, 256, 65536)), dim3(256), 0, c->stream,
-                       d_build_keys, nbuild, slot, tk, tcap, dup);
+                       d_build_keys, nbuild, ent, tcap, sid, dup);
   }
   ALN_TRY(check_launch("join_build"));
   uint32_t hdup = 0;
   ALN_TRY(copy_to_host(c, &hdup, dup, 4));
-  uint32_t *rstart = nullptr, *rlen = nullptr, *srow = nullptr;
-  if (hdup) {
-    // runs mode: stable sort of the build side by key, one slot per run of equal keys
-    int64_t kmin, kmax;
-    ALN_TRY(minmax_i64(c, d_build_keys, nbuild, &kmin, &kmax));
-    uint64_t *code;
-    uint32_t *head;
-    uint64_t *pos;
-    ALN_TRY(ws(c, nbuild, &code));
+  if (hdup) {  // the rows of one key side by side, in row order
     ALN_TRY(ws(c, nbuild, &srow));
-    ALN_TRY(ws(c, nbuild, &head));
-    ALN_TRY(ws(c, nbuild, &pos));
-    hipLaunchKernelGGL(k_join_codes, dim3(grid_for(nbuild, 256, 65536)), dim3(256), 0, c->stream,
-                       d_build_keys, nbuild, kmin, code, srow);
-    ALN_TRY(check_launch("join_codes"));
-    ALN_TRY(radix_sort_pairs(c, code, srow, nbuild, bits_for_range_u((uint64_t)kmax - (uint64_t)kmin)));
-    hipLaunchKernelGGL(k_join_heads, dim3(grid_for(nbuild, 256, 65536)), dim3(256), 0, c->stream, code,
-                       nbuild, head);
-    ALN_TRY(check_launch("join_heads"));
-    uint64_t nruns = 0;
-    ALN_TRY(exclusive_scan_u32(c, head, nbuild, pos, &nruns));
-    int64_t *rkey;
-    ALN_TRY(ws(c, nruns, &rstart));
-    ALN_TRY(ws(c, nruns, &rlen));
-    ALN_TRY(ws(c, nruns, &rkey));
-    hipLaunchKernelGGL(k_join_runs, dim3(grid_for(nbuild, 256, 65536)), dim3(256), 0, c->stream, code,
-                       head, pos, nbuild, kmin, rstart, rlen, rkey);
-    ALN_TRY(check_launch("join_runs"));
-    ALN_TRY(fill_u32(c, slot, tcap, J_EMPTY));
-    {
-      ProfScope p(c, "join_build");
-      hipLaunchKernelGGL(k_join_insert, dim3(grid_for(nruns, 256, 65536)), dim3(256), 0, c->stream,
-                         (const int64_t *)rkey, nruns, slot, tk, tcap, dup);
-    }
+    ALN_TRY(iota_u32(c, srow, nbuild));
+    ALN_TRY(radix_sort_pairs(c, sid, srow, nbuild, bits_for_range_u(tcap)));
+    ProfScope p(c, "join_build");
+    hipLaunchKernelGGL(k_join_runs, dim3(grid_for(nbuild, 256, 65536)), dim3(256), 0, c->stream,
+                       (const uint64_t *)sid, nbuild, ent);
     ALN_TRY(check_launch("join_build_runs"));
   }
-  uint64_t ntiles = (nprobe + J_TILE - 1) / J_TILE;
-  uint32_t *match, *tcount;
-  uint64_t *toff;
-  ALN_TRY(ws(c, nprobe, &match));
-  ALN_TRY(ws(c, ntiles, &tcount));
+  const uint64_t ntiles = (nprobe + J_TILE - 1) / J_TILE;
+  uint32_t *match = nullptr, *tcount = nullptr;
+  uint2 *runs = nullptr;
+  uint64_t *tcount64 = nullptr, *toff, total = 0;
   ALN_TRY(ws(c, ntiles, &toff));
+  if (hdup) {
+    ALN_TRY(ws(c, nprobe, &runs));
+    ALN_TRY(ws(c, ntiles, &tcount64));
+  } else {
+    ALN_TRY(ws(c, nprobe, &match));
+    ALN_TRY(ws(c, ntiles, &tcount));
+  }
   {
     ProfScope p(c, "join_probe");
-    hipLaunchKernelGGL(k_join_probe_count, dim3((unsigned)ntiles), dim3(J_BLOCK), 0, c->stream,
-                       d_probe_keys, nprobe, slot, tk, tcap - 1, rlen, match, tcount);
+    if (hdup)
+      hipLaunchKernelGGL(k_join_probe<true>, dim3((unsigned)ntiles), dim3(J_BLOCK), 0, c->stream, d_probe_keys,
+                         nprobe, (const uint4 *)ent, tcap - 1, match, runs, tcount, tcount64);
+    else
+      hipLaunchKernelGGL(k_join_probe<false>, dim3((unsigned)ntiles), dim3(J_BLOCK), 0, c->stream, d_probe_keys,
+                         nprobe, (const uint4 *)ent, tcap - 1, match, runs, tcount, tcount64);
   }
-  ALN_TRY(check_launch("join_probe_count"));
-  // unique keys: match holds the build row itself, written out through LDS
-  if (!rlen)
-    return join_write_pairs(c, match, nullptr, nprobe, tcount, toff, ntiles, d_probe_idx, d_build_idx, cap,
-                            h_npairs);
-  uint64_t total = 0;
-  ALN_TRY(exclusive_scan_u32(c, tcount, ntiles, toff, &total));
-  *h_npairs = total;
-  if (total > cap)
-    return set_error(ALN_E_CAPACITY, "aln_hash_join: %llu pairs, capacity %llu",
-                     (unsigned long long)total, (unsigned long long)cap);
-  if (total == 0) return ALN_OK;
-  ALN_REQUIRE(d_probe_idx && d_build_idx, "aln_hash_join: no output buffers");
-  {
-    ProfScope p(c, "join_write");
-    hipLaunchKernelGGL(k_join_probe_write, dim3((unsigned)ntiles), dim3(J_BLOCK), 0, c->stream, nprobe,
-                       match, rstart, rlen, srow, toff, d_probe_idx, d_build_idx);
-  }
-  ALN_TRY(check_launch("join_probe_write"));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  ALN_TRY(check_launch("join_probe"));
+  if (hdup)
+    ALN_TRY(exclusive_scan_u64(c, tcount64, ntiles, toff, &total));
+  else
+    ALN_TRY(exclusive_scan_u32(c, tcount, ntiles, toff, &total));
+  return join_counted(c, nprobe, ntiles, match, nullptr, runs, srow, toff, total, h_npairs);
 }
+
+}  // namespace aln
+
+using namespace aln;
+
+extern "C" {
+
+int aln_hash_join_count(aln_ctx *c, const int64_t *d_build_keys, uint64_t nbuild, const int64_t *d_probe_keys,
+                        uint64_t nprobe, uint64_t *h_npairs) {
+  ALN_REQUIRE(c && h_npairs, "aln_hash_join: bad arguments");
+  ALN_REQUIRE(nbuild < 0xFFFFFFFFull && nprobe < 0xFFFFFFFFull, "aln_hash_join: more than 2^32-1 rows");
+  ALN_REQUIRE((nbuild == 0 || d_build_keys) && (nprobe == 0 || d_probe_keys),
+              "aln_hash_join: NULL keys");
+  return join_count(c, d_build_keys, nbuild, d_probe_keys, nprobe, h_npairs);
+}
+
+int aln_hash_join_pairs(aln_ctx *c, uint32_t *d_probe_idx, uint32_t *d_build_idx, uint64_t cap, uint64_t *h_npairs) {
+  ALN_REQUIRE(c && h_npairs, "aln_hash_join_pairs: bad arguments");
+  ALN_REQUIRE(c->join.valid, "aln_hash_join_pairs: no counted join (another call came between)");
+  return join_pairs(c, d_probe_idx, d_build_idx, cap, h_npairs);
+}
+
+int aln_hash_join(aln_ctx *c, const int64_t *d_build_keys, uint64_t nbuild,
+                  const int64_t *d_probe_keys, uint64_t nprobe, uint32_t *d_probe_idx,
+                  uint32_t *d_build_idx, uint64_t cap, uint64_t *h_npairs) {
+  ALN_TRY(aln_hash_join_count(c, d_build_keys, nbuild, d_probe_keys, nprobe, h_npairs));
+  return join_pairs(c, d_probe_idx, d_build_idx, cap, h_npairs);
+}
+
+}  // extern "C"
 
 namespace aln {
 

@@ -215,20 +215,24 @@ def apply_perm(ctx, vals, perm):
 
 
 def hash_join(ctx, build_keys, probe_keys, cap=None):
-    """(probe_idx, build_idx) int32 tensors in probe-row order."""
+    """(probe_idx, build_idx) int32 tensors in probe-row order.  cap: pairs to allocate for
+    at first (by default the outputs are sized by the count)."""
     nb, npb = build_keys.numel(), probe_keys.numel()
-    cap = max(npb, 1) if cap is None else cap
-    while True:
-        pi = ctx.empty(cap, torch.int32)
-        bi = ctx.empty(cap, torch.int32)
-        cnt = C.c_uint64()
+    cnt = C.c_uint64()
+    if cap is None:
+        L.check(ctx.lib.aln_hash_join_count(ctx.h, _p(build_keys), nb, _p(probe_keys), npb, C.byref(cnt)),
+                "aln_hash_join_count")
+        cap = cnt.value
+        rc = L.ALN_E_CAPACITY
+    else:
+        pi, bi = ctx.empty(cap, torch.int32), ctx.empty(cap, torch.int32)
         rc = ctx.lib.aln_hash_join(ctx.h, _p(build_keys), nb, _p(probe_keys), npb, _p(pi), _p(bi), cap,
                                    C.byref(cnt))
-        if rc == L.ALN_E_CAPACITY and cnt.value > cap:
-            cap = cnt.value
-            continue
-        L.check(rc, "aln_hash_join")
-        return pi[: cnt.value], bi[: cnt.value]
+    if rc == L.ALN_E_CAPACITY:  # the matches are found: write them into outputs of their size
+        pi, bi = ctx.empty(cnt.value, torch.int32), ctx.empty(cnt.value, torch.int32)
+        rc = ctx.lib.aln_hash_join_pairs(ctx.h, _p(pi), _p(bi), cnt.value, C.byref(cnt))
+    L.check(rc, "aln_hash_join")
+    return pi[: cnt.value], bi[: cnt.value]
 
 
 def like_dict(ctx, entries, width, pattern):

@@ -1166,21 +1166,11 @@ static int join_pair(const std::string &name, const std::string &left, const std
   DBufP lk, rk;
   TRY(plain_copy(lv.cols[eqs[0].first], lv.nrows, lv.seg_rows, &lk));
   TRY(plain_copy(rv.cols[eqs[0].second], rv.nrows, rv.seg_rows, &rk));
-  uint64_t cap = lv.nrows ? lv.nrows : 1, np = 0;
-  DBufP pi, bi;
-  for (;;) {
-    pi = dalloc(4 * cap);
-    bi = dalloc(4 * cap);
-    if (!pi || !bi) return fail(ALN_E_NOMEM, "device allocation failed");
-    int rc = aln_hash_join(g_ctx, (const int64_t *)rk->p, rv.nrows, (const int64_t *)lk->p, lv.nrows,
-                           (uint32_t *)pi->p, (uint32_t *)bi->p, cap, &np);
-    if (rc == ALN_E_CAPACITY && np > cap) {
-      cap = np;
-      continue;
-    }
-    ALN(rc, "join");
-    break;
-  }
+  uint64_t np = 0;
+  ALN(aln_hash_join_count(g_ctx, (const int64_t *)rk->p, rv.nrows, (const int64_t *)lk->p, lv.nrows, &np), "join");
+  DBufP pi = dalloc(4 * (np ? np : 1)), bi = dalloc(4 * (np ? np : 1));
+  if (!pi || !bi) return fail(ALN_E_NOMEM, "device allocation failed");
+  ALN(aln_hash_join_pairs(g_ctx, (uint32_t *)pi->p, (uint32_t *)bi->p, np, &np), "join");
   if (kind != 'I') return semi_anti(name, kind, lv, rv, eqs, pi, bi, np, lneed, rneed);
   // gather every kept column through the pairs
   auto gather_all = [&](const View &v, const std::set<std::string> &cols, const DBufP &idx, uint64_t n,

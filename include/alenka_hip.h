@@ -247,6 +247,16 @@ int aln_hash_join(aln_ctx *ctx, const int64_t *d_build_keys, uint64_t nbuild,
                   const int64_t *d_probe_keys, uint64_t nprobe, uint32_t *d_probe_idx,
                   uint32_t *d_build_idx, uint64_t cap, uint64_t *h_npairs);
 
+/* The same join in two calls, for callers that size their output by the pair count: the
+ * first finds every match and returns the number of pairs, the second writes them (cap >=
+ * that number).  The matches stay in the context's workspace in between (a failed
+ * aln_hash_join with ALN_E_CAPACITY leaves them there too): the next other call that takes
+ * workspace of this context ends them, and aln_hash_join_pairs then returns ALN_E_ARG. */
+int aln_hash_join_count(aln_ctx *ctx, const int64_t *d_build_keys, uint64_t nbuild,
+                        const int64_t *d_probe_keys, uint64_t nprobe, uint64_t *h_npairs);
+int aln_hash_join_pairs(aln_ctx *ctx, uint32_t *d_probe_idx, uint32_t *d_build_idx, uint64_t cap,
+                        uint64_t *h_npairs);
+
 /* Semi / anti reduction of a join (replaces sort + unique and set_difference in
  * operators.cu:1357-1399 and 1473-1480): d_idx holds the row indices (< nrows) one side
  * contributes to the join's pairs, duplicates allowed.  Writes the rows of that side that

@@ -330,6 +330,39 @@ def test_hash_join(ctx, case):
         assert sorted(zip(ol.tolist(), orr.tolist())) == sorted(zip(pi.tolist(), bi.tolist()))
 
 
+J_NOKEY = 0x9A7C0F53D1B24E86 - (1 << 64)  # the join table's mark of a free entry
+
+
+@pytest.mark.parametrize("nb,npb,distinct", [(1, 1, 1), (3, 2049, 1), (2048, 2047, 300), (70001, 6145, 9000),
+                                             (5000, 100003, 2)])
+def test_hash_join_sparse_keys(ctx, nb, npb, distinct):
+    """Build keys spread over the int64 range, repeated (runs of 1 to nb rows, more pairs than
+    probe rows) and unique, with the extremes and the free-entry mark among them, at the edges
+    of the 2048-row probe tiles; in one call with a short capacity, and in two."""
+    import ctypes as C
+
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(nb + npb)
+    pool = np.unique(np.concatenate([r.integers(-(1 << 62), 1 << 62, max(distinct, nb)),
+                                     [J_NOKEY, 0, -(1 << 63), (1 << 63) - 1]]))
+    pool = r.permutation(pool)[-max(distinct, nb):]
+    pool[0] = J_NOKEY if J_NOKEY not in pool else pool[0]
+    for build in (pool[r.integers(0, distinct, nb)], pool[:nb]):
+        probe = np.concatenate([pool, r.integers(-(1 << 62), 1 << 62, 8), [J_NOKEY]])[r.integers(0, distinct + 9, npb)]
+        order = np.argsort(build, kind="stable")
+        lo, hi = (np.searchsorted(build[order], probe, side=x) for x in ("left", "right"))
+        want_p = np.repeat(np.arange(npb), hi - lo)
+        want_b = np.concatenate([order[a:b] for a, b in zip(lo, hi)]) if npb else order[:0]
+        db, dp = dev(ctx, build), dev(ctx, probe)
+        for cap in (None, 1):
+            pi, bi = D.hash_join(ctx, db, dp, cap=cap)
+            assert np.array_equal(host(pi), want_p) and np.array_equal(host(bi), want_b)
+    D.join_rows(ctx, pi, npb, False)  # takes the workspace: the counted join is over
+    n = C.c_uint64()
+    assert ctx.lib.aln_hash_join_pairs(ctx.h, D._p(pi), D._p(bi), pi.numel(), C.byref(n)) == L.ALN_E_ARG
+
+
 @pytest.mark.parametrize("width", [3, 8, 25])
 def test_like_dict_matches_oracle(ctx, width):
     """LIKE over a dictionary on the device against the oracle's restatement of gpu_regex
