@@ -1112,6 +1112,282 @@ int topk_codes(aln_ctx *c, uint64_t *code, uint32_t *idx, uint64_t n, uint32_t k
   }
 }
 
+// ---- top-k: candidates by a bound on the first key -------------------------------------------
+// Sorting every tile (above) reads and compares all rows log^2 times: 1.6 of 2.0 ms for the
+// first 100 of 50M rows.  The k-th smallest of the minima of disjoint chunks of rows bounds the
+// k-th smallest of all rows, so one pass over the first key (the chunk minima, HBM-bound)
+// leaves about k candidates when that key is spread, and all keys are compared only among them:
+//   k_tk_min      a wave per chunk of 64 to 1024 rows: its minimum code
+//   k_tk_bound    one block: the k-th smallest of (up to 4096 strided groups of) the minima
+//   k_tk_collect  the rows within the bound, read again only in chunks that have one
+//   k_tk_final    one block sorts up to tf_max candidates by all keys and row number
+// With one key, equal codes are ordered by row, so the bound is a (code, chunk) pair and rows
+// of the bound's code count only up to its chunk: at most k chunks of candidates whatever the
+// values.  With more keys every row that ties on the first is a candidate; when those are too
+// many (a flag), the keys' codes are written out and bounded as one key.  Candidates too many
+// for k_tk_final go through the tile sort.
+constexpr uint32_t TK_GROUPS = 4096;
+constexpr uint32_t TK_CAND = 1u << 20;
+constexpr int TF_BLOCK = 1024;
+
+// Order-preserving unsigned code of a key value over the whole int64 range; of a code (desc
+// TK_RAW) itself.
+constexpr int TK_RAW = 2;
+__device__ __forceinline__ uint64_t tk_code(int64_t v, int desc) {
+  if (desc == TK_RAW) return (uint64_t)v;
+  const uint64_t c = (uint64_t)v ^ 0x8000000000000000ull;
+  return desc ? ~c : c;
+}
+
+// Chunk c: rows [c * 64 * U, +64 * U).
+template <int U>
+__global__ void __launch_bounds__(256) k_tk_min(const int64_t *__restrict__ key, int desc, uint64_t n,
+                                                uint32_t nchunks, uint64_t *__restrict__ cmin) {
+  const uint32_t c = blockIdx.x * 4 + threadIdx.x / 64;
+  if (c >= nchunks) return;
+  const uint64_t i0 = (uint64_t)c * (64 * U) + __lane_id();
+  uint64_t m = ~0ull;
+  int64_t v[U];
+  // the last chunk's missing rows repeat its first row
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    v[u] = __builtin_nontemporal_load(key + (i0 + 64 * u < n ? i0 + 64 * u : (uint64_t)c * (64 * U)));
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint64_t x = tk_code(v[u], desc);
+    m = x < m ? x : m;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const uint64_t x = __shfl_xor(m, o, 64);
+    m = x < m ? x : m;
+  }
+  if (__lane_id() == 0) cmin[c] = m;
+}
+
+// ctl[0], ctl[1] = code and chunk of the k-th smallest group minimum (k <= min(nchunks,
+// TK_GROUPS)), ctl[2] = 0 (the candidate count).  Groups are strided so that rows in order
+// spread over them.
+__global__ void __launch_bounds__(TF_BLOCK) k_tk_bound(const uint64_t *__restrict__ cmin, uint32_t nchunks,
+                                                       uint32_t k, uint64_t *__restrict__ ctl) {
+  __shared__ uint64_t s[TK_GROUPS];
+  __shared__ uint32_t sc[TK_GROUPS];
+  for (uint32_t g = threadIdx.x; g < TK_GROUPS; g += TF_BLOCK) {
+    uint64_t m = ~0ull;
+    uint32_t at = g < nchunks ? g : 0xFFFFFFFFu;
+    for (uint32_t c = g; c < nchunks; c += TK_GROUPS)
+      if (cmin[c] < m) {
+        m = cmin[c];
+        at = c;
+      }
+    s[g] = m;
+    sc[g] = at;
+  }
+  uint32_t p2 = 64;
+  while (p2 < nchunks && p2 < TK_GROUPS) p2 <<= 1;
+  __syncthreads();
+  for (uint32_t size = 2; size <= p2; size <<= 1)
+    for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+      for (uint32_t t = threadIdx.x; t < p2 / 2; t += TF_BLOCK) {
+        const uint32_t lo = 2 * t - (t & (stride - 1)), hi = lo + stride;
+        const uint64_t a = s[lo], b = s[hi];
+        const uint32_t ca = sc[lo], cb = sc[hi];
+        if ((a > b || (a == b && ca > cb)) == ((lo & size) == 0)) {
+          s[lo] = b;
+          s[hi] = a;
+          sc[lo] = cb;
+          sc[hi] = ca;
+        }
+      }
+      __syncthreads();
+    }
+  if (threadIdx.x == 0) {
+    ctl[0] = s[k - 1];
+    ctl[1] = sc[k - 1];
+    ctl[2] = 0;
+  }
+}
+
+// by_row: the key is the only one (see above).
+template <int U>
+__global__ void __launch_bounds__(256) k_tk_collect(const int64_t *__restrict__ key, int desc, uint64_t n,
+                                                    uint32_t nchunks, int by_row, const uint64_t *__restrict__ cmin,
+                                                    uint64_t *ctl, uint32_t *__restrict__ cand) {
+  const uint32_t c = blockIdx.x * 4 + threadIdx.x / 64;
+  if (c >= nchunks) return;
+  uint64_t bound = ctl[0];
+  if (cmin[c] > bound) return;
+  if (by_row && c > ctl[1]) {  // past the bound's chunk only smaller codes count
+    if (cmin[c] == bound) return;
+    --bound;
+  }
+  const uint64_t i0 = (uint64_t)c * (64 * U) + __lane_id();
+  uint64_t in[U];
+  uint32_t cnt = 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint64_t i = i0 + 64 * u;
+    in[u] = __builtin_amdgcn_ballot_w64(i < n && tk_code(key[i < n ? i : 0], desc) <= bound);
+    cnt += (uint32_t)__popcll(in[u]);
+  }
+  unsigned long long pos = 0;
+  if (__lane_id() == 0) pos = atomicAdd(reinterpret_cast<unsigned long long *>(ctl + 2), (unsigned long long)cnt);
+  pos = __shfl(pos, 0, 64);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    if (in[u] >> __lane_id() & 1) {
+      const uint64_t q = pos + below_count(in[u]);
+      if (q < TK_CAND) cand[q] = (uint32_t)(i0 + 64 * u);
+    }
+    pos += (uint32_t)__popcll(in[u]);
+  }
+}
+
+// The candidates k_tk_final sorts in LDS (8 bytes per key and 4 for the row each).
+static inline uint32_t tf_max(int nkeys) { return nkeys <= 3 ? 2048u : 1024u; }
+
+// The first k of the rows cand[0, m) (cand NULL: rows 0..m-1) by keys and row number, m =
+// *count (count NULL: n); nothing when m exceeds `most`.
+struct TfArgs {
+  const int64_t *k[ALN_MAX_KEYS];
+  int32_t desc[ALN_MAX_KEYS];
+  int nk;
+};
+__global__ void __launch_bounds__(TF_BLOCK) k_tk_final(TfArgs a, const uint32_t *__restrict__ cand,
+                                                       const uint64_t *__restrict__ count, uint64_t n,
+                                                       uint32_t most, uint32_t k, uint32_t *__restrict__ out) {
+  extern __shared__ __align__(16) uint64_t tf_lds[];
+  const uint64_t m = count ? *count : n;
+  if (m > most) return;
+  uint32_t p2 = 2;
+  while (p2 < m) p2 <<= 1;
+  uint64_t *code = tf_lds;  // [key][p2]
+  uint32_t *row = reinterpret_cast<uint32_t *>(tf_lds + (size_t)a.nk * p2);
+  for (uint32_t i = threadIdx.x; i < p2; i += TF_BLOCK) {
+    const uint32_t r = i < m ? (cand ? cand[i] : i) : 0xFFFFFFFFu;  // no row has that number: padding sorts last
+    row[i] = r;
+    for (int j = 0; j < a.nk; ++j) code[(size_t)j * p2 + i] = i < m ? tk_code(a.k[j][r], a.desc[j]) : ~0ull;
+  }
+  __syncthreads();
+  for (uint32_t size = 2; size <= p2; size <<= 1)
+    for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+      for (uint32_t t = threadIdx.x; t < p2 / 2; t += TF_BLOCK) {
+        const uint32_t lo = 2 * t - (t & (stride - 1)), hi = lo + stride;
+        bool greater = row[lo] > row[hi];
+        for (int j = a.nk - 1; j >= 0; --j) {
+          const uint64_t x = code[(size_t)j * p2 + lo], y = code[(size_t)j * p2 + hi];
+          greater = x > y || (x == y && greater);
+        }
+        if (greater == ((lo & size) == 0)) {
+          const uint32_t r = row[lo];
+          row[lo] = row[hi];
+          row[hi] = r;
+          for (int j = 0; j < a.nk; ++j) {
+            const uint64_t x = code[(size_t)j * p2 + lo];
+            code[(size_t)j * p2 + lo] = code[(size_t)j * p2 + hi];
+            code[(size_t)j * p2 + hi] = x;
+          }
+        }
+      }
+      __syncthreads();
+    }
+  for (uint32_t i = threadIdx.x; i < k && i < m; i += TF_BLOCK) out[i] = row[i];
+}
+
+// One key: the candidates' codes; more: their gathered key values.
+__global__ void k_tk_gather(const int64_t *__restrict__ key, int desc, const uint32_t *__restrict__ cand, uint64_t m,
+                            int64_t *__restrict__ out) {
+  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < m; i += (uint64_t)gridDim.x * 256)
+    out[i] = (int64_t)tk_code(key[cand[i]], desc);
+}
+
+template <int U>
+static void tk_candidates(aln_ctx *c, const TfArgs &a, uint64_t n, uint32_t nchunks, uint32_t k, uint64_t *cmin,
+                          uint64_t *ctl, uint32_t *cand) {
+  const dim3 grid((nchunks + 3) / 4);
+  hipLaunchKernelGGL(k_tk_min<U>, grid, dim3(256), 0, c->stream, a.k[0], a.desc[0], n, nchunks, cmin);
+  hipLaunchKernelGGL(k_tk_bound, dim3(1), dim3(TF_BLOCK), 0, c->stream, (const uint64_t *)cmin, nchunks, k, ctl);
+  hipLaunchKernelGGL(k_tk_collect<U>, grid, dim3(256), 0, c->stream, a.k[0], a.desc[0], n, nchunks,
+                     a.nk == 1 ? 1 : 0, (const uint64_t *)cmin, ctl, cand);
+}
+
+// The candidate path; *done = false when there are too many candidates (nothing written).
+// Taken when the rows make at least k chunks of 64, or fit the final sort as they are.
+static int topk_bounded(aln_ctx *c, const TfArgs &a, uint64_t n, uint32_t k, uint32_t *d_out_idx, bool *done) {
+  *done = false;
+  const uint32_t most = tf_max(a.nk);
+  const size_t lds = (size_t)most * (8 * a.nk + 4);
+  if (n <= most) {
+    hipLaunchKernelGGL(k_tk_final, dim3(1), dim3(TF_BLOCK), lds, c->stream, a, (const uint32_t *)nullptr,
+                       (const uint64_t *)nullptr, n, most, k, d_out_idx);
+    ALN_TRY(check_launch("topk_final"));
+    ALN_HIP(hipStreamSynchronize(c->stream));
+    *done = true;
+    return ALN_OK;
+  }
+  if (n < 64ull * k) return ALN_OK;
+  // chunks as large as leave 8k of them (the bound is then near the k-th row's key)
+  uint32_t u = 16;
+  while (u > 1 && n / (64 * u) < 8ull * k) u >>= 1;
+  const uint32_t nchunks = (uint32_t)((n + 64 * u - 1) / (64 * u));
+  uint64_t *cmin, *ctl;
+  uint32_t *cand;
+  ALN_TRY(ws(c, nchunks, &cmin));
+  ALN_TRY(ws(c, 3, &ctl));
+  ALN_TRY(ws(c, (size_t)TK_CAND, &cand));
+  {
+    ProfScope ps(c, "topk_candidates");
+    if (u == 16)
+      tk_candidates<16>(c, a, n, nchunks, k, cmin, ctl, cand);
+    else if (u == 8)
+      tk_candidates<8>(c, a, n, nchunks, k, cmin, ctl, cand);
+    else if (u == 4)
+      tk_candidates<4>(c, a, n, nchunks, k, cmin, ctl, cand);
+    else if (u == 2)
+      tk_candidates<2>(c, a, n, nchunks, k, cmin, ctl, cand);
+    else
+      tk_candidates<1>(c, a, n, nchunks, k, cmin, ctl, cand);
+  }
+  ALN_TRY(check_launch("topk_candidates"));
+  hipLaunchKernelGGL(k_tk_final, dim3(1), dim3(TF_BLOCK), lds, c->stream, a, (const uint32_t *)cand,
+                     (const uint64_t *)(ctl + 2), n, most, k, d_out_idx);
+  ALN_TRY(check_launch("topk_final"));
+  uint64_t m = 0;
+  ALN_TRY(copy_to_host(c, &m, ctl + 2, 8));
+  if (m <= most) {
+    *done = true;
+    return ALN_OK;
+  }
+  if (m > TK_CAND) return ALN_OK;
+  // the tile sort of the candidates' codes
+  const unsigned gm = grid_for(m, 256, 65536);
+  uint64_t *code;
+  uint32_t nout;
+  ALN_TRY(ws(c, m, &code));
+  if (a.nk == 1) {
+    hipLaunchKernelGGL(k_tk_gather, dim3(gm), dim3(256), 0, c->stream, a.k[0], a.desc[0], (const uint32_t *)cand, m,
+                       reinterpret_cast<int64_t *>(code));
+  } else {
+    const int64_t *ck[ALN_MAX_KEYS];
+    for (int j = 0; j < a.nk; ++j) {
+      int64_t *g;
+      ALN_TRY(ws(c, m, &g));
+      ck[j] = g;
+      hipLaunchKernelGGL(k_tk_gather, dim3(gm), dim3(256), 0, c->stream, a.k[j], TK_RAW, (const uint32_t *)cand, m, g);
+    }
+    KeyRanges r;
+    ALN_TRY(key_ranges(c, ck, a.nk, m, &r));
+    if (r.total > 64) return ALN_OK;
+    KeySet ks;
+    key_set(r, ck, a.desc, 0, a.nk, &ks);
+    hipLaunchKernelGGL(k_codes, dim3(gm), dim3(256), 0, c->stream, ks, (const uint32_t *)nullptr, m, code,
+                       (uint32_t *)nullptr);
+  }
+  ALN_TRY(check_launch("topk_codes"));
+  ALN_TRY(topk_codes(c, code, cand, m, k, d_out_idx, &nout));
+  *done = true;
+  return ALN_OK;
+}
+
 }  // namespace aln
 
 using namespace aln;
@@ -1145,6 +1421,22 @@ int aln_topk(aln_ctx *c, const int64_t *const *d_keys, const int32_t *desc, int 
   *h_nout = 0;
   if (n == 0 || k == 0) return ALN_OK;
   ALN_REQUIRE(d_out_idx, "aln_topk: no output buffer");
+  TfArgs a;
+  memset(&a, 0, sizeof(a));
+  a.nk = nkeys;
+  for (int j = 0; j < nkeys; ++j) {
+    a.k[j] = d_keys[j];
+    a.desc[j] = desc && desc[j] ? 1 : 0;
+  }
+  bool done = false;
+  if (k <= TK_TILE / 2) {
+    ALN_TRY(topk_bounded(c, a, n, k, d_out_idx, &done));
+    if (done) {
+      *h_nout = (uint32_t)(n < k ? n : k);
+      return ALN_OK;
+    }
+    ws_reset(c);
+  }
   KeyRanges r;
   ALN_TRY(key_ranges(c, d_keys, nkeys, n, &r));
   if (r.total > 64 || k > TK_TILE / 2) {
@@ -1167,6 +1459,16 @@ int aln_topk(aln_ctx *c, const int64_t *const *d_keys, const int32_t *desc, int 
   hipLaunchKernelGGL(k_codes, dim3(grid_for(n, 256, 65536)), dim3(256), 0, c->stream, ks,
                      (const uint32_t *)nullptr, n, code, idx);
   ALN_TRY(check_launch("codes"));
+  if (nkeys > 1) {  // too many rows tie on the first key: the codes of all of them as one key
+    a.nk = 1;
+    a.k[0] = reinterpret_cast<const int64_t *>(code);
+    a.desc[0] = TK_RAW;
+    ALN_TRY(topk_bounded(c, a, n, k, d_out_idx, &done));
+    if (done) {
+      *h_nout = (uint32_t)(n < k ? n : k);
+      return ALN_OK;
+    }
+  }
   return topk_codes(c, code, idx, n, k, d_out_idx, h_nout);
 }
 

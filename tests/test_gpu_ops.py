@@ -421,6 +421,32 @@ def test_sort_and_topk(ctx, wide):
         assert np.array_equal(top, want[:k])
 
 
+@pytest.mark.parametrize("n,k", [(1, 1), (2048, 512), (2049, 32), (2049, 40), (4099, 64), (70001, 100),
+                                 (70001, 512), (600000, 3), (1500000, 100)])
+@pytest.mark.parametrize("kind", ["spread", "ties", "sorted", "one", "wide"])
+def test_topk_candidates(ctx, n, k, kind):
+    """ORDER BY .. LIMIT k at the edges of its routes (all rows in one block; chunks of 64 to
+    1024 rows; few, many and too many candidates) against the stable multi-key sort: spread
+    first keys with the int64 extremes among them, few distinct ones, rows already in (and
+    against) the order, one value everywhere, and keys of more than 64 bits together."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n + k)
+    k0 = {"spread": lambda: r.integers(-(1 << 62), 1 << 62, n), "ties": lambda: r.integers(0, 7, n),
+          "sorted": lambda: np.arange(n) * 3 - 50, "one": lambda: np.full(n, -5),
+          "wide": lambda: r.integers(-(1 << 40), 1 << 40, n)}[kind]().astype(np.int64)
+    if kind == "spread" and n > 8:
+        k0[3], k0[n - 2], k0[n // 2] = -(1 << 63), (1 << 63) - 1, -(1 << 63)
+    k1 = r.integers(0, 5, n).astype(np.int64)
+    k2 = r.integers(-(1 << 30), 1 << 30, n).astype(np.int64)
+    for keys, desc in (([k0], [0]), ([k0], [1]), ([k0, k1], [1, 0]), ([k0, k1, k2], [0, 1, 1]),
+                       ([k0, k1, k2, k0], [1, 1, 0, 0])):
+        got = host(D.topk(ctx, [dev(ctx, x) for x in keys], desc, k)).astype(np.int64)
+        cols = [(~x if d else x) for x, d in zip(keys, desc)]  # ~x reverses the int64 order
+        want = np.lexsort([np.arange(n)] + cols[::-1])[:k]
+        assert np.array_equal(got, want), (len(keys), desc)
+
+
 def test_radix_sort_pairs(ctx):
     from alenka_amd import device as D
 
