@@ -202,71 +202,121 @@ struct RangeC {
   int64_t lo, hi;
 };
 
-// PASS 0: count passing rows per tile.  PASS 1: write ascending global row ids.
-template <int PASS, bool FAST>
-__global__ void __launch_bounds__(SC_BLOCK) k_scan(const ColTable *__restrict__ ct,
-                                                   const aln_insn *__restrict__ prog, int nprog,
-                                                   const RangeC *__restrict__ rg, int nrg,
-                                                   uint32_t seg_rows, uint32_t tiles_per_seg,
-                                                   const char *__restrict__ modes,
-                                                   uint32_t *__restrict__ counts,
-                                                   const uint64_t *__restrict__ offs,
-                                                   uint32_t *__restrict__ out) {
-  __shared__ int64_t stk[FAST ? 1 : ALN_MAX_STACK * SC_BLOCK];
+// What one scan kernel call evaluates, by value (no upload).
+struct ScanArgs {
+  ColTable ct;
+  uint32_t seg_rows, tiles_per_seg;
+  const char *modes;
+};
+// At most one interval per column plus one set test per two instructions.
+constexpr int MAX_RANGES_C = ALN_MAX_COLS + ALN_MAX_INSN / 2;
+struct RangeSet {
+  RangeC r[MAX_RANGES_C];
+  int n;
+};
+
+// Which of the U rows idx[u] of a segment lie in every term.  An interval over codes narrower
+// than 64 bits is compared with the codes themselves.
+template <int U>
+__device__ __forceinline__ void ranges_pass(const RangeSet &rs, const ColTable &ct, uint32_t seg, uint32_t r0,
+                                            const uint32_t (&idx)[U], bool (&pass)[U]) {
+  for (int k = 0; k < rs.n; ++k) {
+    const RangeC t = rs.r[k];
+    const aln_seg sg = ct.segs[t.col][seg];
+    uint64_t c[U];
+    unpack_codes<U>(ct.words[t.col] + sg.word_off + (uint64_t)(r0 >> 5) * sg.bits, sg.bits, idx, c);
+    if (t.set) {
+      const uint32_t *bs = reinterpret_cast<const uint32_t *>(t.lo);
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t v = (int64_t)((uint64_t)sg.base + c[u]);
+        pass[u] = pass[u] && v >= 0 && v < t.hi && ((bs[v >> 5] >> (v & 31)) & 1u);
+      }
+    } else if (sg.bits == 64) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t v = (int64_t)((uint64_t)sg.base + c[u]);
+        pass[u] = pass[u] && v >= t.lo && v <= t.hi;
+      }
+    } else {
+      const uint64_t most = (1ull << sg.bits) - 1;
+      const uint64_t clo = t.lo <= sg.base ? 0 : (uint64_t)t.lo - (uint64_t)sg.base;
+      uint64_t chi = (uint64_t)t.hi - (uint64_t)sg.base;
+      chi = chi < most ? chi : most;
+      const bool none = t.hi < sg.base || clo > most;
+      if (sg.bits <= 32) {
+        const uint32_t lo = (uint32_t)clo, width = (uint32_t)chi - lo;
+#pragma unroll
+        for (int u = 0; u < U; ++u) pass[u] = pass[u] && !none && (uint32_t)c[u] - lo <= width;
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) pass[u] = pass[u] && !none && c[u] - clo <= chi - clo;
+      }
+    }
+  }
+}
+
+// One tile of SC_TILE rows per block: its passing rows as one bit per row and their number
+// (OUT SCAN_MASK), the number alone (SCAN_COUNT), or their global row ids (SCAN_WRITE).  Each
+// predicate is decoded and evaluated once, U rows of a thread at a time; the row ids then come
+// from the masks (k_scan_expand).  Bound by the instructions of the decode and of the program:
+// 40M rows of (date < d AND disc != 5) OR price * (100 - disc) > x took two passes of 1.03 ms
+// each with one row per instruction and the predicate evaluated by the count and by the write.
+enum { SCAN_MASK = 0, SCAN_COUNT = 1, SCAN_WRITE = 2 };
+template <int OUT, int U, typename Pred>
+__device__ __forceinline__ void scan_tile(const ScanArgs &a, uint64_t *__restrict__ masks,
+                                          uint32_t *__restrict__ counts, const uint64_t *__restrict__ offs,
+                                          uint32_t *__restrict__ out, Pred pred) {
   __shared__ uint32_t wc[SC_BLOCK / 64];
-  const uint32_t seg = blockIdx.x / tiles_per_seg, tile = blockIdx.x % tiles_per_seg;
-  const uint32_t nrows = ct->segs[0][seg].nrows;
+  const uint32_t seg = blockIdx.x / a.tiles_per_seg, tile = blockIdx.x % a.tiles_per_seg;
+  const uint32_t nrows = a.ct.segs[0][seg].nrows;
   const uint32_t r0 = tile * SC_TILE;
-  const char mode = modes ? modes[seg] : 'R';
+  const char mode = a.modes ? a.modes[seg] : 'R';
   if (r0 >= nrows || mode == 'N') {
-    if (PASS == 0 && threadIdx.x == 0) counts[blockIdx.x] = 0;
+    if (OUT != SCAN_WRITE && threadIdx.x == 0) counts[blockIdx.x] = 0;
     return;
   }
   const unsigned lane = __lane_id(), wid = threadIdx.x / 64;
-  const uint64_t gbase = (uint64_t)seg * seg_rows;
-  uint64_t run = PASS ? offs[blockIdx.x] : 0;
+  const uint32_t left = nrows - r0;
+  uint64_t run = OUT == SCAN_WRITE ? offs[blockIdx.x] : 0, mine = 0;
   uint32_t total = 0;
-  for (int j = 0; j < SC_ITEMS; ++j) {
-    uint32_t local = r0 + j * SC_BLOCK + threadIdx.x;
-    bool pass = false;
-    if (local < nrows) {
-      if (mode == 'A') {
-        pass = true;
-      } else if (FAST) {
-        pass = true;
-        for (int k = 0; k < nrg; ++k) {
-          const int c = rg[k].col;
-          int64_t v = decode_row(ct->words[c], ct->segs[c][seg], local);
-          if (rg[k].set) {
-            const uint32_t *bs = reinterpret_cast<const uint32_t *>(rg[k].lo);
-            pass = pass && v >= 0 && v < rg[k].hi && ((bs[v >> 5] >> (v & 31)) & 1u);
-          } else {
-            pass = pass && v >= rg[k].lo && v <= rg[k].hi;
-          }
-        }
-      } else {
-        auto load = [&](int c) -> int64_t { return decode_row(ct->words[c], ct->segs[c][seg], local); };
-        pass = vm_run(prog, nprog, load, stk + threadIdx.x) != 0;
-      }
+#pragma unroll 1
+  for (int j0 = 0; j0 < SC_ITEMS; j0 += U) {
+    uint32_t idx[U];
+    bool pass[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {  // rows past the segment's end read its last row
+      const uint32_t i = (uint32_t)(j0 + u) * SC_BLOCK + threadIdx.x;
+      idx[u] = i < left ? i : left - 1;
+      pass[u] = true;
     }
-    uint64_t bal = __ballot(pass);
-    if (PASS == 0) {
-      total += __popcll(bal);
-    } else {
-      if (lane == 0) wc[wid] = (uint32_t)__popcll(bal);
-      __syncthreads();
-      uint32_t before = 0, all = 0;
-      for (int w = 0; w < SC_BLOCK / 64; ++w) {
-        uint32_t x = wc[w];
-        before += w < (int)wid ? x : 0;
-        all += x;
+    if (mode != 'A') pred(seg, r0, idx, pass);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t i = (uint32_t)(j0 + u) * SC_BLOCK + threadIdx.x;
+      const uint64_t bal = __builtin_amdgcn_ballot_w64(pass[u] && i < left);
+      if (OUT != SCAN_WRITE) {
+        total += (uint32_t)__popcll(bal);
+        if (OUT == SCAN_MASK && lane == (unsigned)(j0 + u)) mine = bal;
+      } else {
+        if (lane == 0) wc[wid] = (uint32_t)__popcll(bal);
+        __syncthreads();
+        uint32_t before = 0, all = 0;
+        for (int w = 0; w < SC_BLOCK / 64; ++w) {
+          const uint32_t x = wc[w];
+          before += w < (int)wid ? x : 0;
+          all += x;
+        }
+        if (bal >> lane & 1) out[run + before + below_count(bal)] = (uint32_t)((uint64_t)seg * a.seg_rows + r0 + i);
+        run += all;
+        __syncthreads();
       }
-      if (pass) out[run + before + below_count(bal)] = (uint32_t)(gbase + local);
-      run += all;
-      __syncthreads();
     }
   }
-  if (PASS == 0) {
+  if (OUT != SCAN_WRITE) {
+    // mask word 4 * j + wave of the tile: rows j * 256 + wave * 64 .. + 63
+    if (OUT == SCAN_MASK && lane < SC_ITEMS)
+      masks[(uint64_t)blockIdx.x * (SC_TILE / 64) + lane * (SC_BLOCK / 64) + wid] = mine;
     if (lane == 0) wc[wid] = total;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -277,11 +327,74 @@ __global__ void __launch_bounds__(SC_BLOCK) k_scan(const ColTable *__restrict__ 
   }
 }
 
+template <int OUT>
+__global__ void __launch_bounds__(SC_BLOCK) k_scan_ranges(ScanArgs a, RangeSet rs, uint64_t *__restrict__ masks,
+                                                          uint32_t *__restrict__ counts,
+                                                          const uint64_t *__restrict__ offs,
+                                                          uint32_t *__restrict__ out) {
+  constexpr int U = 8;
+  scan_tile<OUT, U>(a, masks, counts, offs, out,
+                    [&](uint32_t seg, uint32_t r0, const uint32_t(&idx)[U], bool(&pass)[U]) {
+                      ranges_pass<U>(rs, a.ct, seg, r0, idx, pass);
+                    });
+}
+
+template <int OUT, int U>
+__global__ void __launch_bounds__(SC_BLOCK) k_scan_prog(ScanArgs a, VProg p, uint64_t *__restrict__ masks,
+                                                        uint32_t *__restrict__ counts,
+                                                        const uint64_t *__restrict__ offs,
+                                                        uint32_t *__restrict__ out) {
+  extern __shared__ __align__(16) int64_t vm_stack[];
+  scan_tile<OUT, U>(a, masks, counts, offs, out,
+                    [&](uint32_t seg, uint32_t r0, const uint32_t(&idx)[U], bool(&pass)[U]) {
+                      auto load = [&](int col, int64_t(&v)[U]) {
+                        const aln_seg sg = a.ct.segs[col][seg];
+                        uint64_t c[U];
+                        unpack_codes<U>(a.ct.words[col] + sg.word_off + (uint64_t)(r0 >> 5) * sg.bits, sg.bits, idx, c);
+#pragma unroll
+                        for (int u = 0; u < U; ++u) v[u] = (int64_t)((uint64_t)sg.base + c[u]);
+                      };
+                      int64_t t[U];
+                      vm_eval<U>(p, load, vm_stack + threadIdx.x, t);
+#pragma unroll
+                      for (int u = 0; u < U; ++u) pass[u] = t[u] != 0;
+                    });
+}
+
+// Row ids of a tile's set mask bits.  Every wave scans the bit counts of the tile's 64 words
+// and writes the rows of 16 of them.
+__global__ void __launch_bounds__(SC_BLOCK) k_scan_expand(const uint64_t *__restrict__ masks, uint32_t seg_rows,
+                                                          uint32_t tiles_per_seg,
+                                                          const uint32_t *__restrict__ counts,
+                                                          const uint64_t *__restrict__ offs,
+                                                          uint32_t *__restrict__ out) {
+  if (counts[blockIdx.x] == 0) return;
+  const uint32_t seg = blockIdx.x / tiles_per_seg, tile = blockIdx.x % tiles_per_seg;
+  const unsigned lane = __lane_id(), wid = threadIdx.x / 64;
+  const uint64_t word = masks[(uint64_t)blockIdx.x * (SC_TILE / 64) + lane];
+  const uint32_t n = (uint32_t)__popcll(word);
+  uint32_t incl = n;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t y = __shfl_up(incl, o, 64);
+    if (lane >= (unsigned)o) incl += y;
+  }
+  const uint32_t first = incl - n;
+  uint32_t *dst = out + offs[blockIdx.x];
+  const uint32_t row = (uint32_t)((uint64_t)seg * seg_rows + tile * SC_TILE) + lane;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    const int w = (int)wid * 16 + j;
+    const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(word >> 32), w) << 32 |
+                       (uint32_t)__builtin_amdgcn_readlane((int)word, w);
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)first, w);
+    if (m >> lane & 1) dst[at + below_count(m)] = row + 64u * (uint32_t)w;
+  }
+}
+
 // Recognise a conjunction of "column OP constant" terms (multiplier 1) and code-set tests
 // (LIKE) and turn it into one closed interval per column plus the set tests.  Returns false
 // when the program has another shape.
-// At most one interval per column plus one set test per two instructions.
-constexpr int MAX_RANGES_C = ALN_MAX_COLS + ALN_MAX_INSN / 2;
 static bool as_intervals(const aln_insn *p, int n, RangeC *out, int *nout, bool *empty) {
   *empty = false;
   *nout = 0;
@@ -405,6 +518,44 @@ static int check_prog_cols(const aln_insn *prog, int nprog, int ncols) {
   return ALN_OK;
 }
 
+// A checked scan: a conjunction of intervals and set tests, or a program of any shape.
+struct ScanPlan {
+  ScanArgs a;
+  bool fast, empty;
+  RangeSet rs;
+  VProg prog;
+};
+static int scan_plan(const aln_col *cols, int ncols, uint32_t seg_rows, const aln_insn *prog, int nprog,
+                     ScanPlan *s) {
+  ALN_TRY(fill_cols(cols, ncols, &s->a.ct));
+  ALN_TRY(check_prog(prog, nprog));
+  s->a.seg_rows = seg_rows;
+  s->a.tiles_per_seg = (seg_rows + SC_TILE - 1) / SC_TILE;
+  s->a.modes = nullptr;
+  s->rs.n = 0;
+  s->empty = false;
+  s->fast = as_intervals(prog, nprog, s->rs.r, &s->rs.n, &s->empty);
+  if (!s->fast) vm_lower(prog, nprog, &s->prog);
+  return ALN_OK;
+}
+
+// Eight rows per thread and instruction while their LDS stack leaves five blocks per CU
+// (two values below the top, 32 KB), else two (up to 15 values, 60 KB).
+template <int OUT>
+static int scan_launch(hipStream_t st, const ScanPlan &s, uint32_t nblocks, uint64_t *masks, uint32_t *counts,
+                       const uint64_t *offs, uint32_t *out) {
+  const size_t row = sizeof(int64_t) * VM_BLOCK;
+  if (s.fast)
+    hipLaunchKernelGGL(k_scan_ranges<OUT>, dim3(nblocks), dim3(SC_BLOCK), 0, st, s.a, s.rs, masks, counts, offs, out);
+  else if (s.prog.slots <= 2)
+    hipLaunchKernelGGL((k_scan_prog<OUT, 8>), dim3(nblocks), dim3(SC_BLOCK), 8 * s.prog.slots * row, st, s.a, s.prog,
+                       masks, counts, offs, out);
+  else
+    hipLaunchKernelGGL((k_scan_prog<OUT, 2>), dim3(nblocks), dim3(SC_BLOCK), 2 * s.prog.slots * row, st, s.a, s.prog,
+                       masks, counts, offs, out);
+  return check_launch(OUT == SCAN_WRITE ? "scan_write" : "scan_count");
+}
+
 // Segment of the source row behind each index: r = rows ? rows[idx[i]] : idx[i]; the last
 // segment start <= r when starts are given (uneven file segments), else r / seg_rows.
 __global__ void __launch_bounds__(256) k_row_segments(const uint32_t *__restrict__ idx, uint64_t n,
@@ -430,23 +581,18 @@ __global__ void __launch_bounds__(256) k_row_segments(const uint32_t *__restrict
 
 // ---- fixed scratch of the allocation-free scan -----------------------------------------------
 // aln_scan_filter_noalloc keeps its temporaries in this array instead of the context's
-// workspace: the column table, program and intervals it uploads, the per-segment zone-map
-// verdicts, the per-tile counts, their exclusive scan and the scan's partial sums and total.
-// Every byte a call reads is written earlier in the same call, so nothing is cleared.  Each
-// GPU holds its own copy for the life of the process; host code reaches it only through the
-// address hipGetSymbolAddress returns on that device.
+// workspace: the per-segment zone-map verdicts it uploads, the per-tile counts, their exclusive
+// scan and the scan's partial sums and total (a mask bit per row would not fit: it evaluates
+// the predicate again to write).  Every byte a call reads is written earlier in the same call,
+// so nothing is cleared.  Each GPU holds its own copy for the life of the process; host code
+// reaches it only through the address hipGetSymbolAddress returns on that device.
 constexpr uint64_t NA_TILES = ALN_SCAN_NOALLOC_MAX_TILES;
-constexpr size_t NA_CT = 0;                                               // ColTable
-constexpr size_t NA_PROG = 256;                                           // ALN_MAX_INSN insns
-constexpr size_t NA_RANGES = NA_PROG + sizeof(aln_insn) * ALN_MAX_INSN;   // MAX_RANGES_C
-constexpr size_t NA_TOTAL = 2560;                                         // u64 scan total
+constexpr size_t NA_TOTAL = 0;                                            // u64 scan total
 constexpr size_t NA_MODES = 4096;                                         // u8 per segment
 constexpr size_t NA_COUNTS = NA_MODES + NA_TILES;                         // u32 per tile
 constexpr size_t NA_OFFS = NA_COUNTS + 4 * NA_TILES;                      // u64 per tile
 constexpr size_t NA_SUMS = NA_OFFS + 8 * NA_TILES;                        // u64 per scan tile
 constexpr size_t NA_BYTES = NA_SUMS + 8 * ((NA_TILES + 4095) / 4096 + 32);
-static_assert(sizeof(ColTable) <= NA_PROG, "column table overlaps the program");
-static_assert(NA_RANGES + sizeof(RangeC) * MAX_RANGES_C <= NA_TOTAL, "intervals overlap the total");
 static_assert(NA_TILES % 256 == 0, "scratch regions lose their alignment");
 
 static __device__ __align__(256) unsigned char scratch[NA_BYTES];
@@ -684,44 +830,26 @@ int aln_scan_filter(aln_ctx *c, const aln_col *cols, int ncols, uint32_t seg_row
   ALN_REQUIRE((uint64_t)nsegs * seg_rows <= (1ull << 32), "aln_scan_filter: more than 2^32 rows");
   *h_count = 0;
   if (nsegs == 0) return ALN_OK;
-  ColTable *ct;
-  aln_insn *dp;
-  ALN_TRY(upload_cols(c, cols, ncols, &ct));
-  ALN_TRY(upload_prog(c, prog, nprog, &dp));
-  RangeC rgs[MAX_RANGES_C];
-  int nrg = 0;
-  bool empty = false;
-  bool fast = as_intervals(prog, nprog, rgs, &nrg, &empty);
-  if (fast && empty) return ALN_OK;
-  RangeC *drg = nullptr;
-  if (fast && nrg > 0) {
-    ALN_TRY(ws(c, nrg, &drg));
-    ALN_HIP(hipMemcpyAsync(drg, rgs, sizeof(RangeC) * nrg, hipMemcpyHostToDevice, c->stream));
-  }
-  char *dmodes = nullptr;
+  ScanPlan s;
+  ALN_TRY(scan_plan(cols, ncols, seg_rows, prog, nprog, &s));
+  if (s.fast && s.empty) return ALN_OK;
   if (seg_modes) {
+    char *dmodes;
     ALN_TRY(ws(c, nsegs, &dmodes));
     ALN_HIP(hipMemcpyAsync(dmodes, seg_modes, nsegs, hipMemcpyHostToDevice, c->stream));
+    s.a.modes = dmodes;
   }
-  uint32_t tps = (seg_rows + SC_TILE - 1) / SC_TILE;
-  uint64_t nblocks = (uint64_t)nsegs * tps;
+  const uint64_t nblocks = (uint64_t)nsegs * s.a.tiles_per_seg;
   ALN_REQUIRE(nblocks < (1ull << 31), "aln_scan_filter: grid too large");
   uint32_t *counts;
-  uint64_t *offs;
+  uint64_t *offs, *masks;
   ALN_TRY(ws(c, nblocks, &counts));
   ALN_TRY(ws(c, nblocks, &offs));
+  ALN_TRY(ws(c, nblocks * (SC_TILE / 64), &masks));
   {
     ProfScope p(c, "scan_count");
-    if (fast)
-      hipLaunchKernelGGL((k_scan<0, true>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream,
-                         ct, dp, nprog, drg, nrg, seg_rows, tps, dmodes, counts,
-                         (const uint64_t *)nullptr, (uint32_t *)nullptr);
-    else
-      hipLaunchKernelGGL((k_scan<0, false>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream,
-                         ct, dp, nprog, drg, 0, seg_rows, tps, dmodes, counts,
-                         (const uint64_t *)nullptr, (uint32_t *)nullptr);
+    ALN_TRY(scan_launch<SCAN_MASK>(c->stream, s, (uint32_t)nblocks, masks, counts, nullptr, nullptr));
   }
-  ALN_TRY(check_launch("scan_count"));
   uint64_t total = 0;
   ALN_TRY(exclusive_scan_u32(c, counts, nblocks, offs, &total));
   *h_count = total;
@@ -731,13 +859,8 @@ int aln_scan_filter(aln_ctx *c, const aln_col *cols, int ncols, uint32_t seg_row
   ALN_REQUIRE(d_row_ids, "aln_scan_filter: no output buffer");
   {
     ProfScope p(c, "scan_write");
-    if (fast)
-      hipLaunchKernelGGL((k_scan<1, true>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream,
-                         ct, dp, nprog, drg, nrg, seg_rows, tps, dmodes, counts, offs,
-                         d_row_ids);
-    else
-      hipLaunchKernelGGL((k_scan<1, false>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream,
-                         ct, dp, nprog, drg, 0, seg_rows, tps, dmodes, counts, offs, d_row_ids);
+    hipLaunchKernelGGL(k_scan_expand, dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream, (const uint64_t *)masks,
+                       seg_rows, s.a.tiles_per_seg, (const uint32_t *)counts, (const uint64_t *)offs, d_row_ids);
   }
   ALN_TRY(check_launch("scan_write"));
   ALN_HIP(hipStreamSynchronize(c->stream));
@@ -759,48 +882,30 @@ int aln_scan_filter_noalloc(aln_ctx *c, const aln_col *cols, int ncols, uint32_t
                             uint32_t *d_row_ids, uint64_t cap, uint64_t *h_count) {
   ALN_REQUIRE(c && cols && h_count && seg_rows > 0, "aln_scan_filter_noalloc: bad arguments");
   ALN_TRY(check_prog_cols(prog, nprog, ncols));
-  ColTable hct;
-  ALN_TRY(fill_cols(cols, ncols, &hct));
-  ALN_TRY(check_prog(prog, nprog));
+  ScanPlan s;
+  ALN_TRY(scan_plan(cols, ncols, seg_rows, prog, nprog, &s));
   const uint32_t nsegs = cols[0].nsegs;
   ALN_REQUIRE((uint64_t)nsegs * seg_rows <= (1ull << 32), "aln_scan_filter_noalloc: more than 2^32 rows");
   *h_count = 0;
   if (nsegs == 0) return ALN_OK;
-  const uint32_t tps = (seg_rows + SC_TILE - 1) / SC_TILE;
-  const uint64_t nblocks = (uint64_t)nsegs * tps;
+  const uint64_t nblocks = (uint64_t)nsegs * s.a.tiles_per_seg;
   if (nblocks > NA_TILES)
     return set_error(ALN_E_ARG,
                      "aln_scan_filter_noalloc: %u segments of %u rows are %llu tiles of %d rows; the fixed "
                      "scratch holds %llu tiles (use aln_scan_filter)",
                      nsegs, seg_rows, (unsigned long long)nblocks, SC_TILE, (unsigned long long)NA_TILES);
-  RangeC rgs[MAX_RANGES_C];
-  int nrg = 0;
-  bool empty = false;
-  const bool fast = as_intervals(prog, nprog, rgs, &nrg, &empty);
-  if (fast && empty) return ALN_OK;
+  if (s.fast && s.empty) return ALN_OK;
   char *base;
   ALN_TRY(scan_scratch(c, &base));
-  ColTable *ct = reinterpret_cast<ColTable *>(base + NA_CT);
-  aln_insn *dp = reinterpret_cast<aln_insn *>(base + NA_PROG);
-  RangeC *drg = fast && nrg > 0 ? reinterpret_cast<RangeC *>(base + NA_RANGES) : nullptr;
   uint64_t *tot = reinterpret_cast<uint64_t *>(base + NA_TOTAL);
-  char *dmodes = seg_modes ? base + NA_MODES : nullptr;
   uint32_t *counts = reinterpret_cast<uint32_t *>(base + NA_COUNTS);
   uint64_t *offs = reinterpret_cast<uint64_t *>(base + NA_OFFS);
   uint64_t *sums = reinterpret_cast<uint64_t *>(base + NA_SUMS);
-  ALN_HIP(hipMemcpyAsync(ct, &hct, sizeof(hct), hipMemcpyHostToDevice, c->stream));
-  ALN_HIP(hipMemcpyAsync(dp, prog, sizeof(aln_insn) * nprog, hipMemcpyHostToDevice, c->stream));
-  if (drg) ALN_HIP(hipMemcpyAsync(drg, rgs, sizeof(RangeC) * nrg, hipMemcpyHostToDevice, c->stream));
-  if (dmodes) ALN_HIP(hipMemcpyAsync(dmodes, seg_modes, nsegs, hipMemcpyHostToDevice, c->stream));
-  if (fast)
-    hipLaunchKernelGGL((k_scan<0, true>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream, ct, dp,
-                       nprog, drg, nrg, seg_rows, tps, dmodes, counts, (const uint64_t *)nullptr,
-                       (uint32_t *)nullptr);
-  else
-    hipLaunchKernelGGL((k_scan<0, false>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream, ct, dp,
-                       nprog, drg, 0, seg_rows, tps, dmodes, counts, (const uint64_t *)nullptr,
-                       (uint32_t *)nullptr);
-  ALN_TRY(check_launch("scan_count"));
+  if (seg_modes) {
+    s.a.modes = base + NA_MODES;
+    ALN_HIP(hipMemcpyAsync(base + NA_MODES, seg_modes, nsegs, hipMemcpyHostToDevice, c->stream));
+  }
+  ALN_TRY(scan_launch<SCAN_COUNT>(c->stream, s, (uint32_t)nblocks, nullptr, counts, nullptr, nullptr));
   ALN_TRY(exclusive_scan_u32_buf(c->stream, counts, nblocks, offs, sums, tot));
   uint64_t total = 0;
   ALN_HIP(hipMemcpyAsync(&total, tot, sizeof(total), hipMemcpyDeviceToHost, c->stream));
@@ -811,13 +916,7 @@ int aln_scan_filter_noalloc(aln_ctx *c, const aln_col *cols, int ncols, uint32_t
                      (unsigned long long)total, (unsigned long long)cap);
   if (total == 0) return ALN_OK;
   ALN_REQUIRE(d_row_ids, "aln_scan_filter_noalloc: no output buffer");
-  if (fast)
-    hipLaunchKernelGGL((k_scan<1, true>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream, ct, dp,
-                       nprog, drg, nrg, seg_rows, tps, dmodes, counts, offs, d_row_ids);
-  else
-    hipLaunchKernelGGL((k_scan<1, false>), dim3((unsigned)nblocks), dim3(SC_BLOCK), 0, c->stream, ct, dp,
-                       nprog, drg, 0, seg_rows, tps, dmodes, counts, offs, d_row_ids);
-  ALN_TRY(check_launch("scan_write"));
+  ALN_TRY(scan_launch<SCAN_WRITE>(c->stream, s, (uint32_t)nblocks, nullptr, counts, offs, d_row_ids));
   ALN_HIP(hipStreamSynchronize(c->stream));
   return ALN_OK;
 }

@@ -126,6 +126,85 @@ def test_scan_filter(ctx, name, ops, zone_maps):
     assert np.array_equal(got, want)
 
 
+def run_program(prog, cols):
+    """A compiled integer program over numpy int64 columns (wrapping arithmetic)."""
+    st = []
+    for op, a, k in prog:
+        if op == L.I_COL:
+            st.append(cols[a] * np.int64(k))
+        elif op == L.I_CONST:
+            st.append(np.full(cols[0].size, k, np.int64))
+        else:
+            r, l = st.pop(), st.pop()
+            if op == L.I_DIV:
+                q = np.array([0 if y == 0 else abs(int(x)) // abs(int(y)) * (1 if (x < 0) == (y < 0) else -1)
+                              for x, y in zip(l, r)], object)
+                v = ((q + (1 << 63)) % (1 << 64) - (1 << 63)).astype(np.int64)
+            else:
+                v = {L.I_ADD: lambda: l + r, L.I_SUB: lambda: l - r, L.I_MUL: lambda: l * r,
+                     L.I_AND: lambda: (l != 0) & (r != 0), L.I_OR: lambda: (l != 0) | (r != 0),
+                     L.I_CMP: lambda: [None, l < r, l > r, l != r, l == r, l <= r, l >= r][a]}[op]().astype(np.int64)
+            st.append(v)
+    assert len(st) == 1
+    return st[0]
+
+
+def random_program(r, ncols, depth, lo, hi):
+    """A random integer expression in postfix, `depth` operations deep at most."""
+    if depth == 0 or r.random() < 0.2:
+        if r.random() < 0.6:
+            return [(L.I_COL, int(r.integers(ncols)), int(r.choice([1, 1, 1, 100, -3])))]
+        return [(L.I_CONST, 0, int(r.choice([0, 1, 2, -7, 1000, 99999, 1 << 40, int(r.integers(lo, hi))])))]
+    op = int(r.choice([L.I_ADD, L.I_SUB, L.I_MUL, L.I_DIV, L.I_CMP, L.I_CMP, L.I_AND, L.I_OR]))
+    return (random_program(r, ncols, depth - 1, lo, hi) + random_program(r, ncols, depth - 1, lo, hi) +
+            [(op, int(r.integers(1, 7)) if op == L.I_CMP else 0, 0)])
+
+
+@pytest.mark.parametrize("n,seg_rows", [(1, 1), (63, 64), (4097, 4096), (4096, 5000), (8191, 8191), (9001, 700)])
+def test_programs_random(ctx, n, seg_rows):
+    """Scans and expressions of random programs (conjunctions of intervals and any shape; one
+    to five values on the stack) over columns of every code width class (0, 1 to 32, 33 to 63,
+    64 bits, plain), at the edges of the 4096-row tiles and of short segments, against numpy;
+    the allocation-free scan gives the same rows."""
+    import ctypes as C
+
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n * 31 + seg_rows)
+    cols = [r.integers(0, 2, n), r.integers(-50000, 80000, n), r.integers(0, 1 << 31, n) * 2 + 1,
+            r.integers(-(1 << 44), 1 << 44, n), np.full(n, -77), r.integers(-(1 << 63), (1 << 63) - 1, n),
+            r.integers(-(1 << 62), 1 << 62, n)]
+    cols = [c.astype(np.int64) for c in cols]
+    dcols = [D.Column.encode(ctx, dev(ctx, c), seg_rows) for c in cols[:-1]]
+    dcols.append(D.Column.plain(ctx, dev(ctx, cols[-1]), seg_rows))
+    progs = [[(L.I_COL, c, 1), (L.I_CONST, 0, int(np.median(cols[c])) + d), (L.I_CMP, cmp, 0)]
+             for c in range(len(cols)) for cmp in (1, 2, 4, 5, 6) for d in (0, 1)]
+    progs += [p + q + [(L.I_AND, 0, 0)] for p, q in zip(progs, reversed(progs))]
+    progs += [random_program(r, len(cols), d, -90000, 90000) for d in (1, 2, 3, 3, 4, 4) for _ in range(8)]
+    rows = np.sort(r.choice(n, n // 2 + 1, replace=False)).astype(np.int32)
+    mixed = r.permutation(rows)  # rows of one wave in several segments
+    with np.errstate(over="ignore"):
+        for prog in progs:
+            if len(prog) > L.MAX_INSN:
+                continue
+            want = run_program(prog, cols)
+            got = host(D.scan_filter(ctx, dcols, prog))
+            assert np.array_equal(got, np.nonzero(want)[0]), prog
+            out, cnt = ctx.empty(n, torch.int32), C.c_uint64()
+            L.check(ctx.lib.aln_scan_filter_noalloc(ctx.h, D._cols_array(dcols), len(dcols), seg_rows,
+                                                    L.insn_array(prog), len(prog), None, D._p(out), n, C.byref(cnt)))
+            assert np.array_equal(host(out)[: cnt.value], got), prog
+            assert np.array_equal(host(D.eval_rows(ctx, dcols, prog)), want), prog
+            for sel in (rows, mixed):
+                assert np.array_equal(host(D.eval_rows(ctx, dcols, prog, torch.as_tensor(sel).to(ctx.device))),
+                                      want[sel]), prog
+    for c, dc in zip(cols, dcols):
+        assert np.array_equal(host(D.gather(ctx, dc, torch.as_tensor(mixed).to(ctx.device))), c[mixed])
+        assert np.array_equal(host(D.gather(ctx, dc)), c)
+        for a, b in ((0, n), (n // 3, n - n // 4), (n - 1, n)):
+            assert np.array_equal(host(dc.decode(ctx, a, b)), c[a:b])
+
+
 def test_eval_revenue(ctx):
     from alenka_amd import device as D
 
