@@ -71,48 +71,132 @@ __global__ void __launch_bounds__(256) k_pack(const int64_t *__restrict__ v, uin
 // ---- row-wise kernels ---------------------------------------------------------------------
 
 // Rows outside the column (a segment past nsegs, or past a short last segment) read as 0.
+//
+// Consecutive rows [r0, r0 + n): a block's 2048 rows mostly lie in one segment, whose
+// descriptor is then scalar and whose codes are unpacked with 32-bit bit positions (HBM-bound:
+// 50M 24-bit codes 260 -> 94 us; a descriptor, a division and 64-bit positions per row before).
+constexpr int DEC_ROWS = 8;
 __global__ void __launch_bounds__(256) k_decode(const uint32_t *__restrict__ words,
                                                 const aln_seg *__restrict__ segs, uint32_t nsegs,
                                                 uint32_t seg_rows, uint64_t r0, uint64_t n,
                                                 int64_t *__restrict__ out) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256) {
-    uint64_t r = r0 + i;
-    uint64_t seg = r / seg_rows, local = r - seg * seg_rows;
-    out[i] = (seg < nsegs && local < segs[seg].nrows) ? decode_row(words, segs[seg], local) : 0;
-  }
-}
-
-__global__ void __launch_bounds__(256) k_gather(const uint32_t *__restrict__ words,
-                                                const aln_seg *__restrict__ segs, uint32_t nsegs,
-                                                uint32_t seg_rows,
-                                                const uint32_t *__restrict__ rows, uint64_t n,
-                                                int64_t *__restrict__ out) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256) {
-    uint32_t r = rows ? rows[i] : (uint32_t)i;
-    uint32_t seg = r / seg_rows, local = r - seg * seg_rows;
-    out[i] = (seg < nsegs && local < segs[seg].nrows) ? decode_row(words, segs[seg], local) : 0;
-  }
-}
-
-__global__ void __launch_bounds__(VM_BLOCK) k_eval(const ColTable *__restrict__ ct,
-                                                   const aln_insn *__restrict__ prog, int nprog,
-                                                   uint32_t nsegs, uint32_t seg_rows,
-                                                   const uint32_t *__restrict__ rows, uint64_t n,
-                                                   int64_t *__restrict__ out) {
-  __shared__ int64_t stk[ALN_MAX_STACK * VM_BLOCK];
-  for (uint64_t i0 = (uint64_t)blockIdx.x * VM_BLOCK; i0 < n; i0 += (uint64_t)gridDim.x * VM_BLOCK) {
-    uint64_t i = i0 + threadIdx.x;
-    if (i < n) {
-      uint32_t r = rows ? rows[i] : (uint32_t)i;
-      uint32_t seg = r / seg_rows, local = r - seg * seg_rows;
-      bool inside = seg < nsegs && local < ct->segs[0][seg < nsegs ? seg : 0].nrows;
-      auto load = [&](int c) -> int64_t {
-        return inside ? decode_row(ct->words[c], ct->segs[c][seg], local) : 0;
-      };
-      out[i] = vm_run(prog, nprog, load, stk + threadIdx.x);
+  const uint64_t b0 = (uint64_t)blockIdx.x * (256 * DEC_ROWS);
+  const uint32_t m = n - b0 < 256 * DEC_ROWS ? (uint32_t)(n - b0) : 256 * DEC_ROWS;
+  const uint64_t seg = (r0 + b0) / seg_rows;
+  const uint32_t l0 = (uint32_t)(r0 + b0 - seg * seg_rows);
+  out += b0;
+  if (seg < nsegs && (uint64_t)l0 + m <= segs[seg].nrows) {
+    const aln_seg sg = segs[seg];
+    const uint64_t bit = (uint64_t)l0 * sg.bits;
+    uint32_t idx[DEC_ROWS];
+    uint64_t c[DEC_ROWS];
+#pragma unroll
+    for (int u = 0; u < DEC_ROWS; ++u) {
+      const uint32_t i = threadIdx.x + 256 * u;
+      idx[u] = i < m ? i : m - 1;
     }
+    unpack_codes<DEC_ROWS>(words + sg.word_off + (bit >> 5), sg.bits, idx, c, (uint32_t)bit & 31);
+#pragma unroll
+    for (int u = 0; u < DEC_ROWS; ++u)
+      if (threadIdx.x + 256 * u < m)
+        __builtin_nontemporal_store((int64_t)((uint64_t)sg.base + c[u]), out + threadIdx.x + 256 * u);
+    return;
+  }
+  for (uint32_t i = threadIdx.x; i < m; i += 256) {
+    const uint64_t r = r0 + b0 + i, s = r / seg_rows, local = r - s * seg_rows;
+    out[i] = (s < nsegs && local < segs[s].nrows) ? decode_row(words, segs[s], local) : 0;
+  }
+}
+
+// The rows of an expression or a gather: U rows of a thread, 256 apart, each row's segment by a
+// product with ceil(2^64 / seg_rows) (seg_mul; 0 for one-row segments).  Selected rows ascend,
+// so a wave's rows mostly share a segment: its descriptors are then read once, as scalars
+// (price * (100 - disc) of 30M of 60M rows 461 -> 122 us, 240 MB written and 340 MB read).
+struct RowArgs {
+  ColTable ct;
+  uint32_t nsegs, seg_rows;
+  uint64_t seg_mul;
+  const uint32_t *rows;  // NULL: rows 0 .. n-1
+  uint64_t n;
+};
+template <int U>
+struct RowSet {
+  uint32_t seg[U], local[U];
+  bool in[U];   // the row exists in the first column's segment
+  bool same;    // every row of the wave lies in segment seg0 (and exists)
+  uint32_t seg0;
+};
+
+template <int U>
+__device__ __forceinline__ void row_set(const RowArgs &a, uint64_t i0, RowSet<U> &s) {
+  uint32_t r[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {  // past the end: the block's first row
+    const uint64_t i = i0 + threadIdx.x + 256 * u;
+    r[u] = a.rows ? a.rows[i < a.n ? i : i0] : (uint32_t)(i < a.n ? i : i0);
+  }
+  bool same = true;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    s.seg[u] = a.seg_mul ? (uint32_t)__umul64hi(a.seg_mul, (uint64_t)r[u]) : r[u];
+    s.local[u] = r[u] - s.seg[u] * a.seg_rows;
+  }
+  s.seg0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)s.seg[0]);
+  const uint32_t nrows0 = s.seg0 < a.nsegs ? a.ct.segs[0][s.seg0].nrows : 0;
+#pragma unroll
+  for (int u = 0; u < U; ++u) same = same && s.seg[u] == s.seg0 && s.local[u] < nrows0;
+  s.same = __builtin_amdgcn_ballot_w64(!same) == 0;
+  if (!s.same) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) s.in[u] = s.seg[u] < a.nsegs && s.local[u] < a.ct.segs[0][s.seg[u]].nrows;
+  }
+}
+
+// A column's values of the rows.  P: uint32_t when a segment's bits fit in 32 bits.
+template <int U, typename P>
+__device__ __forceinline__ void row_values(const RowArgs &a, const RowSet<U> &s, int col, int64_t (&v)[U]) {
+  if (s.same) {
+    const aln_seg sg = a.ct.segs[col][s.seg0];
+    P idx[U];
+    uint64_t c[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) idx[u] = s.local[u];
+    unpack_codes<U>(a.ct.words[col] + sg.word_off, sg.bits, idx, c);
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = (int64_t)((uint64_t)sg.base + c[u]);
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      v[u] = s.in[u] ? decode_row(a.ct.words[col], a.ct.segs[col][s.seg[u]], s.local[u]) : 0;
+  }
+}
+
+template <int U, typename P>
+__global__ void __launch_bounds__(VM_BLOCK) k_eval(RowArgs a, VProg p, int64_t *__restrict__ out) {
+  extern __shared__ __align__(16) int64_t vm_stack[];
+  const uint64_t i0 = (uint64_t)blockIdx.x * (VM_BLOCK * U);
+  RowSet<U> s;
+  row_set<U>(a, i0, s);
+  int64_t t[U];
+  vm_eval<U>(p, [&](int col, int64_t(&v)[U]) { row_values<U, P>(a, s, col, v); }, vm_stack + threadIdx.x, t);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint64_t i = i0 + threadIdx.x + VM_BLOCK * u;
+    if (i < a.n) __builtin_nontemporal_store(t[u], out + i);
+  }
+}
+
+template <int U, typename P>
+__global__ void __launch_bounds__(256) k_gather(RowArgs a, int64_t *__restrict__ out) {
+  const uint64_t i0 = (uint64_t)blockIdx.x * (256 * U);
+  RowSet<U> s;
+  row_set<U>(a, i0, s);
+  int64_t v[U];
+  row_values<U, P>(a, s, 0, v);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const uint64_t i = i0 + threadIdx.x + 256 * u;
+    if (i < a.n) __builtin_nontemporal_store(v[u], out + i);
   }
 }
 
@@ -492,23 +576,33 @@ static int check_prog(const aln_insn *prog, int nprog) {
   return ALN_OK;
 }
 
-int upload_cols(aln_ctx *c, const aln_col *cols, int ncols, ColTable **out) {
-  ColTable h;
-  ALN_TRY(fill_cols(cols, ncols, &h));
-  ColTable *d;
-  ALN_TRY(ws(c, 1, &d));
-  ALN_HIP(hipMemcpyAsync(d, &h, sizeof(h), hipMemcpyHostToDevice, c->stream));
-  *out = d;
+static int row_args(const aln_col *cols, int ncols, uint32_t seg_rows, const uint32_t *rows, uint64_t n, RowArgs *a) {
+  ALN_TRY(fill_cols(cols, ncols, &a->ct));
+  a->nsegs = cols[0].nsegs;
+  a->seg_rows = seg_rows;
+  a->seg_mul = seg_rows > 1 ? ~0ull / seg_rows + 1 : 0;
+  a->rows = rows;
+  a->n = n;
   return ALN_OK;
 }
+// Segments whose widest code positions fit in 32 bits.
+static bool narrow_segments(uint32_t seg_rows) { return seg_rows <= (1u << 26); }
 
-int upload_prog(aln_ctx *c, const aln_insn *prog, int nprog, aln_insn **out) {
-  ALN_TRY(check_prog(prog, nprog));
-  aln_insn *d;
-  ALN_TRY(ws(c, nprog, &d));
-  ALN_HIP(hipMemcpyAsync(d, prog, sizeof(aln_insn) * nprog, hipMemcpyHostToDevice, c->stream));
-  *out = d;
-  return ALN_OK;
+// Four rows per thread while their LDS stack is at most 32 KB (four values below the top),
+// else one (up to 15 values, 30 KB).
+template <int U>
+static int eval_launch_rows(hipStream_t st, const RowArgs &a, const VProg &p, int64_t *out) {
+  const uint64_t nb = (a.n + VM_BLOCK * U - 1) / (VM_BLOCK * U);
+  ALN_REQUIRE(nb < (1ull << 31), "aln_eval: grid too large");
+  const size_t lds = (size_t)p.slots * U * sizeof(int64_t) * VM_BLOCK;
+  if (narrow_segments(a.seg_rows))
+    hipLaunchKernelGGL((k_eval<U, uint32_t>), dim3((unsigned)nb), dim3(VM_BLOCK), lds, st, a, p, out);
+  else
+    hipLaunchKernelGGL((k_eval<U, uint64_t>), dim3((unsigned)nb), dim3(VM_BLOCK), lds, st, a, p, out);
+  return check_launch("eval");
+}
+static int eval_launch(hipStream_t st, const RowArgs &a, const VProg &p, int64_t *out) {
+  return p.slots <= 4 ? eval_launch_rows<4>(st, a, p, out) : eval_launch_rows<1>(st, a, p, out);
 }
 
 static int check_prog_cols(const aln_insn *prog, int nprog, int ncols) {
@@ -740,6 +834,15 @@ int aln_plain_col(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t se
   return ALN_OK;
 }
 
+static int launch_decode(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_begin, uint64_t n,
+                         int64_t *d_out) {
+  const uint64_t nb = (n + 256 * DEC_ROWS - 1) / (256 * DEC_ROWS);
+  ALN_REQUIRE(nb < (1ull << 31), "decode: grid too large");
+  hipLaunchKernelGGL(k_decode, dim3((unsigned)nb), dim3(256), 0, c->stream, col->words, col->segs, col->nsegs,
+                     seg_rows, row_begin, n, d_out);
+  return check_launch("decode");
+}
+
 int aln_decode(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_begin,
                uint64_t row_end, int64_t *d_out) {
   ALN_REQUIRE(c && col && seg_rows > 0 && row_end >= row_begin, "aln_decode: bad arguments");
@@ -747,9 +850,8 @@ int aln_decode(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_b
   uint64_t n = row_end - row_begin;
   if (!n) return ALN_OK;
   ProfScope p(c, "decode");
-  hipLaunchKernelGGL(k_decode, dim3(grid_for(n, 256, 65536)), dim3(256), 0, c->stream, col->words,
-                     col->segs, col->nsegs, seg_rows, row_begin, n, d_out);
-  return check_launch("decode");
+  ALN_TRY(launch_decode(c, col, seg_rows, row_begin, n, d_out));
+  return ALN_OK;
 }
 
 int aln_gather(aln_ctx *c, const aln_col *col, uint32_t seg_rows, const uint32_t *d_rows,
@@ -758,8 +860,22 @@ int aln_gather(aln_ctx *c, const aln_col *col, uint32_t seg_rows, const uint32_t
   if (!n) return ALN_OK;
   ProfScope p(c, "gather");
   if (col->nsegs == 0) return fill_i64(c, d_out, n, 0);
-  hipLaunchKernelGGL(k_gather, dim3(grid_for(n, 256, 65536)), dim3(256), 0, c->stream, col->words,
-                     col->segs, col->nsegs, seg_rows, d_rows, n, d_out);
+  if (!d_rows && n < (1ull << 32)) return launch_decode(c, col, seg_rows, 0, n, d_out);
+  constexpr int U = 4;
+  RowArgs a;
+  a.ct.words[0] = col->words;
+  a.ct.segs[0] = col->segs;
+  a.nsegs = col->nsegs;
+  a.seg_rows = seg_rows;
+  a.seg_mul = seg_rows > 1 ? ~0ull / seg_rows + 1 : 0;
+  a.rows = d_rows;
+  a.n = n;
+  const uint64_t nb = (n + 256 * U - 1) / (256 * U);
+  ALN_REQUIRE(nb < (1ull << 31), "aln_gather: grid too large");
+  if (narrow_segments(seg_rows))
+    hipLaunchKernelGGL((k_gather<U, uint32_t>), dim3((unsigned)nb), dim3(256), 0, c->stream, a, d_out);
+  else
+    hipLaunchKernelGGL((k_gather<U, uint64_t>), dim3((unsigned)nb), dim3(256), 0, c->stream, a, d_out);
   return check_launch("gather");
 }
 
@@ -770,15 +886,14 @@ int aln_eval(aln_ctx *c, const aln_col *cols, int ncols, uint32_t seg_rows,
   ws_reset(c);
   if (!n) return ALN_OK;
   ALN_TRY(check_prog_cols(prog, nprog, ncols));
-  ColTable *ct;
-  aln_insn *dp;
-  ALN_TRY(upload_cols(c, cols, ncols, &ct));
-  ALN_TRY(upload_prog(c, prog, nprog, &dp));
-  ProfScope p(c, "eval");
+  RowArgs a;
+  VProg p;
+  ALN_TRY(row_args(cols, ncols, seg_rows, d_rows, n, &a));
+  ALN_TRY(check_prog(prog, nprog));
+  vm_lower(prog, nprog, &p);
+  ProfScope ps(c, "eval");
   if (cols[0].nsegs == 0) return fill_i64(c, d_out, n, 0);
-  hipLaunchKernelGGL(k_eval, dim3(grid_for(n, VM_BLOCK, 65536)), dim3(VM_BLOCK), 0, c->stream, ct,
-                     dp, nprog, cols[0].nsegs, seg_rows, d_rows, n, d_out);
-  return check_launch("eval");
+  return eval_launch(c->stream, a, p, d_out);
 }
 
 int aln_apply_perm(aln_ctx *c, const int64_t *d_in, const uint32_t *d_perm, uint64_t n,

@@ -1,6 +1,5 @@
-// Device interpreter of compiled RPN programs (aln_insn).  The program is read from
-// device memory at a wave-uniform index, so instructions come through scalar loads; the
-// value stack lives in LDS, one column of VM_BLOCK entries per depth level.
+// Device interpreter of compiled RPN programs (aln_insn) and the unpacking of column codes for
+// the kernels that run over rows.
 #pragma once
 
 #include <string.h>
@@ -22,57 +21,6 @@ __device__ __forceinline__ int64_t vm_div(int64_t l, int64_t r) {
   return l / r;
 }
 
-// stk points at this thread's entry of depth 0; depth d is stk[d * VM_BLOCK].
-template <typename Load>
-__device__ __forceinline__ int64_t vm_run(const aln_insn *__restrict__ prog, int n, Load load,
-                                          int64_t *stk) {
-  int sp = 0;
-  for (int i = 0; i < n; ++i) {
-    const int op = prog[i].op;
-    if (op == ALN_I_COL) {
-      stk[sp * VM_BLOCK] = wmul(load(prog[i].a), prog[i].k);
-      ++sp;
-    } else if (op == ALN_I_CONST) {
-      stk[sp * VM_BLOCK] = prog[i].k;
-      ++sp;
-    } else if (op == ALN_I_INSET) {
-      const int64_t v = stk[(sp - 1) * VM_BLOCK];
-      const uint32_t *set = reinterpret_cast<const uint32_t *>(prog[i].k);
-      stk[(sp - 1) * VM_BLOCK] = (v >= 0 && v < prog[i].a) ? (set[v >> 5] >> (v & 31)) & 1u : 0;
-    } else if (op == ALN_I_I2F) {
-      int64_t *e = &stk[(sp - 1 - prog[i].a) * VM_BLOCK];
-      *e = f64_bits((double)*e);
-    } else if (op >= ALN_I_FADD) {
-      const double r = bits_f64(stk[(sp - 1) * VM_BLOCK]), l = bits_f64(stk[(sp - 2) * VM_BLOCK]);
-      int64_t v;
-      switch (op) {
-        case ALN_I_FADD: v = f64_bits(l + r); break;
-        case ALN_I_FSUB: v = f64_bits(l - r); break;
-        case ALN_I_FMUL: v = f64_bits(l * r); break;
-        case ALN_I_FDIV: v = f64_bits(l / r); break;
-        default: v = fcmp_code(prog[i].a, l, r); break;
-      }
-      stk[(sp - 2) * VM_BLOCK] = v;
-      --sp;
-    } else {
-      int64_t r = stk[(sp - 1) * VM_BLOCK], l = stk[(sp - 2) * VM_BLOCK], v;
-      switch (op) {
-        case ALN_I_ADD: v = (int64_t)((uint64_t)l + (uint64_t)r); break;
-        case ALN_I_SUB: v = (int64_t)((uint64_t)l - (uint64_t)r); break;
-        case ALN_I_MUL: v = wmul(l, r); break;
-        case ALN_I_DIV: v = vm_div(l, r); break;
-        case ALN_I_CMP: v = cmp_code(prog[i].a, l, r); break;
-        case ALN_I_AND: v = (l != 0) && (r != 0); break;
-        default: v = (l != 0) || (r != 0); break;
-      }
-      stk[(sp - 2) * VM_BLOCK] = v;
-      --sp;
-    }
-  }
-  return stk[0];
-}
-
-// ---- lowered programs --------------------------------------------------------------------------
 // The program as the row kernels run it: U rows per thread and instruction, so that fetching
 // and dispatching an instruction (uniform: scalar loads and branches) is paid once per U rows;
 // the top of the stack in registers, only the values below it in LDS; and a constant or a
@@ -250,12 +198,13 @@ __device__ __forceinline__ void vm_eval(const VProg &p, Load load, int64_t *stk,
   }
 }
 
-// Codes of U rows idx[u] of a packed segment of `bits`-wide codes (both wave-uniform).  Only
-// words that hold a code are read, so a column's last row never touches the next word.  P: a
-// type that idx * bits fits in.
+// Codes of U rows idx[u] of packed `bits`-wide codes, the first `first` (< 32) bits into w
+// (w, bits and first wave-uniform; first 0 when bits is 64).  Only words that hold a code are
+// read, so a column's last row never touches the next word.  P: a type that first + idx * bits
+// fits in.
 template <int U, typename P>
 __device__ __forceinline__ void unpack_codes(const uint32_t *__restrict__ w, uint32_t bits, const P (&idx)[U],
-                                             uint64_t (&c)[U]) {
+                                             uint64_t (&c)[U], uint32_t first = 0) {
   if (bits == 0) {
 #pragma unroll
     for (int u = 0; u < U; ++u) c[u] = 0;
@@ -264,14 +213,14 @@ __device__ __forceinline__ void unpack_codes(const uint32_t *__restrict__ w, uin
     uint32_t lo[U], hi[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const P pos = idx[u] * bits;
+      const P pos = idx[u] * bits + first;
       const uint32_t *q = w + (pos >> 5);
       lo[u] = q[0];
       hi[u] = q[((uint32_t)pos & 31) + bits > 32 ? 1 : 0];
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
-      c[u] = __builtin_amdgcn_alignbit(hi[u], lo[u], (uint32_t)(idx[u] * bits) & 31) & mask;
+      c[u] = __builtin_amdgcn_alignbit(hi[u], lo[u], (uint32_t)(idx[u] * bits + first) & 31) & mask;
   } else if (bits == 64) {
 #pragma unroll
     for (int u = 0; u < U; ++u) __builtin_memcpy(&c[u], w + 2 * idx[u], 8);
@@ -280,7 +229,7 @@ __device__ __forceinline__ void unpack_codes(const uint32_t *__restrict__ w, uin
     uint32_t a[U], b[U], d[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const P pos = idx[u] * bits;
+      const P pos = idx[u] * bits + first;
       const uint32_t *q = w + (pos >> 5);
       a[u] = q[0];
       b[u] = q[1];
@@ -288,7 +237,7 @@ __device__ __forceinline__ void unpack_codes(const uint32_t *__restrict__ w, uin
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const uint32_t s = (uint32_t)(idx[u] * bits) & 31;
+      const uint32_t s = (uint32_t)(idx[u] * bits + first) & 31;
       const uint32_t lo = __builtin_amdgcn_alignbit(b[u], a[u], s), hi = __builtin_amdgcn_alignbit(d[u], b[u], s);
       c[u] = ((uint64_t)hi << 32 | lo) & mask;
     }
