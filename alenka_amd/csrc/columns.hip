@@ -16,17 +16,31 @@ namespace aln {
 
 // ---- encoding -----------------------------------------------------------------------------
 
+// Partial minima and maxima of each segment's blocks, then one wave per segment over its
+// partials.  HBM-bound: 50M values 313 -> 76 us (one atomic pair per wave on the segment's two
+// words, 100,000 of them on 100 addresses, took the rest).
 __global__ void __launch_bounds__(256) k_seg_minmax(const int64_t *__restrict__ v, uint64_t nrows,
                                                     uint32_t seg_rows, uint32_t blocks_per_seg,
-                                                    unsigned long long *mn,
-                                                    unsigned long long *mx) {
-  uint32_t seg = blockIdx.x / blocks_per_seg, part = blockIdx.x % blocks_per_seg;
-  uint64_t s0 = (uint64_t)seg * seg_rows;
-  uint64_t s1 = s0 + seg_rows < nrows ? s0 + seg_rows : nrows;
+                                                    int64_t *__restrict__ pmin, int64_t *__restrict__ pmax) {
+  __shared__ int64_t smn[4], smx[4];
+  const uint32_t seg = blockIdx.x / blocks_per_seg, part = blockIdx.x % blocks_per_seg;
+  const uint64_t s0 = (uint64_t)seg * seg_rows;
+  const uint64_t s1 = s0 + seg_rows < nrows ? s0 + seg_rows : nrows;
+  const uint64_t stride = (uint64_t)blocks_per_seg * 256;
   int64_t lo = INT64_MAX, hi = INT64_MIN;
-  for (uint64_t i = s0 + (uint64_t)part * 256 + threadIdx.x; i < s1;
-       i += (uint64_t)blocks_per_seg * 256) {
-    int64_t x = v[i];
+  uint64_t i = s0 + (uint64_t)part * 256 + threadIdx.x;
+  for (; i + 7 * stride < s1; i += 8 * stride) {  // eight loads in flight per thread
+    int64_t x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = v[i + k * stride];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      lo = x[k] < lo ? x[k] : lo;
+      hi = x[k] > hi ? x[k] : hi;
+    }
+  }
+  for (; i < s1; i += stride) {
+    const int64_t x = v[i];
     lo = x < lo ? x : lo;
     hi = x > hi ? x : hi;
   }
@@ -36,36 +50,94 @@ __global__ void __launch_bounds__(256) k_seg_minmax(const int64_t *__restrict__ 
     hi = b > hi ? b : hi;
   }
   if (__lane_id() == 0) {
-    atomicMin(&mn[seg], (unsigned long long)lo ^ 0x8000000000000000ull);
-    atomicMax(&mx[seg], (unsigned long long)hi ^ 0x8000000000000000ull);
+    smn[threadIdx.x / 64] = lo;
+    smx[threadIdx.x / 64] = hi;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < 4; ++w) {
+      lo = smn[w] < lo ? smn[w] : lo;
+      hi = smx[w] > hi ? smx[w] : hi;
+    }
+    pmin[blockIdx.x] = lo;
+    pmax[blockIdx.x] = hi;
   }
 }
 
-// One thread per output word: gathers the bits of every code overlapping the word.
-__global__ void __launch_bounds__(256) k_pack(const int64_t *__restrict__ v, uint64_t nrows,
-                                              uint32_t seg_rows, uint32_t seg0,
-                                              const aln_seg *__restrict__ segs,
-                                              uint32_t *__restrict__ words) {
-  uint32_t seg = seg0 + blockIdx.y;
-  aln_seg sg = segs[seg];
-  if (sg.bits == 0) return;
-  uint64_t nw = ((uint64_t)sg.nrows * sg.bits + 31) / 32;
-  const int64_t *sv = v + (uint64_t)seg * seg_rows;
-  for (uint64_t w = (uint64_t)blockIdx.x * 256 + threadIdx.x; w < nw;
-       w += (uint64_t)gridDim.x * 256) {
-    uint64_t b0 = w * 32, b1 = b0 + 32;
-    uint64_t r = b0 / sg.bits;
-    uint32_t acc = 0;
-    for (; r < sg.nrows && r * sg.bits < b1; ++r) {
-      uint64_t code = (uint64_t)sv[r] - (uint64_t)sg.base;
-      int64_t sh = (int64_t)(r * sg.bits) - (int64_t)b0;  // bit position of code bit 0
-      if (sh >= 0)
-        acc |= (uint32_t)(code << sh);
-      else
-        acc |= (uint32_t)(code >> (-sh));
-    }
-    words[sg.word_off + w] = acc;
+__global__ void __launch_bounds__(64) k_seg_minmax_final(const int64_t *__restrict__ pmin,
+                                                         const int64_t *__restrict__ pmax, uint32_t blocks_per_seg,
+                                                         uint32_t nsegs, int64_t *__restrict__ out) {
+  const uint32_t seg = blockIdx.x;
+  int64_t lo = INT64_MAX, hi = INT64_MIN;
+  for (uint32_t i = threadIdx.x; i < blocks_per_seg; i += 64) {
+    const int64_t a = pmin[(uint64_t)seg * blocks_per_seg + i], b = pmax[(uint64_t)seg * blocks_per_seg + i];
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
   }
+  for (int o = 32; o > 0; o >>= 1) {
+    int64_t a = __shfl_xor(lo, o, 64), b = __shfl_xor(hi, o, 64);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  if (threadIdx.x == 0) {
+    out[seg] = lo;
+    out[nsegs + seg] = hi;
+  }
+}
+
+// A tile of 2048 rows per block, so that it starts on a word: a thread concatenates the codes of
+// 8 consecutive rows in registers and ORs the words they make into LDS (two threads share only
+// the words at their ends), and the tile's words are stored as whole lines (50M 24-bit codes
+// 137 -> 93 us, 5.9 TB/s; a thread per word read its rows again and divided to find them).
+constexpr int PK_ROWS = 8;
+constexpr int PK_TILE = 256 * PK_ROWS;
+__global__ void __launch_bounds__(256) k_pack(const int64_t *__restrict__ v, uint32_t seg_rows, uint32_t seg0,
+                                              const aln_seg *__restrict__ segs, uint32_t *__restrict__ words) {
+  __shared__ uint32_t out[PK_TILE / 32 * 64];
+  const uint32_t seg = seg0 + blockIdx.y;
+  const aln_seg sg = segs[seg];
+  const uint64_t t0 = (uint64_t)blockIdx.x * PK_TILE;
+  if (sg.bits == 0 || t0 >= sg.nrows) return;
+  const uint32_t m = sg.nrows - t0 < PK_TILE ? (uint32_t)(sg.nrows - t0) : PK_TILE;
+  const uint32_t nw = (m * sg.bits + 31) / 32;
+  const int64_t *sv = v + (uint64_t)seg * seg_rows + t0;
+  const uint32_t r0 = threadIdx.x * PK_ROWS;
+  int64_t x[PK_ROWS];
+  if (r0 + PK_ROWS <= m) {
+#pragma unroll
+    for (int j = 0; j < PK_ROWS; ++j) x[j] = sv[r0 + j];
+  } else {
+#pragma unroll
+    for (int j = 0; j < PK_ROWS; ++j) x[j] = r0 + j < m ? sv[r0 + j] : sg.base;
+  }
+  for (uint32_t w = threadIdx.x; w < nw; w += 256) out[w] = 0;
+  __syncthreads();
+  if (r0 < m) {
+    const uint32_t bits = sg.bits, lb = bits < 32 ? bits : 32, hb = bits - lb;
+    const uint32_t lmask = lb == 32 ? 0xFFFFFFFFu : (1u << lb) - 1u, hmask = hb == 32 ? 0xFFFFFFFFu : (1u << hb) - 1u;
+    uint32_t w = r0 * bits >> 5, fill = r0 * bits & 31;
+    uint64_t acc = 0;
+    auto put = [&](uint32_t part, uint32_t width) {
+      acc |= (uint64_t)part << fill;
+      fill += width;
+      if (fill >= 32) {
+        if (w < nw) atomicOr(&out[w], (uint32_t)acc);
+        ++w;
+        acc >>= 32;
+        fill -= 32;
+      }
+    };
+#pragma unroll
+    for (int j = 0; j < PK_ROWS; ++j) {  // rows past the end are code 0
+      const uint64_t code = (uint64_t)x[j] - (uint64_t)sg.base;
+      put((uint32_t)code & lmask, lb);
+      if (hb) put((uint32_t)(code >> 32) & hmask, hb);
+    }
+    if (fill && w < nw) atomicOr(&out[w], (uint32_t)acc);
+  }
+  __syncthreads();
+  uint32_t *dst = words + sg.word_off + t0 / 32 * sg.bits;
+  for (uint32_t w = threadIdx.x; w < nw; w += 256) __builtin_nontemporal_store(out[w], dst + w);
 }
 
 // ---- row-wise kernels ---------------------------------------------------------------------
@@ -744,29 +816,28 @@ int aln_encode_plan(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t 
   uint32_t nsegs = (uint32_t)((nrows + seg_rows - 1) / seg_rows);
   *h_words = 0;
   if (nsegs == 0) return ALN_OK;
-  unsigned long long *mm;
+  const uint32_t bps = (uint32_t)grid_for(seg_rows, 256 * 16, 256);
+  int64_t *part, *mm;
+  ALN_TRY(ws(c, 2 * (size_t)nsegs * bps, &part));
   ALN_TRY(ws(c, 2 * (size_t)nsegs, &mm));
-  std::vector<unsigned long long> init(2 * (size_t)nsegs);
-  for (uint32_t s = 0; s < nsegs; ++s) {
-    init[s] = ~0ull;
-    init[nsegs + s] = 0;
-  }
-  ALN_HIP(hipMemcpyAsync(mm, init.data(), 16 * (size_t)nsegs, hipMemcpyHostToDevice, c->stream));
-  uint32_t bps = (uint32_t)grid_for(seg_rows, 256 * 16, 256);
   {
     ProfScope p(c, "seg_minmax");
+    int64_t *pmax = part + (size_t)nsegs * bps;
     hipLaunchKernelGGL(k_seg_minmax, dim3(nsegs * bps), dim3(256), 0, c->stream, d_vals, nrows,
-                       seg_rows, bps, mm, mm + nsegs);
+                       seg_rows, bps, part, pmax);
+    hipLaunchKernelGGL(k_seg_minmax_final, dim3(nsegs), dim3(64), 0, c->stream, (const int64_t *)part,
+                       (const int64_t *)pmax, bps, nsegs, mm);
   }
   ALN_TRY(check_launch("seg_minmax"));
-  ALN_TRY(copy_to_host(c, init.data(), mm, 16 * (size_t)nsegs));
+  std::vector<int64_t> range(2 * (size_t)nsegs);
+  ALN_TRY(copy_to_host(c, range.data(), mm, 16 * (size_t)nsegs));
   uint64_t off = 0;
   for (uint32_t s = 0; s < nsegs; ++s) {
     aln_seg &g = h_segs[s];
     uint64_t r0 = (uint64_t)s * seg_rows;
     g.nrows = (uint32_t)((r0 + seg_rows <= nrows) ? seg_rows : nrows - r0);
-    g.vmin = (int64_t)(init[s] ^ 0x8000000000000000ull);
-    g.vmax = (int64_t)(init[nsegs + s] ^ 0x8000000000000000ull);
+    g.vmin = range[s];
+    g.vmax = range[nsegs + s];
     g.base = g.vmin;
     g.bits = bits_for_range_u((uint64_t)g.vmax - (uint64_t)g.vmin);
     if (force_bits) {
@@ -788,7 +859,7 @@ int aln_encode_pack(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t 
   ws_reset(c);
   uint32_t nsegs = (uint32_t)((nrows + seg_rows - 1) / seg_rows);
   if (nsegs == 0) return ALN_OK;
-  uint64_t maxw = 0;
+  uint64_t maxw = 0, maxr = 0;
   for (uint32_t s = 0; s < nsegs; ++s) {
     uint64_t r0 = (uint64_t)s * seg_rows;
     uint32_t nr = (uint32_t)((r0 + seg_rows <= nrows) ? seg_rows : nrows - r0);
@@ -796,6 +867,7 @@ int aln_encode_pack(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t 
                 "aln_encode_pack: descriptor %u does not match the plan", s);
     uint64_t w = ((uint64_t)nr * h_segs[s].bits + 31) / 32;
     maxw = w > maxw ? w : maxw;
+    maxr = nr > maxr ? nr : maxr;
   }
   ALN_REQUIRE(maxw == 0 || d_words, "aln_encode_pack: no word buffer");
   ALN_HIP(hipMemcpyAsync(d_segs, h_segs, sizeof(aln_seg) * nsegs, hipMemcpyHostToDevice, c->stream));
@@ -803,8 +875,8 @@ int aln_encode_pack(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t 
     ProfScope p(c, "pack");
     for (uint32_t s0 = 0; s0 < nsegs; s0 += 65535) {
       uint32_t ns = nsegs - s0 < 65535 ? nsegs - s0 : 65535;
-      hipLaunchKernelGGL(k_pack, dim3(grid_for(maxw, 256, 4096), ns), dim3(256), 0, c->stream,
-                         d_vals, nrows, seg_rows, s0, d_segs, d_words);
+      hipLaunchKernelGGL(k_pack, dim3(grid_for(maxr, PK_TILE), ns), dim3(256), 0, c->stream,
+                         d_vals, seg_rows, s0, (const aln_seg *)d_segs, d_words);
     }
   }
   ALN_TRY(check_launch("pack"));

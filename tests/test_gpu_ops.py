@@ -71,6 +71,32 @@ def test_encode_decode(ctx, name, gen, n, seg_rows):
     assert np.array_equal(host(got), v[rows])
 
 
+@pytest.mark.parametrize("n,seg_rows", [(7, 7), (2047, 5000), (2049, 2049), (4129, 4096), (6200, 3000)])
+def test_codec_every_width(ctx, n, seg_rows):
+    """Every code width, natural and forced, at the edges of the 2048-row tiles the codes are
+    packed and unpacked in: the words are the oracle's and decode to the values."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n)
+    for bits in range(1, 65):
+        lo = 0 if bits < 63 else -(1 << 62)
+        v = (r.integers(0, 1 << min(bits, 62), n) + lo).astype(np.int64)
+        if bits == 64:
+            v[:: 3], v[1:: 3] = -(1 << 63), (1 << 63) - 1
+        for force in (0, bits, 64):
+            col = D.Column.encode(ctx, dev(ctx, v), seg_rows, force_bits=force)
+            words = host(col.words).view(np.uint32)
+            for s in range(col.nsegs):
+                sg = col.hsegs[s]
+                nw = (sg.nrows * sg.bits + 31) // 32
+                if force:
+                    assert sg.bits == force
+                if nw:
+                    part = v[s * seg_rows: s * seg_rows + sg.nrows]
+                    assert np.array_equal(words[sg.word_off: sg.word_off + nw], O.pack(part, sg.base, sg.bits)[:nw])
+            assert np.array_equal(host(col.decode(ctx)), v), (bits, force)
+
+
 # ---- scan / filter -----------------------------------------------------------------------
 NAME, NUM, CMP, AND, OR = L.RPN_NAME, L.RPN_NUMBER, L.RPN_CMP, L.RPN_AND, L.RPN_OR
 PREDICATES = [
