@@ -112,6 +112,18 @@ int check_launch(const char *name);
 int copy_to_host(aln_ctx *c, void *h, const void *d, size_t bytes);  // synchronous
 int copy_to_device(aln_ctx *c, void *d, const void *h, size_t bytes);
 
+// Results a kernel hands to the host itself: it writes them to dst and calls result_done after
+// its last write (one thread, after a fence by any other that wrote).  dst is coherent host
+// memory whose flag word the host polls, or (flag NULL) a device buffer that is copied.  One
+// at a time per context, and no copy_to_host between open and wait.
+struct DevResult {
+  uint64_t *dst;
+  uint32_t *flag;
+  uint32_t seq;
+};
+int result_open(aln_ctx *c, size_t words, DevResult *r);
+int result_wait(aln_ctx *c, const DevResult &r, void *h, size_t bytes);
+
 // ---- shared utilities (host) -------------------------------------------------------------
 int exclusive_scan_u32(aln_ctx *c, const uint32_t *d_in, uint64_t n, uint64_t *d_out,
                        uint64_t *h_total);
@@ -126,6 +138,8 @@ int exclusive_scan_u32_buf(hipStream_t s, const uint32_t *d_in, uint64_t n, uint
 // must be current; once per device, later calls return the recorded status.
 int scan_scratch_attach(int device);
 int minmax_i64(aln_ctx *c, const int64_t *d, uint64_t n, int64_t *h_min, int64_t *h_max);
+// The same of nk (<= ALN_MAX_KEYS) arrays of n values, one pair of launches and one wait.
+int minmax_keys(aln_ctx *c, const int64_t *const *d, int nk, uint64_t n, int64_t *h_min, int64_t *h_max);
 int sum_u32(aln_ctx *c, const uint32_t *d_in, uint64_t n, uint64_t *d_out);  // no sync
 // *out[i] += sum of in[i][0, n[i]) for up to SUM_MULTI_MAX arrays, one launch (no sync);
 // for the arrays whose bit is set in popc, the number of set bits of the words instead
@@ -182,6 +196,12 @@ struct DevProg {
 
 // ---- device helpers ---------------------------------------------------------------------
 namespace aln {
+
+__device__ __forceinline__ void result_done(const DevResult &r) {
+  if (!r.flag) return;
+  __threadfence_system();
+  __hip_atomic_store(r.flag, r.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
 
 // Code of row `i` of a segment of width `bits` starting at word `w`.  Reads only the
 // words that hold the code, so a segment's last row never touches the next word.

@@ -119,13 +119,14 @@ static bool readback_ready(aln_ctx *c) {
   return true;
 }
 
-static int readback_small(aln_ctx *c, void *h, const void *d, size_t bytes) {
+static uint32_t readback_seq(aln_ctx *c) {
   uint32_t seq = ++c->rb_seq;
   if (seq == 0) seq = ++c->rb_seq;  // 0 is the buffer's initial value
+  return seq;
+}
+
+static int readback_wait(aln_ctx *c, uint32_t seq, void *h, size_t bytes) {
   volatile uint32_t *flag = reinterpret_cast<volatile uint32_t *>(static_cast<char *>(c->rb) + RB_BYTES);
-  hipLaunchKernelGGL(k_readback, dim3(1), dim3(256), 0, c->stream, static_cast<const uint32_t *>(d),
-                     (uint32_t)((bytes + 3) / 4), c->rb_dev, c->rb_dev + RB_BYTES / 4, seq);
-  ALN_TRY(check_launch("readback"));
   // poll; after a while give the thread up between polls, and after 200 ms fall back to a
   // stream synchronisation (which also reports a failed launch)
   const auto t0 = std::chrono::steady_clock::now();
@@ -143,6 +144,31 @@ static int readback_small(aln_ctx *c, void *h, const void *d, size_t bytes) {
   std::atomic_thread_fence(std::memory_order_acquire);
   memcpy(h, c->rb, bytes);
   return ALN_OK;
+}
+
+static int readback_small(aln_ctx *c, void *h, const void *d, size_t bytes) {
+  const uint32_t seq = readback_seq(c);
+  hipLaunchKernelGGL(k_readback, dim3(1), dim3(256), 0, c->stream, static_cast<const uint32_t *>(d),
+                     (uint32_t)((bytes + 3) / 4), c->rb_dev, c->rb_dev + RB_BYTES / 4, seq);
+  ALN_TRY(check_launch("readback"));
+  return readback_wait(c, seq, h, bytes);
+}
+
+int result_open(aln_ctx *c, size_t words, DevResult *r) {
+  if (words * 8 <= RB_BYTES && readback_ready(c)) {
+    r->dst = reinterpret_cast<uint64_t *>(c->rb_dev);
+    r->flag = c->rb_dev + RB_BYTES / 4;
+    r->seq = readback_seq(c);
+    return ALN_OK;
+  }
+  r->flag = nullptr;
+  r->seq = 0;
+  return ws(c, words, &r->dst);
+}
+
+int result_wait(aln_ctx *c, const DevResult &r, void *h, size_t bytes) {
+  if (r.flag) return readback_wait(c, r.seq, h, bytes);
+  return copy_to_host(c, h, r.dst, bytes);
 }
 
 int copy_to_host(aln_ctx *c, void *h, const void *d, size_t bytes) {
@@ -318,6 +344,55 @@ static int exclusive_scan_launch(hipStream_t s, const T *d_in, uint64_t n, uint6
   return check_launch("exclusive_scan");
 }
 
+// A scan of up to SCAN_ONE items by one block (16 waves of 16 rows of 64 items), which also
+// hands the total to the host: one launch where the tile scan takes three and a readback.
+constexpr uint32_t SCAN_ONE_WAVES = 16;
+constexpr uint64_t SCAN_ONE = SCAN_ONE_WAVES * 64 * SCAN_ITEMS;
+template <typename T>
+__global__ void __launch_bounds__(64 * SCAN_ONE_WAVES) k_scan_one(const T *__restrict__ in, uint32_t n,
+                                                                  uint64_t *__restrict__ out, DevResult r) {
+  __shared__ uint64_t wsum[SCAN_ONE_WAVES];
+  const unsigned lane = __lane_id(), wid = threadIdx.x / 64;
+  // rows of a wave: as few as cover n, so that short inputs spread over the waves
+  const uint32_t rows = (n + 64 * SCAN_ONE_WAVES - 1) / (64 * SCAN_ONE_WAVES);
+  const uint32_t base = wid * rows * 64 + lane;
+  uint64_t v[SCAN_ITEMS];
+#pragma unroll
+  for (int j = 0; j < SCAN_ITEMS; ++j) {
+    const uint32_t i = base + (uint32_t)j * 64;
+    v[j] = (uint32_t)j < rows && i < n ? (uint64_t)in[i] : 0;
+  }
+  uint64_t carry = 0;
+#pragma unroll
+  for (int j = 0; j < SCAN_ITEMS; ++j) {
+    if ((uint32_t)j >= rows) break;
+    uint64_t x = v[j];
+    for (int o = 1; o < 64; o <<= 1) {
+      const uint64_t y = __shfl_up(x, o, 64);
+      if (lane >= (unsigned)o) x += y;
+    }
+    const uint64_t row = __shfl(x, 63, 64);
+    v[j] = carry + x - v[j];
+    carry += row;
+  }
+  if (lane == 0) wsum[wid] = carry;
+  __syncthreads();
+  uint64_t off = 0, total = 0;
+  for (unsigned w = 0; w < SCAN_ONE_WAVES; ++w) {
+    off += w < wid ? wsum[w] : 0;
+    total += wsum[w];
+  }
+#pragma unroll
+  for (int j = 0; j < SCAN_ITEMS; ++j) {
+    const uint32_t i = base + (uint32_t)j * 64;
+    if ((uint32_t)j < rows && i < n) out[i] = off + v[j];
+  }
+  if (threadIdx.x == 0) {
+    r.dst[0] = total;
+    result_done(r);
+  }
+}
+
 uint64_t scan_tiles(uint64_t n) {
   const uint64_t nt = (n + SCAN_TILE - 1) / SCAN_TILE;
   return nt == 0 ? 1 : nt;
@@ -331,6 +406,16 @@ int exclusive_scan_u32_buf(hipStream_t s, const uint32_t *d_in, uint64_t n, uint
 template <typename T>
 static int exclusive_scan_impl(aln_ctx *c, const T *d_in, uint64_t n, uint64_t *d_out,
                                uint64_t *h_total) {
+  if (h_total && n <= SCAN_ONE) {
+    DevResult r;
+    ALN_TRY(result_open(c, 1, &r));
+    {
+      ProfScope p(c, "scan");
+      hipLaunchKernelGGL(k_scan_one<T>, dim3(1), dim3(64 * SCAN_ONE_WAVES), 0, c->stream, d_in, (uint32_t)n, d_out, r);
+    }
+    ALN_TRY(check_launch("exclusive_scan"));
+    return result_wait(c, r, h_total, 8);
+  }
   uint64_t *sums, *tot;
   ALN_TRY(ws(c, scan_tiles(n), &sums));
   ALN_TRY(ws(c, 1, &tot));
@@ -426,12 +511,14 @@ int sum_u32_multi(aln_ctx *c, int k, const uint32_t *const *in, const uint64_t *
   return check_launch("sum_u32_multi");
 }
 
-// Min/max of an int64 array: per-block partials, then one block folds them (no atomics on
-// a shared address).
-__global__ void __launch_bounds__(256) k_minmax_part(const int64_t *__restrict__ d, uint64_t n,
-                                                     int64_t *__restrict__ pmin,
-                                                     int64_t *__restrict__ pmax) {
+// Min/max of int64 arrays (one per grid row): per-block partials, then one block folds them
+// (no atomics on a shared address) and hands the results to the host.
+struct MinmaxSet {
+  const int64_t *d[ALN_MAX_KEYS];
+};
+__global__ void __launch_bounds__(256) k_minmax_part(MinmaxSet set, uint64_t n, int64_t *__restrict__ part) {
   __shared__ int64_t smn[4], smx[4];
+  const int64_t *__restrict__ d = set.d[blockIdx.y];
   int64_t lo = INT64_MAX, hi = INT64_MIN;
   const uint64_t stride = (uint64_t)gridDim.x * 256;
   uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
@@ -466,32 +553,67 @@ __global__ void __launch_bounds__(256) k_minmax_part(const int64_t *__restrict__
       lo = smn[w] < lo ? smn[w] : lo;
       hi = smx[w] > hi ? smx[w] : hi;
     }
-    lo = smn[0] < lo ? smn[0] : lo;
-    hi = smx[0] > hi ? smx[0] : hi;
-    pmin[blockIdx.x] = lo;
-    pmax[blockIdx.x] = hi;
+    part[2 * ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x)] = lo;
+    part[2 * ((uint64_t)blockIdx.y * gridDim.x + blockIdx.x) + 1] = hi;
   }
 }
 
-int minmax_i64(aln_ctx *c, const int64_t *d, uint64_t n, int64_t *h_min, int64_t *h_max) {
-  const unsigned nb = grid_for(n, 256 * 16, 2048);  // 8 blocks per CU; 32 KB of partials
+// Wave k folds the nb partials of array k.
+__global__ void __launch_bounds__(64 * ALN_MAX_KEYS) k_minmax_final(const int64_t *__restrict__ part, uint32_t nb,
+                                                                    DevResult r) {
+  const uint32_t k = threadIdx.x / 64;
+  int64_t lo = INT64_MAX, hi = INT64_MIN;
+#pragma unroll 8
+  for (uint32_t i = __lane_id(); i < nb; i += 64) {
+    const int64_t a = part[2 * ((uint64_t)k * nb + i)], b = part[2 * ((uint64_t)k * nb + i) + 1];
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    int64_t a = __shfl_xor(lo, o, 64), b = __shfl_xor(hi, o, 64);
+    lo = a < lo ? a : lo;
+    hi = b > hi ? b : hi;
+  }
+  if (__lane_id() == 0) {
+    r.dst[2 * k] = (uint64_t)lo;
+    r.dst[2 * k + 1] = (uint64_t)hi;
+    __threadfence_system();
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) result_done(r);
+}
+
+int minmax_keys(aln_ctx *c, const int64_t *const *d, int nk, uint64_t n, int64_t *h_min, int64_t *h_max) {
+  ALN_REQUIRE(nk >= 1 && nk <= ALN_MAX_KEYS, "minmax: %d arrays", nk);
+  for (int k = 0; k < nk; ++k) {
+    h_min[k] = INT64_MAX;
+    h_max[k] = INT64_MIN;
+  }
+  if (!n) return ALN_OK;
+  const unsigned nb = grid_for(n, 256 * 16, 2048);  // 8 blocks per CU
   int64_t *part;
-  ALN_TRY(ws(c, 2 * (size_t)nb, &part));
-  if (n) {
+  ALN_TRY(ws(c, 2 * (size_t)nb * nk, &part));
+  MinmaxSet set;
+  for (int k = 0; k < nk; ++k) set.d[k] = d[k];
+  DevResult r;
+  ALN_TRY(result_open(c, 2 * ALN_MAX_KEYS, &r));
+  {
     ProfScope p(c, "minmax");
-    hipLaunchKernelGGL(k_minmax_part, dim3(nb), dim3(256), 0, c->stream, d, n, part, part + nb);
+    hipLaunchKernelGGL(k_minmax_part, dim3(nb, nk), dim3(256), 0, c->stream, set, n, part);
+    hipLaunchKernelGGL(k_minmax_final, dim3(1), dim3(64 * nk), 0, c->stream, (const int64_t *)part, nb, r);
   }
   ALN_TRY(check_launch("minmax"));
-  std::vector<int64_t> h(2 * (size_t)nb);
-  *h_min = INT64_MAX;
-  *h_max = INT64_MIN;
-  if (!n) return ALN_OK;
-  ALN_TRY(copy_to_host(c, h.data(), part, 16ull * nb));
-  for (unsigned i = 0; i < nb; ++i) {
-    *h_min = h[i] < *h_min ? h[i] : *h_min;
-    *h_max = h[nb + i] > *h_max ? h[nb + i] : *h_max;
+  int64_t h[2 * ALN_MAX_KEYS];
+  ALN_TRY(result_wait(c, r, h, 16 * (size_t)nk));
+  for (int k = 0; k < nk; ++k) {
+    h_min[k] = h[2 * k];
+    h_max[k] = h[2 * k + 1];
   }
   return ALN_OK;
+}
+
+int minmax_i64(aln_ctx *c, const int64_t *d, uint64_t n, int64_t *h_min, int64_t *h_max) {
+  return minmax_keys(c, &d, 1, n, h_min, h_max);
 }
 
 template <typename T>

@@ -948,7 +948,7 @@ int radix_sort_pairs(aln_ctx *c, uint64_t *d_keys, uint32_t *d_vals, uint64_t n,
   return rs_sort(c, in, false, n, bits, d_keys, d_vals);
 }
 
-// Range of every key column: one min/max pass each.
+// Range of every key column.
 struct KeyRanges {
   int64_t mn[ALN_MAX_KEYS], mx[ALN_MAX_KEYS];
   uint32_t bits[ALN_MAX_KEYS], total;
@@ -956,8 +956,8 @@ struct KeyRanges {
 
 static int key_ranges(aln_ctx *c, const int64_t *const *keys, int nkeys, uint64_t n, KeyRanges *r) {
   r->total = 0;
+  ALN_TRY(minmax_keys(c, keys, nkeys, n, r->mn, r->mx));
   for (int k = 0; k < nkeys; ++k) {
-    ALN_TRY(minmax_i64(c, keys[k], n, &r->mn[k], &r->mx[k]));
     r->bits[k] = bits_for_range_u((uint64_t)r->mx[k] - (uint64_t)r->mn[k]);
     r->total += r->bits[k];
   }

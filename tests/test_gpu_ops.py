@@ -435,6 +435,19 @@ def test_hash_join(ctx, case):
         assert sorted(zip(ol.tolist(), orr.tolist())) == sorted(zip(pi.tolist(), bi.tolist()))
 
 
+@pytest.mark.parametrize("ntiles", [1, 2, 64, 65, 1023, 1025, 16383, 16384, 16385])
+def test_scan_tile_counts(ctx, ntiles):
+    """Row ids of a scan whose tile counts are scanned by one wave row, one block (up to 16384
+    tiles) or the tile scan: one-row segments, of which about a third pass."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(ntiles)
+    v = r.integers(0, 3, ntiles).astype(np.int64)
+    col = D.Column.plain(ctx, dev(ctx, v), 1)
+    got = host(D.scan_filter(ctx, [col], [(L.I_COL, 0, 1), (L.I_CONST, 0, 1), (L.I_CMP, 4, 0)]))
+    assert np.array_equal(got, np.nonzero(v == 1)[0])
+
+
 J_NOKEY = 0x9A7C0F53D1B24E86 - (1 << 64)  # the join table's mark of a free entry
 
 
