@@ -14,6 +14,8 @@
 //     segmented wave scan, and each block adds its rows into an LDS table first, so hot
 //     keys and small group counts aggregate in LDS and reach the global table once per
 //     block;
+//   * few codes (all accumulators fit in LDS): every block keeps them all, in one copy per
+//     lane while they fit, and the blocks' results are added up at the end;
 //   * no GROUP BY (or keys that never vary) is one group: a block reduction;
 //   * the groups are compacted and put in the reference's output order: ascending key
 //     tuple (one segment) or ascending MurmurHash64A(keys, 8*nkeys, seed) (the
@@ -46,9 +48,10 @@ struct GbArgs {
   int64_t kmin[ALN_MAX_KEYS];
   uint32_t shift[ALN_MAX_KEYS];
   uint64_t fmask[ALN_MAX_KEYS];
-  const int64_t *vals[ALN_MAX_AGGS];
-  int32_t aggs[ALN_MAX_AGGS];
-  int64_t *tab[ALN_MAX_AGGS];
+  // one more than a call can ask for: the few-groups path counts rows by itself
+  const int64_t *vals[ALN_MAX_AGGS + 1];
+  int32_t aggs[ALN_MAX_AGGS + 1];
+  int64_t *tab[ALN_MAX_AGGS + 1];
   int nk, nv;
 };
 
@@ -269,6 +272,200 @@ __global__ void __launch_bounds__(256) k_gb_agg(GbArgs a, uint64_t n, uint64_t *
   }
 }
 
+// ---- few groups: all accumulators in LDS -----------------------------------------------------
+// Every block keeps an accumulator per (aggregate, code), in 2^lr copies spread over the lanes
+// (one bank column each: with 64 copies a wave's LDS atomics never meet), so no row touches
+// global memory and no wave-wide combination is needed; the blocks' accumulators go to part[]
+// and one wave per accumulator adds them up.  60M rows, 8 codes, count + 2 sums + f64 sum, min,
+// max: 3.68 ms (a segmented wave scan of every value and one copy) -> 0.53 ms, 6.3 TB/s.
+// Bounded by HBM: the keys and values once.  f64 MIN / MAX are kept as int64 keys in the order
+// of the doubles (NaN never enters, as in agg_combine).
+constexpr int GL_U = 8;  // rows of a thread in flight
+constexpr size_t GL_COPIES = 32768;  // copies are made while they fit this
+constexpr size_t GL_MOST = 65536;    // one copy fits this
+constexpr uint64_t GL_PART = 1ull << 22;  // block results kept, at most (accumulators x blocks)
+
+constexpr uint64_t GL_SAMPLE_MIN = 1ull << 20;  // rows from which a sample's ranges are tried
+constexpr uint32_t GL_SAMPLE_BITS = 10;  // and the codes: wider ranges than 1024 values are
+                                         // seldom hit in full by a sample of 16384 rows
+
+struct GlArgs {
+  GbArgs g;         // g.nv accumulators per code, accumulator `cnt` the row count
+  int cnt;
+  uint32_t ncodes, lr;
+};
+
+__device__ __forceinline__ int64_t gl_identity(int a) { return f64_unorder_key(agg_identity(a)); }
+
+// Combines accumulators (f64 MIN / MAX as keys).
+__device__ __forceinline__ int64_t gl_combine(int a, int64_t x, int64_t y) {
+  if (a == ALN_AGG_MIN || a == ALN_AGG_FMIN) return x < y ? x : y;
+  if (a == ALN_AGG_MAX || a == ALN_AGG_FMAX) return x > y ? x : y;
+  return agg_combine(a, x, y);
+}
+
+__global__ void __launch_bounds__(256) k_gl_agg(GlArgs a, uint64_t n, int64_t *__restrict__ part,
+                                                uint32_t *__restrict__ bad) {
+  extern __shared__ __align__(16) int64_t gl_acc[];
+  const uint32_t per = a.ncodes << a.lr;  // one aggregate's accumulators
+  for (int v = 0; v < a.g.nv; ++v) {
+    const int64_t id = a.g.aggs[v] == ALN_AGG_FMIN || a.g.aggs[v] == ALN_AGG_FMAX ? gl_identity(a.g.aggs[v])
+                                                                                 : agg_identity(a.g.aggs[v]);
+    for (uint32_t i = threadIdx.x; i < per; i += 256) gl_acc[(size_t)v * per + i] = id;
+  }
+  __syncthreads();
+  const uint32_t copy = threadIdx.x & ((1u << a.lr) - 1u);
+  bool outside = false;
+  for (uint64_t i0 = (uint64_t)blockIdx.x * (256 * GL_U); i0 < n; i0 += (uint64_t)gridDim.x * (256 * GL_U)) {
+    uint32_t at[GL_U];
+    bool in[GL_U];
+#pragma unroll
+    for (int u = 0; u < GL_U; ++u) {
+      at[u] = 0;
+      in[u] = i0 + threadIdx.x + 256 * u < n;
+    }
+    for (int k = 0; k < a.g.nk; ++k) {
+      const int64_t *__restrict__ key = a.g.keys[k] + i0 + threadIdx.x;
+      const uint64_t kmin = (uint64_t)a.g.kmin[k], fmask = a.g.fmask[k];
+      const uint32_t sh = a.g.shift[k] + a.lr;
+      int64_t x[GL_U];
+#pragma unroll
+      for (int u = 0; u < GL_U; ++u) x[u] = in[u] ? __builtin_nontemporal_load(key + 256 * u) : (int64_t)kmin;
+#pragma unroll
+      for (int u = 0; u < GL_U; ++u) {
+        const uint64_t d = (uint64_t)x[u] - kmin;
+        outside = outside || d > fmask;
+        in[u] = in[u] && d <= fmask;
+        at[u] |= (uint32_t)(d & fmask) << sh;
+      }
+    }
+    for (int v = 0; v < a.g.nv; ++v) {
+      const int ag = a.g.aggs[v];
+      int64_t *acc = gl_acc + (size_t)v * per + copy;
+      if (ag == ALN_AGG_COUNT) {
+#pragma unroll
+        for (int u = 0; u < GL_U; ++u)
+          if (in[u]) atomicAdd((unsigned long long *)(acc + at[u]), 1ull);
+        continue;
+      }
+      const int64_t *__restrict__ val = a.g.vals[v] + i0 + threadIdx.x;
+      int64_t x[GL_U];
+#pragma unroll
+      for (int u = 0; u < GL_U; ++u) x[u] = in[u] ? __builtin_nontemporal_load(val + 256 * u) : 0;
+#define GL_EACH(cond, stmt)                     \
+  _Pragma("unroll") for (int u = 0; u < GL_U; ++u) { \
+    int64_t *t = acc + at[u];                   \
+    const int64_t y = x[u];                     \
+    if (in[u] && (cond)) stmt;                  \
+  }                                             \
+  break
+      switch (ag) {
+        case ALN_AGG_SUM: GL_EACH(true, atomicAdd((unsigned long long *)t, (unsigned long long)y));
+        case ALN_AGG_MIN: GL_EACH(true, atomicMin((long long *)t, (long long)y));
+        case ALN_AGG_MAX: GL_EACH(true, atomicMax((long long *)t, (long long)y));
+        case ALN_AGG_FSUM: GL_EACH(true, atomicAdd(reinterpret_cast<double *>(t), bits_f64(y)));
+        case ALN_AGG_FMIN: GL_EACH(bits_f64(y) == bits_f64(y), atomicMin((long long *)t, (long long)f64_unorder_key(y)));
+        default: GL_EACH(bits_f64(y) == bits_f64(y), atomicMax((long long *)t, (long long)f64_unorder_key(y)));
+      }
+#undef GL_EACH
+    }
+  }
+  if (outside) *bad = 1;
+  __syncthreads();
+  const uint32_t nacc = a.ncodes * (uint32_t)a.g.nv;
+  for (uint32_t s = threadIdx.x; s < nacc; s += 256) {
+    const int ag = a.g.aggs[s / a.ncodes];
+    const int64_t *t = gl_acc + ((size_t)s << a.lr);
+    int64_t r = t[0];
+    for (uint32_t c = 1; c < (1u << a.lr); ++c) r = gl_combine(ag, r, t[c]);
+    part[(uint64_t)s * gridDim.x + blockIdx.x] = r;
+  }
+}
+
+// One wave per accumulator: the blocks' results into the tables (g.tab[v][code]).
+__global__ void __launch_bounds__(256) k_gl_sum(GlArgs a, const int64_t *__restrict__ part, uint32_t nb) {
+  const uint32_t s = blockIdx.x * 4 + threadIdx.x / 64;
+  if (s >= a.ncodes * (uint32_t)a.g.nv) return;
+  const int v = (int)(s / a.ncodes), ag = a.g.aggs[v];
+  const int64_t *__restrict__ p = part + (uint64_t)s * nb;
+  // lanes past the blocks repeat block 0's MIN / MAX, or add nothing
+  const bool sum = ag == ALN_AGG_COUNT || ag == ALN_AGG_SUM || ag == ALN_AGG_FSUM;
+  int64_t r = __lane_id() < nb ? p[__lane_id()] : sum ? 0 : p[0];
+  for (uint32_t b = 64 + __lane_id(); b < nb; b += 64) r = gl_combine(ag, r, p[b]);
+  for (int o = 32; o > 0; o >>= 1) r = gl_combine(ag, r, (int64_t)__shfl_xor((long long)r, o, 64));
+  if (__lane_id() == 0)
+    a.g.tab[v][s - v * a.ncodes] = ag == ALN_AGG_FMIN || ag == ALN_AGG_FMAX ? f64_unorder_key(r) : r;
+}
+
+// The groups (codes with rows) in code order into the outputs, at most cap of them; the number
+// of groups and whether a key lay outside the code range to the host.
+__global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uint64_t cap,
+                                                  const uint32_t *__restrict__ bad, DevResult r) {
+  __shared__ uint32_t wsum[16];
+  uint64_t base = 0;
+  for (uint32_t c0 = 0; c0 < a.ncodes; c0 += 1024) {
+    const uint32_t c = c0 + threadIdx.x;
+    const bool f = c < a.ncodes && a.g.tab[a.cnt][c] != 0;
+    const uint64_t bal = __builtin_amdgcn_ballot_w64(f);
+    if (__lane_id() == 0) wsum[threadIdx.x / 64] = (uint32_t)__popcll(bal);
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+    for (uint32_t w = 0; w < 16; ++w) {
+      before += w < threadIdx.x / 64 ? wsum[w] : 0;
+      all += wsum[w];
+    }
+    const uint64_t pos = base + before + below_count(bal);
+    if (f && pos < cap) {
+      for (int k = 0; k < a.g.nk; ++k)
+        o.keys[k][pos] = (int64_t)((uint64_t)a.g.kmin[k] + ((c >> a.g.shift[k]) & a.g.fmask[k]));
+      for (int v = 0; v < nv; ++v) o.vals[v][pos] = a.g.tab[v][c];
+    }
+    base += all;
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    r.dst[0] = base;
+    r.dst[1] = *bad;
+    result_done(r);
+  }
+}
+
+// Smallest and largest key values among 16 spread runs of 1024 rows (n >= 16384), one block.
+__global__ void __launch_bounds__(1024) k_gl_sample(GbArgs a, uint64_t n, DevResult r) {
+  __shared__ int64_t lo[16], hi[16];
+  const uint64_t step = (n - 1024) / 15;
+  for (int k = 0; k < a.nk; ++k) {
+    int64_t x[16], mn = INT64_MAX, mx = INT64_MIN;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) x[j] = a.keys[k][step * j + threadIdx.x];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+      mn = x[j] < mn ? x[j] : mn;
+      mx = x[j] > mx ? x[j] : mx;
+    }
+    for (int d = 32; d > 0; d >>= 1) {
+      const int64_t p = __shfl_xor(mn, d, 64), q = __shfl_xor(mx, d, 64);
+      mn = p < mn ? p : mn;
+      mx = q > mx ? q : mx;
+    }
+    if (__lane_id() == 0) {
+      lo[threadIdx.x / 64] = mn;
+      hi[threadIdx.x / 64] = mx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (int w = 1; w < 16; ++w) {
+        mn = lo[w] < mn ? lo[w] : mn;
+        mx = hi[w] > mx ? hi[w] : mx;
+      }
+      r.dst[2 * k] = (uint64_t)mn;
+      r.dst[2 * k + 1] = (uint64_t)mx;
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) result_done(r);
+}
+
 // No key that varies: one group, a reduction.  Block partials part[block][v], each block's
 // rows grid-strided, combined in a fixed order so the result does not depend on timing.
 __global__ void __launch_bounds__(256) k_gb_reduce(GbArgs a, uint64_t n, int64_t *__restrict__ part) {
@@ -482,6 +679,113 @@ static int groupby_sorted(aln_ctx *c, GbArgs &a, uint64_t n, int order, uint32_t
   return ALN_OK;
 }
 
+// The code layout of keys in [mn, mx]: widths, masks and shifts (key 0 most significant).
+// Returns the total bits (shifts are set when they fit 63).
+static uint32_t gb_layout(GbArgs &a, const int64_t *mn, const int64_t *mx) {
+  uint32_t bits[ALN_MAX_KEYS], total = 0;
+  for (int k = 0; k < a.nk; ++k) {
+    bits[k] = bits_for_range_u((uint64_t)mx[k] - (uint64_t)mn[k]);
+    a.kmin[k] = mn[k];
+    a.fmask[k] = bits[k] == 64 ? ~0ull : ((1ull << bits[k]) - 1);
+    total += bits[k];
+  }
+  uint32_t sh = total;
+  for (int k = 0; k < a.nk; ++k) {
+    sh -= bits[k];
+    a.shift[k] = total > 63 ? 0 : sh;
+  }
+  return total;
+}
+
+// The few-groups path for codes of `total` bits, if all accumulators fit in LDS: *taken, and
+// *outside when a key lay outside the layout (nothing is valid then).  With order KEYS or NONE
+// the groups are written out and *done is set; else the tables stand in a.tab (a.tab[*cnt] the
+// row counts).
+static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, const GbOut &o, uint64_t cap,
+                  uint64_t *h_ngroups, int *cnt, bool *taken, bool *done, bool *outside) {
+  *taken = *done = *outside = false;
+  GlArgs l;
+  l.g = a;
+  l.cnt = -1;
+  for (int v = 0; v < a.nv && l.cnt < 0; ++v)
+    if (a.aggs[v] == ALN_AGG_COUNT) l.cnt = v;
+  if (l.cnt < 0) {
+    l.cnt = l.g.nv++;
+    l.g.aggs[l.cnt] = ALN_AGG_COUNT;
+    l.g.vals[l.cnt] = nullptr;
+  }
+  if (total > 16) return ALN_OK;
+  l.ncodes = 1u << total;
+  const uint32_t nacc = l.ncodes * (uint32_t)l.g.nv;
+  if ((size_t)nacc * 8 > GL_MOST) return ALN_OK;
+  l.lr = 0;
+  while (l.lr < 6 && ((size_t)nacc * 16 << l.lr) <= GL_COPIES) ++l.lr;
+  const size_t lds = (size_t)nacc * 8 << l.lr;
+  *taken = true;
+  // as many blocks as the LDS holds on 256 CUs (5 or 2 per CU), fewer for few rows
+  uint32_t nb = lds <= GL_COPIES ? 1280 : 512;
+  nb = grid_for(n, 256 * GL_U, nb);
+  if ((uint64_t)nb * nacc > GL_PART) nb = (uint32_t)(GL_PART / nacc);
+  int64_t *part, *tab;
+  uint32_t *bad;
+  ALN_TRY(ws(c, (size_t)nb * nacc, &part));
+  ALN_TRY(ws(c, nacc, &tab));
+  ALN_TRY(ws(c, 1, &bad));
+  for (int v = 0; v < l.g.nv; ++v) l.g.tab[v] = tab + (size_t)v * l.ncodes;
+  ALN_TRY(fill_u32(c, bad, 1, 0));
+  {
+    ProfScope p(c, "groupby_insert");
+    hipLaunchKernelGGL(k_gl_agg, dim3(nb), dim3(256), lds, c->stream, l, n, part, bad);
+    hipLaunchKernelGGL(k_gl_sum, dim3((nacc + 3) / 4), dim3(256), 0, c->stream, l, (const int64_t *)part, nb);
+  }
+  ALN_TRY(check_launch("gb_lds"));
+  if (order != ALN_ORDER_HASH) {
+    DevResult r;
+    uint64_t h[2];
+    ALN_TRY(result_open(c, 2, &r));
+    hipLaunchKernelGGL(k_gl_emit, dim3(1), dim3(1024), 0, c->stream, l, o, a.nv, cap, (const uint32_t *)bad, r);
+    ALN_TRY(check_launch("gb_lds_emit"));
+    ALN_TRY(result_wait(c, r, h, 16));
+    *outside = h[1] != 0;
+    if (*outside) return ALN_OK;
+    *h_ngroups = h[0];
+    if (h[0] > cap)
+      return set_error(ALN_E_CAPACITY, "aln_groupby: %llu groups, capacity %llu", (unsigned long long)h[0],
+                       (unsigned long long)cap);
+    *done = true;
+    return ALN_OK;
+  }
+  uint32_t hb = 0;
+  ALN_TRY(copy_to_host(c, &hb, bad, 4));
+  *outside = hb != 0;
+  for (int v = 0; v < l.g.nv; ++v) a.tab[v] = l.g.tab[v];
+  *cnt = l.cnt;
+  return ALN_OK;
+}
+
+// The occupied codes of direct-indexed tables, in order (row counts in gcnt, or, gcnt NULL, in
+// a.tab[cv]).
+static int gb_dense_groups(aln_ctx *c, const GbArgs &a, int cv, const uint32_t *gcnt, uint64_t ncodes, uint64_t cap,
+                           uint64_t *h_ngroups, uint64_t **gcode, uint32_t **gslot) {
+  uint32_t *flag;
+  uint64_t *pos, g = 0;
+  ALN_TRY(ws(c, ncodes, &flag));
+  ALN_TRY(ws(c, ncodes, &pos));
+  hipLaunchKernelGGL(k_gb_dense_flags, dim3(grid_for(ncodes, 256, 65536)), dim3(256), 0, c->stream, a, cv, gcnt,
+                     ncodes, flag);
+  ALN_TRY(check_launch("gb_flags"));
+  ALN_TRY(exclusive_scan_u32(c, flag, ncodes, pos, &g));
+  *h_ngroups = g;
+  if (g > cap)
+    return set_error(ALN_E_CAPACITY, "aln_groupby: %llu groups, capacity %llu", (unsigned long long)g,
+                     (unsigned long long)cap);
+  ALN_TRY(ws(c, g, gcode));
+  ALN_TRY(ws(c, g, gslot));
+  hipLaunchKernelGGL(k_gb_dense_compact, dim3(grid_for(ncodes, 256, 65536)), dim3(256), 0, c->stream, flag,
+                     ncodes, pos, *gcode, *gslot);
+  return check_launch("gb_compact");
+}
+
 }  // namespace aln
 
 using namespace aln;
@@ -505,16 +809,9 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   memset(&a, 0, sizeof(a));
   a.nk = nkeys;
   a.nv = nvals;
-  uint32_t bits[ALN_MAX_KEYS], total = 0;
   for (int k = 0; k < nkeys; ++k) {
     ALN_REQUIRE(d_keys[k], "aln_groupby: key %d is NULL", k);
-    int64_t mn, mx;
-    ALN_TRY(minmax_i64(c, d_keys[k], n, &mn, &mx));
-    bits[k] = bits_for_range_u((uint64_t)mx - (uint64_t)mn);
     a.keys[k] = d_keys[k];
-    a.kmin[k] = mn;
-    a.fmask[k] = bits[k] == 64 ? ~0ull : ((1ull << bits[k]) - 1);
-    total += bits[k];
   }
   for (int v = 0; v < nvals; ++v) {
     ALN_REQUIRE(aggs[v] == ALN_AGG_COUNT || aggs[v] == ALN_AGG_SUM || aggs[v] == ALN_AGG_MIN ||
@@ -530,6 +827,36 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   for (int k = 0; k < nkeys; ++k) o.keys[k] = d_out_keys[k];
   for (int v = 0; v < nvals; ++v) o.vals[v] = d_out_vals[v];
 
+  // A sample's key ranges stand in for the keys' own when they are those of a few groups: the
+  // rows are then checked against them as they are added up (and start again when one lies
+  // outside), which saves reading the keys twice (60M rows of two keys: 0.18 of 0.76 ms).
+  int64_t mn[ALN_MAX_KEYS], mx[ALN_MAX_KEYS];
+  uint32_t total = 0;
+  bool lds_taken = false, lds_done = false, outside = false;
+  int cnt = -1;
+  if (nkeys && n >= GL_SAMPLE_MIN) {
+    DevResult r;
+    int64_t h[2 * ALN_MAX_KEYS];
+    ALN_TRY(result_open(c, 2 * ALN_MAX_KEYS, &r));
+    hipLaunchKernelGGL(k_gl_sample, dim3(1), dim3(1024), 0, c->stream, a, n, r);
+    ALN_TRY(check_launch("gb_sample"));
+    ALN_TRY(result_wait(c, r, h, 16 * (size_t)nkeys));
+    for (int k = 0; k < nkeys; ++k) {
+      mn[k] = h[2 * k];
+      mx[k] = h[2 * k + 1];
+    }
+    total = gb_layout(a, mn, mx);
+    if (total > 0 && total <= GL_SAMPLE_BITS)
+      ALN_TRY(gb_few(c, a, n, total, order, o, cap, h_ngroups, &cnt, &lds_taken, &lds_done, &outside));
+    if (outside) lds_taken = lds_done = false;
+  }
+  if (!lds_taken) {
+    if (nkeys) ALN_TRY(minmax_keys(c, a.keys, nkeys, n, mn, mx));
+    total = gb_layout(a, mn, mx);
+    if (total > 0)
+      ALN_TRY(gb_few(c, a, n, total, order, o, cap, h_ngroups, &cnt, &lds_taken, &lds_done, &outside));
+  }
+  if (lds_done) return ALN_OK;
   if (total == 0) {
     // no GROUP BY, or keys that never vary: one group, a reduction (reduce, select.cu:549)
     *h_ngroups = 1;
@@ -547,15 +874,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     ALN_HIP(hipStreamSynchronize(c->stream));
     return ALN_OK;
   }
-  if (total > 63) {
-    for (int k = 0; k < nkeys; ++k) a.shift[k] = 0;
-    return groupby_sorted(c, a, n, order, seed, o, cap, h_ngroups);
-  }
-  uint32_t sh = total;
-  for (int k = 0; k < nkeys; ++k) {
-    sh -= bits[k];
-    a.shift[k] = sh;
-  }
+  if (total > 63) return groupby_sorted(c, a, n, order, seed, o, cap, h_ngroups);
   // LDS-cached aggregation kernel: blocks of at least 32 rows per thread, its LDS size
   const size_t lds = gb_lds_bytes(nvals);
   const uint32_t nb = grid_for(n, 256 * 32, 2048);
@@ -571,10 +890,12 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   uint32_t *gslot;
   const uint64_t ncodes = 1ull << total;
   const bool dense = total <= GB_DENSE_BITS && ncodes <= std::max<uint64_t>(2 * n, (uint64_t)GB_LT);
-  if (dense) {
+  if (lds_taken) {
+    ALN_TRY(gb_dense_groups(c, a, cnt, nullptr, ncodes, cap, h_ngroups, &gcode, &gslot));
+    g = *h_ngroups;
+  } else if (dense) {
     // direct-indexed accumulators: slot = code, groups come out in key order
-    uint32_t *gcnt = nullptr, *flag;
-    uint64_t *pos;
+    uint32_t *gcnt = nullptr;
     int cv = -1;  // a COUNT aggregate, whose table tells the occupied codes
     for (int v = 0; v < nvals && cv < 0; ++v)
       if (aggs[v] == ALN_AGG_COUNT) cv = v;
@@ -589,21 +910,8 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
                          gcnt, ctl + 1, 0xFFFFFFFFu, ctl);
     }
     ALN_TRY(check_launch("gb_agg"));
-    ALN_TRY(ws(c, ncodes, &flag));
-    ALN_TRY(ws(c, ncodes, &pos));
-    hipLaunchKernelGGL(k_gb_dense_flags, dim3(grid_for(ncodes, 256, 65536)), dim3(256), 0, c->stream, a, cv, gcnt,
-                       ncodes, flag);
-    ALN_TRY(check_launch("gb_flags"));
-    ALN_TRY(exclusive_scan_u32(c, flag, ncodes, pos, &g));
-    *h_ngroups = g;
-    if (g > cap)
-      return set_error(ALN_E_CAPACITY, "aln_groupby: %llu groups, capacity %llu", (unsigned long long)g,
-                       (unsigned long long)cap);
-    ALN_TRY(ws(c, g, &gcode));
-    ALN_TRY(ws(c, g, &gslot));
-    hipLaunchKernelGGL(k_gb_dense_compact, dim3(grid_for(ncodes, 256, 65536)), dim3(256), 0, c->stream, flag,
-                       ncodes, pos, gcode, gslot);
-    ALN_TRY(check_launch("gb_compact"));
+    ALN_TRY(gb_dense_groups(c, a, cv, gcnt, ncodes, cap, h_ngroups, &gcode, &gslot));
+    g = *h_ngroups;
   } else {
     // open addressing: first a table for up to GB_HASH_START keys (half full at most); more
     // keys than that set the overflow flag and the rows are aggregated again in a table of

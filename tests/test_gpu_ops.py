@@ -386,6 +386,59 @@ def test_groupby_paths(ctx, case):
     _gb_check(ctx, keys, [v, v], [L.AGG_SUM, L.AGG_COUNT], order=L.ORDER_HASH, bounds=bounds)
 
 
+@pytest.mark.parametrize("n", [1, 2047, 2049, 20000, (1 << 20) + 5])
+@pytest.mark.parametrize("widths", [(2,), (3, 2), (1000,), (40, 90), (2, 5, 3, 3)])
+def test_groupby_few_groups(ctx, n, widths):
+    """Accumulators in LDS: one to four keys, every aggregate (with and without a COUNT among
+    them, eight at once), both orders, at the edges of the 2048-row blocks, and (from 2^20 rows,
+    where the key ranges come from a sample first) with a key the sample misses; f64 columns with
+    NaN, infinities and -0.0."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n + len(widths))
+    keys = [r.integers(0, w, n).astype(np.int64) - w // 2 for w in widths]
+    if n > 1 << 20:
+        keys[0][12345] = 5000  # in none of the sampled runs
+    vals = [r.integers(-(1 << 62), 1 << 62, n).astype(np.int64) for _ in range(4)]
+    aggs = [L.AGG_SUM, L.AGG_MIN, L.AGG_MAX, L.AGG_SUM]
+    wk, wv = O.groupby(keys, vals, aggs, seed=100)
+    hk, hv = O.groupby(keys, vals, aggs, seg_bounds=[0, n // 2, n] if n > 1 else [0, n], seed=100)
+    f = r.integers(-1000, 1000, n) / 8.0  # sums of these are exact in any order
+    code = np.zeros(n, np.int64)
+    for k in keys:
+        code = code * 12000 + (k + 6000)
+    ucode, inv = np.unique(code, return_inverse=True)
+    bits = lambda x: np.ascontiguousarray(x).view(np.int64)  # noqa: E731
+    special = f.copy()
+    special[:: 5], special[1:: 7], special[2:: 11] = np.nan, np.inf, -0.0
+    fmin, fmax = np.full(ucode.size, np.inf), np.full(ucode.size, -np.inf)
+    ok = ~np.isnan(special)
+    np.minimum.at(fmin, inv[ok], special[ok])
+    np.maximum.at(fmax, inv[ok], special[ok])
+    fsum = np.bincount(inv, weights=f, minlength=ucode.size)
+    cnt = np.bincount(inv, minlength=ucode.size)
+    dk, dv = [dev(ctx, k) for k in keys], [dev(ctx, v) for v in vals]
+    df, ds = dev(ctx, bits(f)), dev(ctx, bits(special))
+    for order, (ek, ev) in ((L.ORDER_KEYS, (wk, wv)), (L.ORDER_HASH, (hk, hv))):
+        ok_, ov = D.groupby(ctx, dk, dv, aggs, order=order, seed=100)
+        for x, y in zip(ok_ + ov, list(ek) + list(ev)):
+            assert np.array_equal(host(x), y)
+    ok_, ov = D.groupby(ctx, dk, [df, ds, ds, None, dv[0], dv[1], dv[2], df],
+                        [L.AGG_FSUM, L.AGG_FMIN, L.AGG_FMAX, L.AGG_COUNT, L.AGG_SUM, L.AGG_MIN, L.AGG_MAX, L.AGG_FSUM])
+    for x, y in zip(ok_, wk):
+        assert np.array_equal(host(x), y)
+    f64 = lambda t: host(t).view(np.float64)  # noqa: E731
+    assert np.array_equal(f64(ov[0]), fsum) and np.array_equal(f64(ov[7]), fsum)
+    assert np.array_equal(f64(ov[1]), fmin) and np.array_equal(f64(ov[2]), fmax)
+    assert np.array_equal(host(ov[3]), cnt)
+    for x, y in zip(ov[4:7], wv[:3]):
+        assert np.array_equal(host(x), y)
+    if len(wk[0]) > 1:
+        with pytest.raises(L.AlnError) as e:
+            D.groupby(ctx, dk, dv, aggs, cap=len(wk[0]) - 1)
+        assert e.value.code == L.ALN_E_CAPACITY
+
+
 # ---- join --------------------------------------------------------------------------------
 @pytest.mark.parametrize("case", ["dense", "dups", "sparse", "wide", "dense_big"])
 def test_hash_join(ctx, case):
