@@ -365,15 +365,16 @@ __global__ void __launch_bounds__(64 * SCAN_ONE_WAVES) k_scan_one(const T *__res
   uint64_t carry = 0;
 #pragma unroll
   for (int j = 0; j < SCAN_ITEMS; ++j) {
-    if ((uint32_t)j >= rows) break;
-    uint64_t x = v[j];
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint64_t y = __shfl_up(x, o, 64);
-      if (lane >= (unsigned)o) x += y;
+    if ((uint32_t)j < rows) {
+      uint64_t x = v[j];
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint64_t y = __shfl_up(x, o, 64);
+        if (lane >= (unsigned)o) x += y;
+      }
+      const uint64_t row = __shfl(x, 63, 64);
+      v[j] = carry + x - v[j];
+      carry += row;
     }
-    const uint64_t row = __shfl(x, 63, 64);
-    v[j] = carry + x - v[j];
-    carry += row;
   }
   if (lane == 0) wsum[wid] = carry;
   __syncthreads();

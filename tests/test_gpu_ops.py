@@ -439,6 +439,39 @@ def test_groupby_few_groups(ctx, n, widths):
         assert e.value.code == L.ALN_E_CAPACITY
 
 
+@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 4097])
+@pytest.mark.parametrize("case", ["2keys", "wide", "skewed", "hot", "edge"])
+def test_groupby_parts(ctx, n, case):
+    """Rows moved into parts of the code range (from 2^20 rows on): a few thousand codes of two
+    keys, 2^21 codes, a skewed column (parts of several blocks), one key almost everywhere, and
+    the smallest code range; all aggregates over one and several value columns, with and without
+    a COUNT, in both orders."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n + len(case))
+    keys = {"2keys": lambda: [r.integers(-20, 100, n), r.integers(0, 100, n)],
+            "wide": lambda: [r.integers(0, 1 << 21, n)],
+            "skewed": lambda: [np.minimum(r.zipf(1.15, n), 1 << 17) + 7],
+            "hot": lambda: [np.where(r.random(n) < 0.98, 4000, r.integers(0, 1 << 18, n))],
+            "edge": lambda: [r.integers(0, 8193, n)]}[case]()
+    keys = [k.astype(np.int64) for k in keys]
+    v, w = r.integers(-(1 << 40), 1 << 40, n).astype(np.int64), r.integers(-1000, 1000, n).astype(np.int64)
+    _gb_check(ctx, keys, [v, v, w, v], AGGS4)
+    _gb_check(ctx, keys, [v], [L.AGG_SUM])
+    _gb_check(ctx, keys, [v, w], [L.AGG_MIN, L.AGG_COUNT], order=L.ORDER_HASH, bounds=[0, n // 2, n])
+    f = r.integers(-1000, 1000, n) / 8.0
+    code = keys[0] * 1000 + keys[1] if len(keys) == 2 else keys[0]
+    ucode, inv = np.unique(code, return_inverse=True)
+    fmin, fmax = np.full(ucode.size, np.inf), np.full(ucode.size, -np.inf)
+    np.minimum.at(fmin, inv, f)
+    np.maximum.at(fmax, inv, f)
+    df = dev(ctx, f.view(np.int64))
+    ok, ov = D.groupby(ctx, [dev(ctx, k) for k in keys], [df, df, df], [L.AGG_FSUM, L.AGG_FMIN, L.AGG_FMAX])
+    assert ok[0].numel() == ucode.size
+    for got, want in zip(ov, (np.bincount(inv, weights=f), fmin, fmax)):
+        assert np.array_equal(host(got).view(np.float64), want)
+
+
 # ---- join --------------------------------------------------------------------------------
 @pytest.mark.parametrize("case", ["dense", "dups", "sparse", "wide", "dense_big"])
 def test_hash_join(ctx, case):
