@@ -22,19 +22,16 @@
 //   * the groups are compacted and put in the reference's output order: ascending key
 //     tuple (one segment) or ascending MurmurHash64A(keys, 8*nkeys, seed) (the
 //     multi-segment merge order).
-// Key tuples wider than 63 bits fall back to the reference's own scheme: stable sort,
-// run heads, per-run reduction.
+// Key tuples wider than 63 bits, and wide codes of which a sample shows many groups, go the
+// reference's way: sort, run heads, per-run reduction (groupsort.hip).
 #include <string.h>
 
 #include <algorithm>
 #include <vector>
 
-#include "aln_internal.h"
+#include "groupby.h"
 
 namespace aln {
-
-int sort_keys_impl(aln_ctx *c, const int64_t *const *keys, const int32_t *desc, int nkeys,
-                   uint64_t n, uint32_t *d_perm);
 
 constexpr uint64_t GB_EMPTY = ~0ull;
 // Packed key codes of at most this many bits (and at most 2n codes) use direct-indexed
@@ -44,77 +41,9 @@ constexpr uint32_t GB_DENSE_BITS = 26;
 // aggregated again in a table of 2n slots.
 constexpr uint64_t GB_HASH_START = 1ull << 20;
 constexpr uint64_t GB_FIRST_PROBES = 64;
-
-struct GbArgs {
-  const int64_t *keys[ALN_MAX_KEYS];
-  int64_t kmin[ALN_MAX_KEYS];
-  uint32_t shift[ALN_MAX_KEYS];
-  uint64_t fmask[ALN_MAX_KEYS];
-  // one more than a call can ask for: the few-groups path counts rows by itself
-  const int64_t *vals[ALN_MAX_AGGS + 1];
-  int32_t aggs[ALN_MAX_AGGS + 1];
-  int64_t *tab[ALN_MAX_AGGS + 1];
-  int nk, nv;
-};
-
-__device__ __forceinline__ int64_t agg_combine(int a, int64_t x, int64_t y) {
-  if (a == ALN_AGG_MIN) return x < y ? x : y;
-  if (a == ALN_AGG_MAX) return x > y ? x : y;
-  if (a == ALN_AGG_FSUM) return f64_bits(bits_f64(x) + bits_f64(y));
-  if (a == ALN_AGG_FMIN) return bits_f64(y) < bits_f64(x) ? y : x;
-  if (a == ALN_AGG_FMAX) return bits_f64(y) > bits_f64(x) ? y : x;
-  return (int64_t)((uint64_t)x + (uint64_t)y);  // SUM, COUNT
-}
-
-// The starting value of an aggregate's accumulator.
-__host__ __device__ __forceinline__ int64_t agg_identity(int a) {
-  switch (a) {
-    case ALN_AGG_MIN: return INT64_MAX;
-    case ALN_AGG_MAX: return INT64_MIN;
-    case ALN_AGG_FMIN: return 0x7FF0000000000000ll;                // +inf
-    case ALN_AGG_FMAX: return (int64_t)0xFFF0000000000000ull;      // -inf
-    default: return 0;                                             // 0, 0.0
-  }
-}
-
-// Adds x into the accumulator at t.
-__device__ __forceinline__ void agg_atomic(int a, int64_t *t, int64_t x) {
-  if (a == ALN_AGG_MIN) {
-    atomicMin((long long *)t, (long long)x);
-  } else if (a == ALN_AGG_MAX) {
-    atomicMax((long long *)t, (long long)x);
-  } else if (a == ALN_AGG_FSUM) {
-    atomicAdd(reinterpret_cast<double *>(t), bits_f64(x));
-  } else if (a == ALN_AGG_FMIN || a == ALN_AGG_FMAX) {
-    unsigned long long *p = reinterpret_cast<unsigned long long *>(t);
-    unsigned long long old = *p, assumed;
-    do {
-      assumed = old;
-      const int64_t nv = agg_combine(a, (int64_t)assumed, x);
-      if (nv == (int64_t)assumed) break;
-      old = atomicCAS(p, assumed, (unsigned long long)nv);
-    } while (old != assumed);
-  } else {
-    atomicAdd((unsigned long long *)t, (unsigned long long)x);
-  }
-}
-
-__device__ __forceinline__ uint64_t murmur64a_tuple(const int64_t *v, int nk, uint32_t seed) {
-  const uint64_t m = 0xc6a4a7935bd1e995ULL;
-  uint64_t h = (uint64_t)seed ^ ((uint64_t)(8 * nk) * m);
-  for (int i = 0; i < nk; ++i) {
-    uint64_t k = (uint64_t)v[i];
-    k *= m;
-    k ^= k >> 47;
-    k *= m;
-    h ^= k;
-    h *= m;
-  }
-  h ^= h >> 47;
-  h *= m;
-  h ^= h >> 47;
-  return h;
-}
+// Rows from which wide codes of many groups are sorted instead (fewer sort in eight passes of
+// their own launches, which the hash table's atomics still beat).
+constexpr uint64_t GB_SORT_MIN = 1ull << 20;
 
 __global__ void __launch_bounds__(256) k_gb_init(uint64_t *tkey, GbArgs a, uint64_t cap) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < cap;
@@ -123,11 +52,6 @@ __global__ void __launch_bounds__(256) k_gb_init(uint64_t *tkey, GbArgs a, uint6
     for (int v = 0; v < a.nv; ++v) a.tab[v][i] = agg_identity(a.aggs[v]);
   }
 }
-
-struct GbOut {
-  int64_t *keys[ALN_MAX_KEYS];
-  int64_t *vals[ALN_MAX_AGGS];
-};
 
 // Adjacent lanes with equal codes (clustered input): the last lane of each run gets the
 // run's combined values and row count and returns true.
@@ -473,6 +397,37 @@ __global__ void __launch_bounds__(1024) k_gl_sample(GbArgs a, uint64_t n, DevRes
     __syncthreads();
   }
   if (threadIdx.x == 0) result_done(r);
+}
+
+// Distinct key codes among GB_SAMPLE rows spread over the table (n >= GB_SAMPLE), by 32-bit
+// fingerprints in an LDS set, one block.
+constexpr uint32_t GB_SAMPLE = 8192;
+__global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevResult r) {
+  __shared__ uint32_t set[2 * GB_SAMPLE];
+  __shared__ uint32_t found;
+  for (uint32_t i = threadIdx.x; i < 2 * GB_SAMPLE; i += 1024) set[i] = 0;
+  if (threadIdx.x == 0) found = 0;
+  __syncthreads();
+  const uint64_t step = (n - 1024) / 7;
+  uint32_t mine = 0;
+#pragma unroll 1
+  for (uint32_t j = 0; j < GB_SAMPLE / 1024; ++j) {
+    const uint64_t h = murmur64a_u64(gb_code(a, step * j + threadIdx.x), 0x9747b28cu);
+    const uint32_t f = (uint32_t)(h >> 32) | 1u;
+    uint32_t at = (uint32_t)h & (2 * GB_SAMPLE - 1);
+    while (true) {  // at most half full
+      const uint32_t old = atomicCAS(&set[at], 0u, f);
+      mine += old == 0;
+      if (old == 0 || old == f) break;
+      at = (at + 1) & (2 * GB_SAMPLE - 1);
+    }
+  }
+  atomicAdd(&found, mine);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    r.dst[0] = found;
+    result_done(r);
+  }
 }
 
 // ---- many codes: partitions of the code range ------------------------------------------------
@@ -910,45 +865,6 @@ __global__ void k_gb_emit(GbArgs a, GbOut o, const uint64_t *gcode, const uint32
   }
 }
 
-// ---- sort-based fallback ------------------------------------------------------------------
-__global__ void k_gb_heads(GbArgs a, const uint32_t *perm, uint64_t n, uint32_t *head) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256) {
-    bool h = i == 0;
-    if (!h)
-      for (int k = 0; k < a.nk; ++k)
-        if (a.keys[k][perm[i]] != a.keys[k][perm[i - 1]]) h = true;
-    head[i] = h;
-  }
-}
-
-__global__ void k_gb_sorted_agg(GbArgs a, GbOut o, const uint32_t *perm, const uint32_t *head,
-                                const uint64_t *gid_ex, uint64_t n) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256) {
-    uint64_t g = gid_ex[i] + head[i] - 1;  // group index of sorted row i
-    uint32_t r = perm[i];
-    if (head[i])
-      for (int k = 0; k < a.nk; ++k) o.keys[k][g] = a.keys[k][r];
-    for (int v = 0; v < a.nv; ++v) {
-      const int ag = a.aggs[v];
-      agg_atomic(ag, &o.vals[v][g], ag == ALN_AGG_COUNT ? 1 : a.vals[v][r]);
-    }
-  }
-}
-
-// Reorders the sort-path groups into hash order (in place through temporaries).
-__global__ void k_gb_hash_keys(GbOut o, int nk, uint64_t g, uint32_t seed, uint64_t *hash,
-                               uint32_t *idx) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < g;
-       i += (uint64_t)gridDim.x * 256) {
-    int64_t kv[ALN_MAX_KEYS];
-    for (int k = 0; k < nk; ++k) kv[k] = o.keys[k][i];
-    hash[i] = murmur64a_tuple(kv, nk, seed);
-    idx[i] = (uint32_t)i;
-  }
-}
-
 __global__ void k_gb_gather(const uint64_t *gc, const uint32_t *gs, const uint32_t *gi, uint64_t g,
                             uint64_t *oc, uint32_t *os) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < g;
@@ -956,12 +872,6 @@ __global__ void k_gb_gather(const uint64_t *gc, const uint32_t *gs, const uint32
     oc[i] = gc[gi[i]];
     os[i] = gs[gi[i]];
   }
-}
-
-__global__ void k_permute_i64(const int64_t *in, const uint32_t *perm, uint64_t n, int64_t *out) {
-  for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
-       i += (uint64_t)gridDim.x * 256)
-    out[i] = in[perm[i]];
 }
 
 __global__ void k_hash_rows(GbArgs a, uint64_t n, uint32_t seed, uint64_t *out) {
@@ -976,57 +886,6 @@ __global__ void k_hash_rows(GbArgs a, uint64_t n, uint32_t seed, uint64_t *out) 
 __global__ void k_f64_keys(const int64_t *in, uint64_t n, int back, int64_t *out) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (uint64_t)gridDim.x * 256)
     out[i] = back ? f64_unorder_key(in[i]) : f64_order_key(in[i]);
-}
-
-static int groupby_sorted(aln_ctx *c, GbArgs &a, uint64_t n, int order, uint32_t seed, GbOut &o,
-                          uint64_t cap, uint64_t *h_ngroups) {
-  uint32_t *perm, *head;
-  uint64_t *gid;
-  ALN_TRY(ws(c, n, &perm));
-  ALN_TRY(ws(c, n, &head));
-  ALN_TRY(ws(c, n, &gid));
-  const int64_t *keys[ALN_MAX_KEYS];
-  for (int k = 0; k < a.nk; ++k) keys[k] = a.keys[k];
-  ALN_TRY(sort_keys_impl(c, keys, nullptr, a.nk, n, perm));
-  hipLaunchKernelGGL(k_gb_heads, dim3(grid_for(n, 256, 65536)), dim3(256), 0, c->stream, a, perm, n,
-                     head);
-  ALN_TRY(check_launch("gb_heads"));
-  uint64_t g = 0;
-  ALN_TRY(exclusive_scan_u32(c, head, n, gid, &g));
-  *h_ngroups = g;
-  if (g > cap)
-    return set_error(ALN_E_CAPACITY, "aln_groupby: %llu groups, capacity %llu",
-                     (unsigned long long)g, (unsigned long long)cap);
-  for (int v = 0; v < a.nv; ++v) ALN_TRY(fill_i64(c, o.vals[v], g, agg_identity(a.aggs[v])));
-  {
-    ProfScope p(c, "groupby_sorted_agg");
-    hipLaunchKernelGGL(k_gb_sorted_agg, dim3(grid_for(n, 256, 65536)), dim3(256), 0, c->stream, a,
-                       o, perm, head, gid, n);
-  }
-  ALN_TRY(check_launch("gb_sorted_agg"));
-  if (order == ALN_ORDER_HASH && g > 1) {
-    uint64_t *hash;
-    uint32_t *idx;
-    int64_t *tmp;
-    ALN_TRY(ws(c, g, &hash));
-    ALN_TRY(ws(c, g, &idx));
-    ALN_TRY(ws(c, g, &tmp));
-    hipLaunchKernelGGL(k_gb_hash_keys, dim3(grid_for(g, 256, 65536)), dim3(256), 0, c->stream, o,
-                       a.nk, g, seed, hash, idx);
-    ALN_TRY(check_launch("gb_hash_keys"));
-    ALN_TRY(radix_sort_pairs(c, hash, idx, g, 64));
-    auto permute = [&](int64_t *col) -> int {
-      hipLaunchKernelGGL(k_permute_i64, dim3(grid_for(g, 256, 65536)), dim3(256), 0, c->stream, col,
-                         idx, g, tmp);
-      ALN_TRY(check_launch("permute"));
-      ALN_HIP(hipMemcpyAsync(col, tmp, 8 * g, hipMemcpyDeviceToDevice, c->stream));
-      return ALN_OK;
-    };
-    for (int k = 0; k < a.nk; ++k) ALN_TRY(permute(o.keys[k]));
-    for (int v = 0; v < a.nv; ++v) ALN_TRY(permute(o.vals[v]));
-  }
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
 }
 
 // The code layout of keys in [mn, mx]: widths, masks and shifts (key 0 most significant).
@@ -1307,7 +1166,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     ALN_HIP(hipStreamSynchronize(c->stream));
     return ALN_OK;
   }
-  if (total > 63) return groupby_sorted(c, a, n, order, seed, o, cap, h_ngroups);
+  if (total > 63) return gb_sorted(c, a, n, total, order, seed, o, cap, h_ngroups);
   // LDS-cached aggregation kernel: blocks of at least 32 rows per thread, its LDS size
   const size_t lds = gb_lds_bytes(nvals);
   const uint32_t nb = grid_for(n, 256 * 32, 2048);
@@ -1348,6 +1207,17 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
       return ALN_OK;
     }
   } else {
+    // many groups: global atomics (24 G/s) cost more than sorting the rows (12M rows of 12M
+    // groups: 1.1 against 12 ms, by a 6M-row call of 8.6 ms).  Half of a sample distinct means some 5000 groups or more.
+    if (n >= GB_SORT_MIN) {
+      DevResult r;
+      uint64_t found = 0;
+      ALN_TRY(result_open(c, 1, &r));
+      hipLaunchKernelGGL(k_gb_distinct, dim3(1), dim3(1024), 0, c->stream, a, n, r);
+      ALN_TRY(check_launch("gb_distinct"));
+      ALN_TRY(result_wait(c, r, &found, 8));
+      if (2 * found >= GB_SAMPLE) return gb_sorted(c, a, n, total, order, seed, o, cap, h_ngroups);
+    }
     // open addressing: first a table for up to GB_HASH_START keys (half full at most); more
     // keys than that set the overflow flag and the rows are aggregated again in a table of
     // 2n slots

@@ -97,6 +97,7 @@ static inline int key_word(uint32_t bits) { return bits <= 32 ? 4 : 8; }
 
 // The items of one pass.  KI (bytes per stored key) 4, 8: keys and values from arrays;
 // KI 0: codes computed from the key columns at row r = vals ? vals[i] : i, with value r.
+// No values: the item's number.
 struct RsIn {
   const void *keys;
   const uint32_t *vals;
@@ -114,7 +115,7 @@ __device__ __forceinline__ uint64_t rs_key(const RsIn &in, uint64_t i) {
 }
 template <int KI>
 __device__ __forceinline__ uint32_t rs_val(const RsIn &in, uint64_t i) {
-  if (KI == 0 && !in.vals) return (uint32_t)i;
+  if (!in.vals) return (uint32_t)i;
   return __builtin_nontemporal_load(in.vals + i);
 }
 
@@ -391,6 +392,7 @@ struct RsLocal {
   const uint64_t *keys;
   const uint32_t *vals;
   uint32_t *vout;
+  uint8_t *heads;  // may be NULL: 1 where a position's code differs from the one before
   uint32_t *overflow;
   uint64_t n;
   uint32_t nblk, topshift, nlow;  // nlow >= 2 remaining varying digits:
@@ -581,7 +583,10 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
     for (int j = 0; j < RS_ITEMS; ++j) {
       if (j >= (int)J) break;
       const uint32_t i = wid * S + j * 64 + lane;
-      if (i < m) a.vout[w0 + lo + i] = val[j];
+      if (i < m) {
+        a.vout[w0 + lo + i] = val[j];
+        if (a.heads) a.heads[w0 + lo + i] = i == 0 || sk[i - 1] != key[j];
+      }
     }
     return;
   }
@@ -600,13 +605,14 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
     const bool em1 = i >= 1 && (km1 >> cut) == p, ep1 = i + 1 < m && (kp1 >> cut) == p;
     const bool em2 = em1 && i >= 2 && (km2 >> cut) == p, ep2 = ep1 && i + 2 < m && (kp2 >> cut) == p;
     uint32_t pos = i;
-    if (em1 && ep1 || em2 || ep2) {
+    if ((em1 && ep1) || em2 || ep2) {
       slow |= 1u << j;
       continue;
     }
     if (em1) pos = km1 <= key[j] ? i : i - 1;  // run [i-1, i]
     if (ep1) pos = kp1 < key[j] ? i + 1 : i;   // run [i, i+1]
     a.vout[w0 + lo + pos] = val[j];
+    if (a.heads) a.heads[w0 + lo + pos] = !(em1 && km1 == key[j]);
   }
 #pragma unroll 1
   for (uint32_t j = 0; j < J; ++j) {
@@ -617,11 +623,14 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
     while (rs > 0 && (sk[rs - 1] >> cut) == p) --rs;
     while (re < m && (sk[re] >> cut) == p) ++re;
     uint32_t pos = rs;
+    bool head = true;
     for (uint32_t k = rs; k < re; ++k) {
       const uint64_t c = sk[k];
       pos += c < kk || (c == kk && k < i);
+      head = head && !(c == kk && k < i);
     }
     a.vout[w0 + lo + pos] = sv[i];
+    if (a.heads) a.heads[w0 + lo + pos] = head;
   }
 }
 
@@ -685,7 +694,7 @@ static int rs_count(aln_ctx *c, int ki, bool vary, uint32_t nsuper, const RsIn &
 // kt and vt: two code arrays of 8n bytes and two row arrays of n words.
 static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uint32_t bits, const uint32_t *run,
                      uint32_t nrun, int counted, uint32_t *cnt, uint32_t *excl, uint32_t *tot,
-                     uint16_t *sub, uint64_t *const kt[2], uint32_t *const vt[2], uint32_t *vout,
+                     uint16_t *sub, uint64_t *const kt[2], uint32_t *const vt[2], uint32_t *vout, uint8_t *heads,
                      bool *done) {
   *done = false;
   const uint32_t nsuper = (uint32_t)((n + RS_SUPER - 1) / RS_SUPER);
@@ -740,6 +749,7 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
   l.keys = kt[1];
   l.vals = vt[1];
   l.vout = alias ? vt[0] : vout;
+  l.heads = heads;
   l.overflow = ovf;
   l.n = n;
   l.nblk = (uint32_t)((n + RL_W - 1) / RL_W);
@@ -788,8 +798,10 @@ static int sample_vary(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, u
 // the codes come from in.ks (first pass), else from the 8-byte array in.keys.  The values
 // land in vout (may be in.vals).  kout given: the codes land there, whole (may be in.keys);
 // otherwise each pass stores only the key bytes the later passes read.
+// heads given: *have_heads tells whether the bucket path filled it (see sort_codes).
 static int rs_sort(aln_ctx *c, RsIn in, bool from_keys, uint64_t n, uint32_t bits, uint64_t *kout,
-                   uint32_t *vout) {
+                   uint32_t *vout, uint8_t *heads = nullptr, bool *have_heads = nullptr) {
+  if (have_heads) *have_heads = false;
   if (n == 0) return ALN_OK;
   ALN_REQUIRE(bits <= 64, "radix sort: %u key bits", bits);
   ALN_REQUIRE(n < (1ull << 32), "radix sort: more than 2^32 items");
@@ -868,7 +880,8 @@ static int rs_sort(aln_ctx *c, RsIn in, bool from_keys, uint64_t n, uint32_t bit
   if (bucket && nrun >= 4) {
     bool done = false;
     uint64_t *const kt64[2] = {static_cast<uint64_t *>(kt[0]), static_cast<uint64_t *>(kt[1])};
-    ALN_TRY(rs_hybrid(c, in, from_keys, n, bits, run, nrun, counted, cnt, excl, tot, sub, kt64, vt, vout, &done));
+    ALN_TRY(rs_hybrid(c, in, from_keys, n, bits, run, nrun, counted, cnt, excl, tot, sub, kt64, vt, vout, heads, &done));
+    if (have_heads) *have_heads = done && heads;
     if (done) return ALN_OK;
     counted = -1;
   }
@@ -937,6 +950,14 @@ static int rs_sort(aln_ctx *c, RsIn in, bool from_keys, uint64_t n, uint32_t bit
     }
   }
   return ALN_OK;
+}
+
+int sort_codes(aln_ctx *c, const uint64_t *d_codes, uint64_t n, uint32_t bits, uint32_t *d_perm, uint8_t *d_heads,
+               bool *have_heads) {
+  RsIn in;
+  memset(&in, 0, sizeof(in));
+  in.keys = d_codes;
+  return rs_sort(c, in, false, n, bits, nullptr, d_perm, d_heads, have_heads);
 }
 
 int radix_sort_pairs(aln_ctx *c, uint64_t *d_keys, uint32_t *d_vals, uint64_t n, uint32_t bits) {

@@ -472,6 +472,104 @@ def test_groupby_parts(ctx, n, case):
         assert np.array_equal(host(got).view(np.float64), want)
 
 
+M64 = (1 << 64) - 1
+MUR = 0xC6A4A7935BD1E995
+
+
+def murmur_step(k):
+    k = k * MUR & M64
+    return (k ^ k >> 47) * MUR & M64
+
+
+def murmur_unstep(x):
+    """The k of murmur_step(k) = x (every part of it is a bijection)."""
+    inv = pow(MUR, -1, 1 << 64)
+    x = x * inv & M64
+    return (x ^ x >> 47) * inv & M64
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 1023, 1025, 4096, 5121, 70001, (1 << 20) + 77])
+@pytest.mark.parametrize("case", ["unique", "pairs", "runs", "one", "wide_values"])
+def test_groupby_sorted(ctx, n, case):
+    """GROUP BY by sorting: key tuples of more than 63 bits with every group one row, two rows,
+    runs over several 64-row words and 1024-row waves, one group; every aggregate (f64 with NaN),
+    one to eight distinct value columns; key and hash order; and (from 2^20 rows) one key of 40 to
+    62 bits with many groups, whose rows are sorted instead of hashed."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n + len(case))
+    groups = {"unique": 4 * n, "pairs": max(1, n // 2), "runs": max(1, n // 1500), "one": 1,
+              "wide_values": max(1, n // 3)}[case]
+    gid = r.integers(0, groups, n)
+    k0 = gid * 0x1234567ABCD1 - (1 << 62)
+    k1 = (gid % 7) * ((1 << 60) + 12345) - (1 << 62)
+    v, w = r.integers(-(1 << 62), 1 << 62, n).astype(np.int64), r.integers(-1000, 1000, n).astype(np.int64)
+    bounds = [0, n // 2, n] if n > 1 else [0, n]
+    keys = [k0.astype(np.int64), k1.astype(np.int64)]
+    if case == "one":  # two rows of other keys make the tuples wide
+        for i, x in zip(range(min(n, 2)), (-(1 << 63), (1 << 63) - 1)):
+            keys[0][i] = x
+    _gb_check(ctx, keys, [v, v, w, v], AGGS4)
+    _gb_check(ctx, keys, [v, v, w], [L.AGG_MAX, L.AGG_COUNT, L.AGG_MIN], order=L.ORDER_HASH, bounds=bounds)
+    if case == "wide_values":
+        cols = [r.integers(-1000, 1000, n).astype(np.int64) for _ in range(8)]
+        _gb_check(ctx, keys, cols, [L.AGG_SUM] * 8)
+        _gb_check(ctx, keys, cols[:5], [L.AGG_SUM] * 5, order=L.ORDER_HASH, bounds=bounds)
+    if n >= 1 << 20 and case != "one":
+        one = [(gid * 0x1234567 + 5).astype(np.int64)]
+        _gb_check(ctx, one, [v, w], [L.AGG_SUM, L.AGG_COUNT])
+        _gb_check(ctx, one, [v, w], [L.AGG_SUM, L.AGG_MIN], order=L.ORDER_HASH, bounds=bounds)
+    f = r.integers(-1000, 1000, n) / 8.0
+    nan = f.copy()
+    nan[r.random(n) < 0.3] = np.nan
+    _, inv = np.unique(keys[0], return_inverse=True)
+    g = inv.max() + 1
+    fmin, fmax = np.full(g, np.inf), np.full(g, -np.inf)
+    ok = ~np.isnan(nan)
+    np.minimum.at(fmin, inv[ok], nan[ok])
+    np.maximum.at(fmax, inv[ok], nan[ok])
+    bits = [dev(ctx, x.view(np.int64)) for x in (f, nan, nan)]
+    gk, gv = D.groupby(ctx, [dev(ctx, k) for k in keys], bits, [L.AGG_FSUM, L.AGG_FMIN, L.AGG_FMAX])
+    for got, want in zip(gv, (np.bincount(inv, weights=f, minlength=g), fmin, fmax)):
+        assert np.array_equal(host(got).view(np.float64), want)
+    if g > 1:
+        for order in (L.ORDER_KEYS, L.ORDER_HASH):
+            with pytest.raises(L.AlnError) as e:
+                D.groupby(ctx, [dev(ctx, k) for k in keys], [dev(ctx, v)], [L.AGG_SUM], order=order, cap=int(g) - 1)
+            assert e.value.code == L.ALN_E_CAPACITY
+
+
+def test_groupby_hash_clash(ctx):
+    """Key tuples made to share a MurmurHash64A stay groups of their own in hash order: by hash,
+    then by key tuple."""
+    from alenka_amd import device as D
+
+    seed, r = 100, np.random.default_rng(5)
+    h0 = seed ^ (16 * MUR & M64)
+    after = lambda k: (h0 ^ murmur_step(k)) * MUR & M64  # noqa: E731
+    sgn = lambda x: x - (1 << 64) if x >> 63 else x  # noqa: E731
+    tuples = []
+    for _ in range(50):
+        a, b, c = (int(x) for x in r.integers(0, 1 << 63, 3))
+        d = murmur_unstep(after(a) ^ after(c) ^ murmur_step(b))
+        tuples += [(a, b), (c, d)]
+        ha, hc = (L.murmur64a(np.array([sgn(x) for x in t], np.int64).tobytes(), seed) for t in ((a, b), (c, d)))
+        assert ha == hc
+    pick = r.integers(0, len(tuples), 5000)
+    keys = [np.array([sgn(tuples[i][j]) for i in pick], np.int64) for j in range(2)]
+    v = r.integers(-1000, 1000, 5000).astype(np.int64)
+    (g0, g1), (s, cnt) = D.groupby(ctx, [dev(ctx, k) for k in keys], [dev(ctx, v)] * 2, [L.AGG_SUM, L.AGG_COUNT],
+                                   order=L.ORDER_HASH, seed=seed)
+    want = {}
+    for x, y, z in zip(*keys, v):
+        t = want.setdefault((int(x), int(y)), [0, 0])
+        t[0] += int(z)
+        t[1] += 1
+    order = sorted(want, key=lambda t: (L.murmur64a(np.array(t, np.int64).tobytes(), seed), t))
+    assert list(zip(host(g0).tolist(), host(g1).tolist())) == order
+    assert host(s).tolist() == [want[t][0] for t in order] and host(cnt).tolist() == [want[t][1] for t in order]
+
+
 # ---- join --------------------------------------------------------------------------------
 @pytest.mark.parametrize("case", ["dense", "dups", "sparse", "wide", "dense_big"])
 def test_hash_join(ctx, case):
