@@ -150,8 +150,9 @@ int sum_u32_multi(aln_ctx *c, int k, const uint32_t *const *in, const uint64_t *
 // back set, heads[i] = 1 where the code at sorted position i differs from the one before.
 int sort_codes(aln_ctx *c, const uint64_t *d_codes, uint64_t n, uint32_t bits, uint32_t *d_perm, uint8_t *d_heads,
                bool *have_heads);
-int sort_keys_impl(aln_ctx *c, const int64_t *const *keys, const int32_t *desc, int nkeys, uint64_t n,
-                   uint32_t *d_perm);
+// Stable ascending order of rows by keys whose ranges are known.
+int sort_keys_ranged(aln_ctx *c, const int64_t *const *keys, int nkeys, uint64_t n, const int64_t *mn,
+                     const int64_t *mx, uint32_t *d_perm);
 int radix_sort_pairs(aln_ctx *c, uint64_t *d_keys, uint32_t *d_vals, uint64_t n,
                      uint32_t bits);
 // Batched queries (batch.hip): a batch whose device tables are carved from a caller-owned

@@ -84,7 +84,8 @@ struct GbOut {
 
 // Groups by sorting the rows (groupsort.hip): packed codes of `total` bits, or, above 63 bits, key
 // tuples.  Writes the groups in the order asked for.
-int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, int order, uint32_t seed, const GbOut &o,
-              uint64_t cap, uint64_t *h_ngroups);
+// kmax: the keys' largest values (the smallest are in a).
+int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, uint32_t seed,
+              const GbOut &o, uint64_t cap, uint64_t *h_ngroups);
 
 }  // namespace aln

@@ -444,8 +444,8 @@ __global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevR
 // added up by several blocks, which then add into the table with atomics.
 // Bounded by the moves: the key twice, each value column read, written and read again.
 constexpr uint32_t GP_LOW = 3;
-constexpr int GP_BLOCK = 512;
-constexpr int GP_ITEMS = 8;
+constexpr int GP_BLOCK = 1024;
+constexpr int GP_ITEMS = 4;
 constexpr uint32_t GP_TILE = GP_BLOCK * GP_ITEMS;
 constexpr uint32_t GP_PARTS_MIN = 64, GP_PARTS_MAX = 2048;
 constexpr uint32_t GP_BLOCKS = 512;     // moving blocks: two per CU (64 KB of LDS each)
@@ -1169,7 +1169,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     ALN_HIP(hipStreamSynchronize(c->stream));
     return ALN_OK;
   }
-  if (total > 63) return gb_sorted(c, a, n, total, order, seed, o, cap, h_ngroups);
+  if (total > 63) return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
   // LDS-cached aggregation kernel: at most 2048 blocks, of at least 4 rows per thread (450,000 rows
   // into 200,000 groups: 119 us in 55 blocks of 32 rows per thread, 50 us)
   const size_t lds = gb_lds_bytes(nvals);
@@ -1220,7 +1220,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
       hipLaunchKernelGGL(k_gb_distinct, dim3(1), dim3(1024), 0, c->stream, a, n, r);
       ALN_TRY(check_launch("gb_distinct"));
       ALN_TRY(result_wait(c, r, &found, 8));
-      if (2 * found >= GB_SAMPLE) return gb_sorted(c, a, n, total, order, seed, o, cap, h_ngroups);
+      if (2 * found >= GB_SAMPLE) return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
     }
     // open addressing: first a table for up to GB_HASH_START keys (half full at most); more
     // keys than that set the overflow flag and the rows are aggregated again in a table of

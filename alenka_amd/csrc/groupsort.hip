@@ -334,8 +334,8 @@ static int gs_by_hash(aln_ctx *c, const GbArgs &a, const GbOut &o, uint64_t g, u
 
 // One sort and reduction.  hashed: by the tuples' hashes (*clash: two tuples share one, and the
 // outputs are void); else in key order.
-static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, bool hashed, uint32_t seed, const GbOut &o,
-                  uint64_t cap, uint64_t *h_ngroups, bool *clash) {
+static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, const int64_t *kmax, bool hashed,
+                  uint32_t seed, const GbOut &o, uint64_t cap, uint64_t *h_ngroups, bool *clash) {
   *clash = false;
   GsArgs a;
   memset(&a, 0, sizeof(a));
@@ -383,7 +383,7 @@ static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, bool 
   if (coded_sort)
     ALN_TRY(sort_codes(c, code, n, hashed ? 64 : total, perm, heads, &have_heads));
   else
-    ALN_TRY(sort_keys_impl(c, g.keys, nullptr, g.nk, n, perm));
+    ALN_TRY(sort_keys_ranged(c, g.keys, g.nk, n, g.kmin, kmax, perm));
   a.row = row;
   a.code = code;
   a.perm = perm;
@@ -449,12 +449,12 @@ static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, bool 
   return ALN_OK;
 }
 
-int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, int order, uint32_t seed, const GbOut &o,
-              uint64_t cap, uint64_t *h_ngroups) {
+int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, uint32_t seed,
+              const GbOut &o, uint64_t cap, uint64_t *h_ngroups) {
   bool clash = false;
   if (order == ALN_ORDER_HASH) {
     const size_t cur = c->cur, off = c->off;
-    ALN_TRY(gs_run(c, a, n, total, true, seed, o, cap, h_ngroups, &clash));
+    ALN_TRY(gs_run(c, a, n, total, kmax, true, seed, o, cap, h_ngroups, &clash));
     if (!clash) {
       ALN_HIP(hipStreamSynchronize(c->stream));
       return ALN_OK;
@@ -462,7 +462,7 @@ int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, int order
     c->cur = cur;
     c->off = off;
   }
-  ALN_TRY(gs_run(c, a, n, total, false, seed, o, cap, h_ngroups, &clash));
+  ALN_TRY(gs_run(c, a, n, total, kmax, false, seed, o, cap, h_ngroups, &clash));
   if (order == ALN_ORDER_HASH) ALN_TRY(gs_by_hash(c, a, o, *h_ngroups, seed));
   ALN_HIP(hipStreamSynchronize(c->stream));
   return ALN_OK;

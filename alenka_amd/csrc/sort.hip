@@ -371,11 +371,14 @@ __global__ void __launch_bounds__(RS_BLOCK) k_rs_scatter(RsPass a) {
 
 // ---- bucket sort after two top-digit passes ------------------------------------------------
 // Once two stable passes on the two most significant varying digits have put the rows in
-// order of their codes' high part (code >> topshift, "buckets"), each block of k_rs_local
-// owns the buckets that start in its window of RL_W positions and sorts them, with their
-// continuation past the window, in LDS; only the permutation is stored.  A bucket that does
-// not end within RS_TILE positions of its window sets *overflow (the host then sorts by the
-// digit passes alone).
+// order of their codes' high part (code >> topshift, "buckets"), each block of k_rs_bins and
+// k_rs_local owns the buckets that start in its window of `w` positions and sorts them, with
+// their continuation past the window, in LDS; only the permutation is stored.  A bucket that
+// does not end within RS_TILE positions of its window sets *overflow (the host then tries
+// smaller windows, or sorts by the digit passes alone).
+//
+// k_rs_bins (below) places the rows by one counting pass; the windows whose rows crowd into few
+// bins (many codes with equal bits there) are left to k_rs_local, which makes no assumption:
 //
 // In the block each code's high part is replaced by its bucket's ordinal, the rows of
 // [lo, hi) are packed to LDS positions 0 .. m-1, and three or four stable LDS passes rank
@@ -385,8 +388,9 @@ __global__ void __launch_bounds__(RS_BLOCK) k_rs_scatter(RsPass a) {
 // or an equal code and an earlier position.  A run longer than RL_RUN makes the block rank
 // all remaining digits by LDS passes instead, from the order it has (which keeps equal
 // codes in input order, so the result is the same).
-constexpr uint32_t RL_W = RS_TILE / 2;
+constexpr uint32_t RL_W = RS_TILE / 2;  // the smallest window, half of a block's positions
 constexpr uint32_t RL_RUN = 32;
+constexpr uint32_t RL_OVERFLOW = 1, RL_REDO = 2;  // bits of *overflow
 
 struct RsLocal {
   const uint64_t *keys;
@@ -394,10 +398,195 @@ struct RsLocal {
   uint32_t *vout;
   uint8_t *heads;  // may be NULL: 1 where a position's code differs from the one before
   uint32_t *overflow;
+  uint8_t *redo;  // per window: left by k_rs_bins to k_rs_local
   uint64_t n;
+  uint32_t w;     // window: positions whose buckets a block owns (a multiple of 64)
+  uint32_t hish, himask;  // the most significant varying digit
   uint32_t nblk, topshift, nlow;  // nlow >= 2 remaining varying digits:
   uint32_t sh[RS_MAX_PASSES], mask[RS_MAX_PASSES];  // least significant first
 };
+
+// The window's rows by one counting pass: RB_BINS bins of (bucket ordinal, next bits of the code),
+// about a third of a row each, so a row's place is its bin's first position plus the number of
+// rows of the bin with a smaller code or an equal code and an earlier position, mostly none or one
+// to compare with (the order in which rows enter a bin does not matter).  A bin of more than
+// RL_RUN rows leaves the window to k_rs_local.  Bound by LDS operations, about 9 per row (three
+// or four stable digit passes took 40): 64M rows 955 -> 366 us.  The rows stay in registers from
+// the load to the placing; LDS holds the bins, then the placed codes with their positions (below
+// nextshift a code's bits and 12 bits of position fit 64), then the permutation.
+constexpr uint32_t RB_BINS = 8192;  // 16-bit counters, two to a word: as large as sv
+__global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) k_rs_bins(RsLocal a) {
+  __shared__ uint64_t sk[RS_TILE];
+  __shared__ uint32_t sv[RS_TILE];
+  __shared__ uint32_t wlast[RS_WAVES], wfirst[RS_WAVES], wnext[RS_WAVES], wstarts[RS_WAVES], winside[RS_WAVES];
+  __shared__ uint32_t wsum[RS_WAVES];
+  __shared__ uint32_t s_long;
+  static_assert(RB_BINS == 2 * RS_TILE && RS_TILE == 4096, "bins alias sv; 12 bits of position");
+  const unsigned t = threadIdx.x, lane = __lane_id(), wid = t / 64;
+  const uint32_t q = a.nblk / RS_XCDS, rm = a.nblk % RS_XCDS, x = blockIdx.x % RS_XCDS;
+  const uint32_t win = x * q + min(x, rm) + blockIdx.x / RS_XCDS;
+  const uint64_t n = a.n, w0 = (uint64_t)win * a.w;
+  uint64_t key[RS_ITEMS];
+  uint32_t val[RS_ITEMS], hi16[RS_ITEMS];
+  // positions w0 + i, i = wave * 512 + row * 64 + lane
+#pragma unroll
+  for (int j = 0; j < RS_ITEMS; ++j) {
+    const uint32_t i = wid * RS_WAVE_ITEMS + j * 64 + lane;
+    key[j] = w0 + i < n ? __builtin_nontemporal_load(a.keys + w0 + i) : ~0ull;
+    val[j] = w0 + i < n ? __builtin_nontemporal_load(a.vals + w0 + i) : 0u;
+  }
+  const uint64_t before = w0 > 0 ? a.keys[w0 - 1] : 0;
+  auto top = [&](uint64_t k) { return ((uint32_t)(k >> a.hish) & a.himask) << RS_BITS | ((uint32_t)(k >> a.topshift) & 0xFFu); };
+#pragma unroll
+  for (int j = 0; j < RS_ITEMS; ++j) {
+    hi16[j] = top(key[j]);
+    sv[j * RS_BLOCK + t] = 0;  // the bins
+  }
+  if (lane == 63) wlast[wid] = hi16[RS_ITEMS - 1];
+  if (t == 0) s_long = 0;
+  __syncthreads();
+  // bucket starts, their number before each row
+  uint64_t st[RS_ITEMS];
+  uint32_t starts = 0, inside = 0, first = 0xFFFFFFFFu, next = 0xFFFFFFFFu;
+#pragma unroll
+  for (int j = 0; j < RS_ITEMS; ++j) {
+    const uint32_t i0 = wid * RS_WAVE_ITEMS + j * 64;
+    uint32_t p = __shfl_up(hi16[j], 1, 64);
+    const uint32_t edge = j > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)hi16[j > 0 ? j - 1 : 0], 63)
+                                : (wid > 0 ? wlast[wid > 0 ? wid - 1 : 0] : top(before));
+    if (lane == 0) p = edge;
+    st[j] = __builtin_amdgcn_ballot_w64(w0 + i0 + lane < n && (p != hi16[j] || w0 + i0 + lane == 0));
+    const uint32_t c = (uint32_t)__popcll(st[j]);
+    starts += c;
+    if (st[j]) {
+      const uint32_t at = i0 + (uint32_t)__builtin_ctzll(st[j]);
+      if (i0 < a.w) {
+        inside += c;
+        first = first < at ? first : at;
+      } else {
+        next = next < at ? next : at;
+      }
+    }
+  }
+  if (lane == 0) {
+    wfirst[wid] = first;
+    wnext[wid] = next;
+    wstarts[wid] = starts;
+    winside[wid] = inside;
+  }
+  __syncthreads();
+  uint32_t lo = 0xFFFFFFFFu, hi = 0xFFFFFFFFu, nb = 0, seen = 0;
+#pragma unroll
+  for (unsigned w = 0; w < RS_WAVES; ++w) {
+    lo = min(lo, wfirst[w]);
+    hi = min(hi, wnext[w]);
+    nb += winside[w];
+    seen += w < wid ? wstarts[w] : 0;
+  }
+  if (lo == 0xFFFFFFFFu) return;  // no bucket starts here (uniform across the block)
+  if (hi == 0xFFFFFFFFu) {
+    if (w0 + RS_TILE < n) {  // the last bucket runs past the block's capacity
+      if (t == 0) atomicOr(a.overflow, RL_OVERFLOW);
+      return;
+    }
+    hi = (uint32_t)(n - w0);
+  }
+  const uint32_t m = hi - lo;
+  // bins: the bucket's ordinal and as many code bits below as leave RB_BINS of them
+  const uint32_t nextshift = a.sh[a.nlow - 1] + RS_BITS;
+  uint32_t kb = 13 - (nb > 1 ? 32 - (uint32_t)__builtin_clz(nb - 1) : 0u);
+  kb = kb < nextshift ? kb : nextshift;
+  const uint32_t bsh = nextshift - kb, bmask = (1u << kb) - 1u;
+  uint32_t bin[RS_ITEMS], rank[RS_ITEMS];
+#pragma unroll
+  for (int j = 0; j < RS_ITEMS; ++j) {
+    const uint32_t i = wid * RS_WAVE_ITEMS + j * 64 + lane;
+    const uint32_t ord = seen + below_count(st[j]) + (uint32_t)(st[j] >> lane & 1) - 1u;
+    seen += (uint32_t)__popcll(st[j]);
+    bin[j] = ord << kb | ((uint32_t)(key[j] >> bsh) & bmask);
+    if (i >= lo && i < hi) {
+      const uint32_t s16 = (bin[j] & 1) * 16;
+      rank[j] = atomicAdd(&sv[bin[j] >> 1], 1u << s16) >> s16 & 0xFFFFu;
+    }
+  }
+  __syncthreads();
+  // first positions of the bins: thread t holds bins 16 t .. 16 t + 15
+  {
+    uint4 *hb = reinterpret_cast<uint4 *>(sv) + 2 * t;
+    uint4 h0 = hb[0], h1 = hb[1];
+    uint32_t c[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w}, sum = 0;
+    bool crowd = false;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const uint32_t e = c[k] & 0xFFFFu, o = c[k] >> 16;
+      crowd = crowd || e > RL_RUN || o > RL_RUN;
+      c[k] = sum | (sum + e) << 16;
+      sum += e + o;
+    }
+    const uint32_t incl = wave_incl_scan(sum);
+    if (lane == 63) wsum[wid] = incl;
+    if (crowd) s_long = 1;
+    __syncthreads();
+    if (s_long) {
+      if (t == 0) {
+        a.redo[win] = 1;
+        atomicOr(a.overflow, RL_REDO);
+      }
+      return;
+    }
+    uint32_t base = incl - sum;
+#pragma unroll
+    for (unsigned w = 0; w < RS_WAVES; ++w) base += w < wid ? wsum[w] : 0;
+    const uint32_t b2 = base | base << 16;
+    hb[0] = make_uint4(c[0] + b2, c[1] + b2, c[2] + b2, c[3] + b2);
+    hb[1] = make_uint4(c[4] + b2, c[5] + b2, c[6] + b2, c[7] + b2);
+  }
+  __syncthreads();
+  const uint64_t lowmask = (1ull << nextshift) - 1;
+#pragma unroll
+  for (int j = 0; j < RS_ITEMS; ++j) {
+    const uint32_t i = wid * RS_WAVE_ITEMS + j * 64 + lane;
+    key[j] = (key[j] & lowmask) << 12 | i;
+    if (i >= lo && i < hi) {
+      const uint32_t b = bin[j], e = b + 1;
+      const uint32_t base = sv[b >> 1] >> ((b & 1) * 16) & 0xFFFFu;
+      const uint32_t end = e < RB_BINS ? sv[e >> 1] >> ((e & 1) * 16) & 0xFFFFu : m;
+      sk[base + rank[j]] = key[j];
+      bin[j] = base;
+      rank[j] = end - base;  // rows of the bin
+    } else {
+      rank[j] = 0;
+    }
+  }
+  __syncthreads();
+  uint32_t heads = 0;
+#pragma unroll
+  for (int j = 0; j < RS_ITEMS; ++j) {
+    if (rank[j] == 0) continue;
+    uint32_t pos = bin[j];
+    bool head = true;
+    if (rank[j] > 1) {
+      for (uint32_t k = bin[j]; k < bin[j] + rank[j]; ++k) {
+        const uint64_t c = sk[k];
+        pos += c < key[j];
+        head = head && !(c < key[j] && c >> 12 == key[j] >> 12);
+      }
+    }
+    sv[pos] = val[j];
+    heads |= (head ? 1u : 0u) << j;
+    bin[j] = pos;
+  }
+  __syncthreads();
+  for (uint32_t k = t; k < m; k += RS_BLOCK) a.vout[w0 + lo + k] = sv[k];
+  if (a.heads) {
+    uint8_t *hb = reinterpret_cast<uint8_t *>(sk);  // the placed codes have been read
+#pragma unroll
+    for (int j = 0; j < RS_ITEMS; ++j)
+      if (rank[j]) hb[bin[j]] = (uint8_t)(heads >> j & 1);
+    __syncthreads();
+    for (uint32_t k = t; k < m; k += RS_BLOCK) a.heads[w0 + lo + k] = hb[k];
+  }
+}
 
 // 6 waves per SIMD: three blocks per CU, as many as the LDS holds
 __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) k_rs_local(RsLocal a) {
@@ -409,7 +598,9 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   const unsigned t = threadIdx.x, lane = __lane_id(), wid = t / 64;
   // each XCD takes a contiguous range of windows: neighbours share RL_W codes and one L2
   const uint32_t q = a.nblk / RS_XCDS, rm = a.nblk % RS_XCDS, x = blockIdx.x % RS_XCDS;
-  const uint64_t n = a.n, w0 = (uint64_t)(x * q + min(x, rm) + blockIdx.x / RS_XCDS) * RL_W;
+  const uint32_t win = x * q + min(x, rm) + blockIdx.x / RS_XCDS;
+  if (!a.redo[win]) return;
+  const uint64_t n = a.n, w0 = (uint64_t)win * a.w;
   uint64_t key[RS_ITEMS];
   uint32_t val[RS_ITEMS], rank[RS_ITEMS];
   if (t == 0) {
@@ -434,7 +625,7 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   for (int j = 0; j < RS_ITEMS; ++j) {
     const uint32_t i = wid * RS_WAVE_ITEMS + j * 64 + lane;
     st[j] = w0 + i < n && (w0 + i == 0 || (i == 0 ? tprev : sk[i - 1]) != sk[i]);
-    if (st[j]) atomicMin(i < RL_W ? &s_lo : &s_hi, i);
+    if (st[j]) atomicMin(i < a.w ? &s_lo : &s_hi, i);
   }
   __syncthreads();
   const uint32_t lo = s_lo;
@@ -442,7 +633,7 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   uint32_t hi = s_hi;
   if (hi == 0xFFFFFFFFu) {
     if (w0 + RS_TILE < n) {  // the last bucket runs past the block's capacity
-      if (t == 0) atomicOr(a.overflow, 1u);
+      if (t == 0) atomicOr(a.overflow, RL_OVERFLOW);
       return;
     }
     hi = (uint32_t)(n - w0);
@@ -693,7 +884,7 @@ static int rs_count(aln_ctx *c, int ki, bool vary, uint32_t nsuper, const RsIn &
 // The bucket path of rs_sort (see k_rs_local): *done = false when a bucket overflowed.
 // kt and vt: two code arrays of 8n bytes and two row arrays of n words.
 static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uint32_t bits, const uint32_t *run,
-                     uint32_t nrun, int counted, uint32_t *cnt, uint32_t *excl, uint32_t *tot,
+                     uint32_t nrun, uint64_t vary, int counted, uint32_t *cnt, uint32_t *excl, uint32_t *tot,
                      uint16_t *sub, uint64_t *const kt[2], uint32_t *const vt[2], uint32_t *vout, uint8_t *heads,
                      bool *done) {
   *done = false;
@@ -705,7 +896,12 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
   };
   uint32_t *ovf;
   ALN_TRY(ws(c, 1, &ovf));
-  ALN_TRY(fill_u32(c, ovf, 1, 0));
+  // the wide window: room for a bucket of 1.25 x the mean (over the codes that the top two
+  // digits' varying bits make) and 256 rows more
+  const int top_bits = __builtin_popcountll(vary >> (RS_BITS * run[nrun - 1]) & pass_mask(run[nrun - 1])) +
+                       __builtin_popcountll(vary >> (RS_BITS * run[nrun - 2]) & pass_mask(run[nrun - 2]));
+  const uint64_t tail = (n >> top_bits) + (n >> top_bits) / 4 + 256;
+  const uint32_t wide = tail < RS_TILE - RL_W ? (uint32_t)(RS_TILE - tail) & ~63u : RL_W;
   // two passes: the second most significant varying digit, then the most significant
   for (uint32_t r = 0; r < 2; ++r) {
     const uint32_t p = run[nrun - 2 + r];
@@ -752,55 +948,57 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
   l.heads = heads;
   l.overflow = ovf;
   l.n = n;
-  l.nblk = (uint32_t)((n + RL_W - 1) / RL_W);
   l.topshift = RS_BITS * run[nrun - 2];
+  l.hish = RS_BITS * run[nrun - 1];
+  l.himask = pass_mask(run[nrun - 1]);
   l.nlow = nrun - 2;
   for (uint32_t r = 0; r + 2 < nrun; ++r) {
     l.sh[r] = RS_BITS * run[r];
     l.mask[r] = pass_mask(run[r]);
   }
-  {
-    ProfScope ps(c, "radix_local");
-    hipLaunchKernelGGL(k_rs_local, dim3(l.nblk), dim3(RS_BLOCK), 0, c->stream, l);
+  uint32_t o = RL_OVERFLOW;
+  ALN_TRY(ws(c, (size_t)((n + RL_W - 1) / RL_W) + 4, &l.redo));
+  // Windows as wide as leave room for the last bucket (each block reads RS_TILE positions for its
+  // window): buckets of spread codes hold the mean and a few deviations more.  If one does
+  // not fit, windows of half a tile.
+  for (uint32_t w = wide; o & RL_OVERFLOW; w = RL_W) {
+    l.w = w;
+    l.nblk = (uint32_t)((n + w - 1) / w);
+    ALN_TRY(fill_u32(c, ovf, 1, 0));
+    ALN_TRY(fill_u32(c, reinterpret_cast<uint32_t *>(l.redo), (l.nblk + 3) / 4, 0));
+    {
+      ProfScope ps(c, "radix_local");
+      hipLaunchKernelGGL(k_rs_bins, dim3(l.nblk), dim3(RS_BLOCK), 0, c->stream, l);
+    }
+    ALN_TRY(check_launch("radix_bins"));
+    ALN_TRY(copy_to_host(c, &o, ovf, 4));
+    if (w == RL_W) break;
   }
-  ALN_TRY(check_launch("radix_local"));
-  uint32_t o = 0;
-  ALN_TRY(copy_to_host(c, &o, ovf, 4));
+  if (o == RL_REDO) {
+    {
+      ProfScope ps(c, "radix_local");
+      hipLaunchKernelGGL(k_rs_local, dim3(l.nblk), dim3(RS_BLOCK), 0, c->stream, l);
+    }
+    ALN_TRY(check_launch("radix_local"));
+    ALN_TRY(copy_to_host(c, &o, ovf, 4));
+    o &= RL_OVERFLOW;
+  }
   *done = o == 0;
   if (*done && alias) ALN_HIP(hipMemcpyAsync(vout, vt[0], 4ull * n, hipMemcpyDeviceToDevice, c->stream));
   return ALN_OK;
 }
 
-// The bits in which the codes of the first RS_SAMPLE positions differ (a subset of those in
-// which all codes differ), computed on the host.
+// Rows of a sample of a key column, read back by the host.
 constexpr uint64_t RS_SAMPLE = 4096;
-static int sample_vary(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uint64_t *vary) {
-  const uint64_t m = std::min<uint64_t>(n, RS_SAMPLE);
-  std::vector<uint64_t> code(m, 0);
-  if (!from_keys) {
-    ALN_TRY(copy_to_host(c, code.data(), in.keys, 8 * m));
-  } else {  // the first rows' keys: a sample of the rows whatever order in.vals gives them
-    std::vector<int64_t> v(m);
-    for (int k = 0; k < in.ks.n; ++k) {
-      ALN_TRY(copy_to_host(c, v.data(), in.ks.k[k], 8 * m));
-      for (uint64_t r = 0; r < m; ++r) {
-        const uint64_t f = in.ks.desc[k] ? (uint64_t)in.ks.ref[k] - (uint64_t)v[r] : (uint64_t)v[r] - (uint64_t)in.ks.ref[k];
-        if (in.ks.shift[k] < 64) code[r] |= f << in.ks.shift[k];
-      }
-    }
-  }
-  *vary = 0;
-  for (uint64_t r = 0; r < m; ++r) *vary |= code[r] ^ code[0];
-  return ALN_OK;
-}
 
 // Stable LSD sort of the items of `in` by the low `bits` bits of their codes.  from_keys:
 // the codes come from in.ks (first pass), else from the 8-byte array in.keys.  The values
 // land in vout (may be in.vals).  kout given: the codes land there, whole (may be in.keys);
 // otherwise each pass stores only the key bytes the later passes read.
-// heads given: *have_heads tells whether the bucket path filled it (see sort_codes).
+// heads given: *have_heads tells whether the bucket path filled it (see sort_codes).  guess: bits
+// in which the codes are expected to differ (what is counted first depends on it, not the result).
 static int rs_sort(aln_ctx *c, RsIn in, bool from_keys, uint64_t n, uint32_t bits, uint64_t *kout,
-                   uint32_t *vout, uint8_t *heads = nullptr, bool *have_heads = nullptr) {
+                   uint32_t *vout, uint8_t *heads = nullptr, bool *have_heads = nullptr, uint64_t guess = ~0ull) {
   if (have_heads) *have_heads = false;
   if (n == 0) return ALN_OK;
   ALN_REQUIRE(bits <= 64, "radix sort: %u key bits", bits);
@@ -832,12 +1030,10 @@ static int rs_sort(aln_ctx *c, RsIn in, bool from_keys, uint64_t n, uint32_t bit
   int counted = -1;  // the digit whose counts of the input are in cnt and sub
   if (passes > 0) {
     counted = 0;
-    if (bucket) {  // the second most significant digit in which a sample of the codes differ
-      uint64_t sv = 0;
-      ALN_TRY(sample_vary(c, in, from_keys, n, &sv));
+    if (bucket) {  // the second most significant digit expected to vary
       int top = -1;
       for (int p = (int)passes - 1; p >= 0; --p)
-        if ((sv >> (RS_BITS * p)) & pass_mask(p)) {
+        if ((guess >> (RS_BITS * p)) & pass_mask(p)) {
           if (top >= 0) {
             counted = p;
             break;
@@ -880,7 +1076,7 @@ static int rs_sort(aln_ctx *c, RsIn in, bool from_keys, uint64_t n, uint32_t bit
   if (bucket && nrun >= 4) {
     bool done = false;
     uint64_t *const kt64[2] = {static_cast<uint64_t *>(kt[0]), static_cast<uint64_t *>(kt[1])};
-    ALN_TRY(rs_hybrid(c, in, from_keys, n, bits, run, nrun, counted, cnt, excl, tot, sub, kt64, vt, vout, heads, &done));
+    ALN_TRY(rs_hybrid(c, in, from_keys, n, bits, run, nrun, vary, counted, cnt, excl, tot, sub, kt64, vt, vout, heads, &done));
     if (have_heads) *have_heads = done && heads;
     if (done) return ALN_OK;
     counted = -1;
@@ -1006,12 +1202,12 @@ static uint32_t key_set(const KeyRanges &r, const int64_t *const *keys, const in
 }
 
 static int sort_with_ranges(aln_ctx *c, const KeyRanges &r, const int64_t *const *keys,
-                            const int32_t *desc, int nkeys, uint64_t n, uint32_t *d_perm) {
+                            const int32_t *desc, int nkeys, uint64_t n, uint32_t *d_perm, uint64_t guess = ~0ull) {
   RsIn in;
   memset(&in, 0, sizeof(in));
   if (r.total <= 64) {  // one sort of the concatenated codes, computed by its first pass
     key_set(r, keys, desc, 0, nkeys, &in.ks);
-    return rs_sort(c, in, true, n, r.total, nullptr, d_perm);
+    return rs_sort(c, in, true, n, r.total, nullptr, d_perm, nullptr, nullptr, guess);
   }
   // LSD over keys, last key first, each sort stable (sorts.cu:17-70); each reads its key at
   // the rows of the permutation so far
@@ -1023,13 +1219,27 @@ static int sort_with_ranges(aln_ctx *c, const KeyRanges &r, const int64_t *const
   return ALN_OK;
 }
 
-int sort_keys_impl(aln_ctx *c, const int64_t *const *keys, const int32_t *desc, int nkeys,
-                   uint64_t n, uint32_t *d_perm) {
+int sort_keys_ranged(aln_ctx *c, const int64_t *const *keys, int nkeys, uint64_t n, const int64_t *mn,
+                     const int64_t *mx, uint32_t *d_perm) {
+  KeyRanges r;
+  r.total = 0;
+  for (int k = 0; k < nkeys; ++k) {
+    r.mn[k] = mn[k];
+    r.mx[k] = mx[k];
+    r.bits[k] = bits_for_range_u((uint64_t)mx[k] - (uint64_t)mn[k]);
+    r.total += r.bits[k];
+  }
+  return sort_with_ranges(c, r, keys, nullptr, nkeys, n, d_perm);
+}
+
+static int sort_keys_impl(aln_ctx *c, const int64_t *const *keys, const int32_t *desc, int nkeys,
+                          uint64_t n, uint32_t *d_perm) {
   ALN_REQUIRE(nkeys >= 1 && nkeys <= ALN_MAX_KEYS, "sort: %d keys", nkeys);
   ALN_REQUIRE(n < (1ull << 32), "sort: more than 2^32 rows");
   if (n == 0) return ALN_OK;
   KeyRanges r;
   bool whole = false;
+  uint64_t guess = ~0ull;
   if (nkeys == 1 && n >= RS_SYNC_MIN) {
     // One key: codes over the whole int64 range, no min/max pass; the count pass finds the
     // digits every key shares and those passes are skipped.  Unless values of a narrow range
@@ -1045,6 +1255,7 @@ int sort_keys_impl(aln_ctx *c, const int64_t *const *keys, const int32_t *desc, 
       hi = std::max(hi, x);
     }
     whole = bits_for_range_u(vary) <= bits_for_range_u((uint64_t)hi - (uint64_t)lo) + RS_BITS;
+    if (whole && vary) guess = vary;
   }
   if (whole) {
     r.mn[0] = INT64_MIN;
@@ -1053,7 +1264,7 @@ int sort_keys_impl(aln_ctx *c, const int64_t *const *keys, const int32_t *desc, 
   } else {
     ALN_TRY(key_ranges(c, keys, nkeys, n, &r));
   }
-  return sort_with_ranges(c, r, keys, desc, nkeys, n, d_perm);
+  return sort_with_ranges(c, r, keys, desc, nkeys, n, d_perm, guess);
 }
 
 // ---- top-k: tile-wise bitonic sort of (code, index), keep the first k of each tile -----
