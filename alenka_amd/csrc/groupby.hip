@@ -444,11 +444,12 @@ __global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevR
 // added up by several blocks, which then add into the table with atomics.
 // Bounded by the moves: the key twice, each value column read, written and read again.
 constexpr uint32_t GP_LOW = 3;
-constexpr int GP_BLOCK = 1024;
-constexpr int GP_ITEMS = 4;
+constexpr int GP_BLOCK = 512;
+constexpr int GP_ITEMS = 8;
 constexpr uint32_t GP_TILE = GP_BLOCK * GP_ITEMS;
 constexpr uint32_t GP_PARTS_MIN = 64, GP_PARTS_MAX = 2048;
-constexpr uint32_t GP_BLOCKS = 512;     // moving blocks: two per CU (64 KB of LDS each)
+constexpr uint32_t GP_SUB = 8;           // tiles a count block counts
+constexpr uint32_t GP_XCDS = 8;
 constexpr uint64_t GP_ROWS_MIN = 1ull << 20;
 constexpr uint64_t GP_BYTES_MAX = 16ull << 30;  // moved rows
 constexpr size_t GP_LDS = 65536, GP_LDS_MAX = 131072;
@@ -461,16 +462,17 @@ struct GpArgs {
   int64_t *moved[ALN_MAX_AGGS];
   int32_t col_of[ALN_MAX_AGGS + 1];
   uint32_t *code;          // moved codes
-  uint64_t n, per;         // rows, rows per moving block
-  uint32_t nblk, lp, ncodes, chunk;
-  uint32_t *cnts, *excl, *tot;   // [part][block], [block][part], [part]
+  uint64_t n;
+  uint32_t ntiles, nsuper, lp, ncodes, chunk;  // nsuper: count blocks, of GP_SUB tiles
+  uint32_t *cnts, *excl, *tot;   // [part][count block], [count block][part], [part]
+  uint16_t *sub;                 // [tile][part]: the part's rows in the count block's earlier tiles
   uint32_t *start, *work;        // [parts + 1]: first row, first work item of a part
 };
 
 __device__ __forceinline__ uint32_t gp_part(uint32_t code, uint32_t lp) { return (code >> GP_LOW) & ((1u << lp) - 1u); }
 
-// The codes of rows i0 + 512 * j + thread below i1 (others 0).
-__device__ __forceinline__ void gp_codes(const GpArgs &a, uint64_t i0, uint64_t i1, uint32_t (&code)[GP_ITEMS]) {
+// The codes of the tile's rows GP_BLOCK * j + thread (past the end: 0).
+__device__ __forceinline__ void gp_codes(const GpArgs &a, uint64_t i0, uint32_t (&code)[GP_ITEMS]) {
 #pragma unroll
   for (int j = 0; j < GP_ITEMS; ++j) code[j] = 0;
   for (int k = 0; k < a.g.nk; ++k) {
@@ -479,7 +481,7 @@ __device__ __forceinline__ void gp_codes(const GpArgs &a, uint64_t i0, uint64_t 
 #pragma unroll
     for (int j = 0; j < GP_ITEMS; ++j) {
       const uint64_t i = i0 + threadIdx.x + GP_BLOCK * j;
-      x[j] = i < i1 ? __builtin_nontemporal_load(key + i) : a.g.kmin[k];
+      x[j] = i < a.n ? __builtin_nontemporal_load(key + i) : a.g.kmin[k];
     }
 #pragma unroll
     for (int j = 0; j < GP_ITEMS; ++j)
@@ -487,34 +489,50 @@ __device__ __forceinline__ void gp_codes(const GpArgs &a, uint64_t i0, uint64_t 
   }
 }
 
+// The counters of a tile: GP_PARTS_MAX of them, that many copies per part, spread over the lanes.
 __global__ void __launch_bounds__(GP_BLOCK) k_gp_count(GpArgs a) {
   __shared__ uint32_t h[GP_PARTS_MAX];
-  const uint32_t parts = 1u << a.lp;
-  for (uint32_t p = threadIdx.x; p < parts; p += GP_BLOCK) h[p] = 0;
-  __syncthreads();
-  const uint64_t r0 = blockIdx.x * a.per, r1 = r0 + a.per < a.n ? r0 + a.per : a.n;
-  for (uint64_t i0 = r0; i0 < r1; i0 += GP_TILE) {
+  constexpr uint32_t PER = GP_PARTS_MAX / GP_BLOCK;
+  const uint32_t parts = 1u << a.lp, copies = GP_PARTS_MAX >> a.lp, copy = threadIdx.x & (copies - 1);
+  uint32_t run[PER];  // of parts thread, thread + GP_BLOCK, ..
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) run[q] = 0;
+  for (uint32_t s = 0; s < GP_SUB; ++s) {
+    const uint64_t tile = (uint64_t)blockIdx.x * GP_SUB + s, i0 = tile * GP_TILE;
+    if (i0 >= a.n) break;
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) h[threadIdx.x + GP_BLOCK * q] = 0;
     uint32_t code[GP_ITEMS];
-    gp_codes(a, i0, r1, code);
+    gp_codes(a, i0, code);
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < GP_ITEMS; ++j)
-      if (i0 + threadIdx.x + GP_BLOCK * j < r1) atomicAdd(&h[gp_part(code[j], a.lp)], 1u);
+      if (i0 + threadIdx.x + GP_BLOCK * j < a.n) atomicAdd(&h[gp_part(code[j], a.lp) * copies + copy], 1u);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+      const uint32_t p = threadIdx.x + GP_BLOCK * q;
+      if (p >= parts) continue;
+      a.sub[tile * parts + p] = (uint16_t)run[q];
+      for (uint32_t k = 0; k < copies; ++k) run[q] += h[p * copies + ((k + p) & (copies - 1))];
+    }
+    __syncthreads();
   }
-  __syncthreads();
-  for (uint32_t p = threadIdx.x; p < parts; p += GP_BLOCK) a.cnts[(uint64_t)p * a.nblk + blockIdx.x] = h[p];
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {
+    const uint32_t p = threadIdx.x + GP_BLOCK * q;
+    if (p < parts) a.cnts[(uint64_t)p * a.nsuper + blockIdx.x] = run[q];
+  }
 }
 
-// Block p: exclusive scan of part p's block counts (nblk <= GP_BLOCKS = 2 * 256).
+// Block p: exclusive scan of part p's counts.
 __global__ void __launch_bounds__(256) k_gp_rows(GpArgs a) {
   __shared__ uint32_t wsum[4];
   const uint32_t p = blockIdx.x, t = threadIdx.x, parts = 1u << a.lp;
-  uint32_t c[2], s = 0;
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const uint32_t b = 2 * t + j;
-    c[j] = b < a.nblk ? a.cnts[(uint64_t)p * a.nblk + b] : 0;
-    s += c[j];
-  }
+  const uint32_t per = (a.nsuper + 255) / 256, b = t * per, e = b + per < a.nsuper ? b + per : a.nsuper;
+  const uint32_t *row = a.cnts + (uint64_t)p * a.nsuper;
+  uint32_t s = 0;
+  for (uint32_t i = b; i < e; ++i) s += row[i];
   uint32_t x = s;
   for (int o = 1; o < 64; o <<= 1) {
     const uint32_t y = __shfl_up(x, o, 64);
@@ -524,11 +542,9 @@ __global__ void __launch_bounds__(256) k_gp_rows(GpArgs a) {
   __syncthreads();
   uint32_t before = x - s;
   for (uint32_t w = 0; w < t / 64; ++w) before += wsum[w];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const uint32_t b = 2 * t + j;
-    if (b < a.nblk) a.excl[(uint64_t)b * parts + p] = before;
-    before += c[j];
+  for (uint32_t i = b; i < e; ++i) {
+    a.excl[(uint64_t)i * parts + p] = before;
+    before += row[i];
   }
   if (t == 255) a.tot[p] = before;
 }
@@ -576,8 +592,11 @@ __global__ void __launch_bounds__(1024) k_gp_base(GpArgs a) {
     if (p + j < parts) a.work[p + j] = w[j];
 }
 
-// Moves a block's rows into part order.  off: each part's next position; within a tile the
-// order of a part's rows is free, so a row's place is an LDS counter's old value.
+// Moves a tile's rows into part order.  Within a tile the order of a part's rows is free, so a
+// row's place is an LDS counter's old value.  Each XCD takes a contiguous range of tiles, so the
+// runs of neighbouring tiles meet in one L2 (a block with tiles and part positions of its own
+// kept 64 x 512 open lines per XCD, more than its L2: 265 against 163 us for 30M rows, one key
+// and one value column).
 __global__ void __launch_bounds__(GP_BLOCK) k_gp_move(GpArgs a) {
   __shared__ int64_t sv[GP_TILE];
   __shared__ uint32_t sc[GP_TILE];
@@ -586,84 +605,86 @@ __global__ void __launch_bounds__(GP_BLOCK) k_gp_move(GpArgs a) {
   static_assert(12 * GP_TILE + 8 * GP_PARTS_MAX <= 65536, "two blocks per CU");
   constexpr uint32_t PER = GP_PARTS_MAX / GP_BLOCK;
   const uint32_t parts = 1u << a.lp, t = threadIdx.x;
-  const uint64_t r0 = blockIdx.x * a.per, r1 = r0 + a.per < a.n ? r0 + a.per : a.n;
-  // thread t owns parts t * PER .. + PER - 1: their next positions stay in registers
-  uint32_t off[PER];
+  const uint32_t copies = GP_PARTS_MAX >> a.lp, copy = t & (copies - 1);
+  const uint32_t xq = a.ntiles / GP_XCDS, xr = a.ntiles % GP_XCDS, xcd = blockIdx.x % GP_XCDS;
+  const uint32_t tile = xcd * xq + (xcd < xr ? xcd : xr) + blockIdx.x / GP_XCDS;
+  const uint64_t i0 = (uint64_t)tile * GP_TILE;
+  const uint32_t m = a.n - i0 < GP_TILE ? (uint32_t)(a.n - i0) : GP_TILE;
+  uint32_t code[GP_ITEMS], rank[GP_ITEMS], off[PER];
+  gp_codes(a, i0, code);
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {  // the tile's first positions in parts t, t + GP_BLOCK, ..
+    const uint32_t p = t + GP_BLOCK * q;
+    off[q] = p < parts ? a.start[p] + a.excl[(uint64_t)(tile / GP_SUB) * parts + p] + a.sub[(uint64_t)tile * parts + p]
+                       : 0;
+    h[t + GP_BLOCK * q] = 0;
+  }
+  int64_t y[GP_ITEMS];  // the first column's values, on their way while the rows are placed
+#pragma unroll
+  for (int j = 0; j < GP_ITEMS; ++j)
+    y[j] = a.ncol && t + GP_BLOCK * j < m ? __builtin_nontemporal_load(a.col[0] + i0 + t + GP_BLOCK * j) : 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < GP_ITEMS; ++j)
+    if (t + GP_BLOCK * j < m) rank[j] = atomicAdd(&h[gp_part(code[j], a.lp) * copies + copy], 1u);
+  __syncthreads();
+  uint32_t c[PER], s = 0;
 #pragma unroll
   for (uint32_t q = 0; q < PER; ++q) {
-    const uint32_t p = t * PER + q;
-    off[q] = p < parts ? a.start[p] + a.excl[(uint64_t)blockIdx.x * parts + p] : 0;
-    h[p] = 0;
+    c[q] = h[t * PER + q];
+    s += c[q];
+  }
+  uint32_t x = s;
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t z = __shfl_up(x, o, 64);
+    if (__lane_id() >= (unsigned)o) x += z;
+  }
+  if (__lane_id() == 63) wsum[t / 64] = x;
+  __syncthreads();
+  uint32_t before = x - s;
+  for (uint32_t w = 0; w < t / 64; ++w) before += wsum[w];
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {
+    h[t * PER + q] = before;  // the counter's first place in the tile
+    before += c[q];
   }
   __syncthreads();
-  for (uint64_t i0 = r0; i0 < r1; i0 += GP_TILE) {
-    uint32_t code[GP_ITEMS], rank[GP_ITEMS];
-    gp_codes(a, i0, r1, code);
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {
+    const uint32_t p = t + GP_BLOCK * q;
+    if (p < parts) del[p] = off[q] - h[p * copies];
+  }
+#pragma unroll
+  for (int j = 0; j < GP_ITEMS; ++j)
+    if (t + GP_BLOCK * j < m) {
+      rank[j] += h[gp_part(code[j], a.lp) * copies + copy];
+      sc[rank[j]] = code[j];
+      if (a.ncol) sv[rank[j]] = y[j];
+    }
+  __syncthreads();
+  uint32_t dest[GP_ITEMS];
+#pragma unroll
+  for (int j = 0; j < GP_ITEMS; ++j) {
+    const uint32_t i = t + GP_BLOCK * j;
+    if (i < m) {
+      const uint32_t cd = sc[i];
+      dest[j] = del[gp_part(cd, a.lp)] + i;
+      a.code[dest[j]] = cd;
+      if (a.ncol) a.moved[0][dest[j]] = sv[i];
+    }
+  }
+  for (int v = 1; v < a.ncol; ++v) {
 #pragma unroll
     for (int j = 0; j < GP_ITEMS; ++j)
-      if (i0 + t + GP_BLOCK * j < r1) rank[j] = atomicAdd(&h[gp_part(code[j], a.lp)], 1u);
-    __syncthreads();
-    uint32_t c[PER], s = 0;
+      y[j] = t + GP_BLOCK * j < m ? __builtin_nontemporal_load(a.col[v] + i0 + t + GP_BLOCK * j) : 0;
+    __syncthreads();  // the last column has left sv
 #pragma unroll
-    for (uint32_t q = 0; q < PER; ++q) {
-      c[q] = h[t * PER + q];
-      s += c[q];
-    }
-    uint32_t x = s;
-    for (int o = 1; o < 64; o <<= 1) {
-      const uint32_t y = __shfl_up(x, o, 64);
-      if (__lane_id() >= (unsigned)o) x += y;
-    }
-    if (__lane_id() == 63) wsum[t / 64] = x;
-    __syncthreads();
-    uint32_t before = x - s;
-    for (uint32_t w = 0; w < t / 64; ++w) before += wsum[w];
-#pragma unroll
-    for (uint32_t q = 0; q < PER; ++q) {
-      h[t * PER + q] = before;  // the part's first place in the tile
-      del[t * PER + q] = off[q] - before;
-      before += c[q];
-      off[q] += c[q];
-    }
+    for (int j = 0; j < GP_ITEMS; ++j)
+      if (t + GP_BLOCK * j < m) sv[rank[j]] = y[j];
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < GP_ITEMS; ++j)
-      if (i0 + t + GP_BLOCK * j < r1) {
-        rank[j] += h[gp_part(code[j], a.lp)];
-        sc[rank[j]] = code[j];
-      }
-    __syncthreads();
-    const uint32_t m = r1 - i0 < GP_TILE ? (uint32_t)(r1 - i0) : GP_TILE;
-    uint32_t dest[GP_ITEMS];
-#pragma unroll
-    for (int j = 0; j < GP_ITEMS; ++j) {
-      const uint32_t i = t + GP_BLOCK * j;
-      if (i < m) {
-        const uint32_t cd = sc[i];
-        dest[j] = del[gp_part(cd, a.lp)] + i;
-        a.code[dest[j]] = cd;
-      }
-    }
-    for (int v = 0; v < a.ncol; ++v) {
-      int64_t y[GP_ITEMS];
-#pragma unroll
-      for (int j = 0; j < GP_ITEMS; ++j) {
-        const uint64_t i = i0 + t + GP_BLOCK * j;
-        y[j] = i < r1 ? __builtin_nontemporal_load(a.col[v] + i) : 0;
-      }
-      if (v) __syncthreads();  // the last column has left sv
-#pragma unroll
-      for (int j = 0; j < GP_ITEMS; ++j)
-        if (i0 + t + GP_BLOCK * j < r1) sv[rank[j]] = y[j];
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < GP_ITEMS; ++j)
-        if (t + GP_BLOCK * j < m) a.moved[v][dest[j]] = sv[t + GP_BLOCK * j];
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t q = 0; q < PER; ++q) h[t * PER + q] = 0;
-    __syncthreads();
+      if (t + GP_BLOCK * j < m) a.moved[v][dest[j]] = sv[t + GP_BLOCK * j];
   }
 }
 
@@ -1039,15 +1060,16 @@ static int gb_parts(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int *cnt,
   if (bytes / parts > GP_LDS_MAX || parts > g.ncodes >> GP_LOW) return ALN_OK;
   g.lp = 31 - __builtin_clz(parts);
   if (n * (4 + 8ull * g.ncol) > GP_BYTES_MAX) return ALN_OK;
-  g.per = (n + GP_BLOCKS - 1) / GP_BLOCKS;
-  g.nblk = (uint32_t)((n + g.per - 1) / g.per);
+  g.ntiles = (uint32_t)((n + GP_TILE - 1) / GP_TILE);
+  g.nsuper = (g.ntiles + GP_SUB - 1) / GP_SUB;
   const uint64_t chunk = 2 * n / parts;
   g.chunk = (uint32_t)(chunk < 32768 ? 32768 : chunk);
   const size_t cur = c->cur, off = c->off;
   int r = ws(c, n, &g.code);
   for (int k = 0; k < g.ncol && r == ALN_OK; ++k) r = ws(c, n, &g.moved[k]);
-  if (r == ALN_OK) r = ws(c, (size_t)parts * g.nblk, &g.cnts);
-  if (r == ALN_OK) r = ws(c, (size_t)parts * g.nblk, &g.excl);
+  if (r == ALN_OK) r = ws(c, (size_t)parts * g.nsuper, &g.cnts);
+  if (r == ALN_OK) r = ws(c, (size_t)parts * g.nsuper, &g.excl);
+  if (r == ALN_OK) r = ws(c, (size_t)parts * g.ntiles, &g.sub);
   if (r == ALN_OK) r = ws(c, parts, &g.tot);
   if (r == ALN_OK) r = ws(c, parts + 1, &g.start);
   if (r == ALN_OK) r = ws(c, parts + 1, &g.work);
@@ -1069,10 +1091,10 @@ static int gb_parts(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int *cnt,
                      (uint64_t)g.ncodes, (uint32_t *)nullptr);
   {
     ProfScope p(c, "groupby_move");
-    hipLaunchKernelGGL(k_gp_count, dim3(g.nblk), dim3(GP_BLOCK), 0, c->stream, g);
+    hipLaunchKernelGGL(k_gp_count, dim3(g.nsuper), dim3(GP_BLOCK), 0, c->stream, g);
     hipLaunchKernelGGL(k_gp_rows, dim3(parts), dim3(256), 0, c->stream, g);
     hipLaunchKernelGGL(k_gp_base, dim3(1), dim3(1024), 0, c->stream, g);
-    hipLaunchKernelGGL(k_gp_move, dim3(g.nblk), dim3(GP_BLOCK), 0, c->stream, g);
+    hipLaunchKernelGGL(k_gp_move, dim3(g.ntiles), dim3(GP_BLOCK), 0, c->stream, g);
   }
   {
     ProfScope p(c, "groupby_insert");
