@@ -109,6 +109,7 @@ struct ProfScope {
 };
 
 int check_launch(const char *name);
+int stream_wait(aln_ctx *c);  // until everything enqueued on the context's stream is done
 int copy_to_host(aln_ctx *c, void *h, const void *d, size_t bytes);  // synchronous
 int copy_to_device(aln_ctx *c, void *d, const void *h, size_t bytes);
 

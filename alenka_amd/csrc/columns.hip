@@ -1050,8 +1050,7 @@ int aln_scan_filter(aln_ctx *c, const aln_col *cols, int ncols, uint32_t seg_row
                        seg_rows, s.a.tiles_per_seg, (const uint32_t *)counts, (const uint64_t *)offs, d_row_ids);
   }
   ALN_TRY(check_launch("scan_write"));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  return stream_wait(c);
 }
 
 int aln_row_segments(aln_ctx *c, const uint32_t *d_idx, uint64_t n, const uint32_t *d_rows,

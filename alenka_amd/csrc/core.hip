@@ -142,7 +142,7 @@ static int readback_wait(aln_ctx *c, uint32_t seq, void *h, size_t bytes) {
     }
   }
   std::atomic_thread_fence(std::memory_order_acquire);
-  memcpy(h, c->rb, bytes);
+  if (bytes) memcpy(h, c->rb, bytes);
   return ALN_OK;
 }
 
@@ -152,6 +152,22 @@ static int readback_small(aln_ctx *c, void *h, const void *d, size_t bytes) {
                      (uint32_t)((bytes + 3) / 4), c->rb_dev, c->rb_dev + RB_BYTES / 4, seq);
   ALN_TRY(check_launch("readback"));
   return readback_wait(c, seq, h, bytes);
+}
+
+__global__ void k_flag(DevResult r) { result_done(r); }
+
+// The work enqueued so far is done when a kernel after it has set the flag: the host's wake-up
+// from a stream synchronisation is what this spares (about 8 us a call).
+int stream_wait(aln_ctx *c) {
+  if (!readback_ready(c)) {
+    ALN_HIP(hipStreamSynchronize(c->stream));
+    return ALN_OK;
+  }
+  DevResult r;
+  ALN_TRY(result_open(c, 1, &r));
+  hipLaunchKernelGGL(k_flag, dim3(1), dim3(1), 0, c->stream, r);
+  ALN_TRY(check_launch("wait"));
+  return readback_wait(c, r.seq, nullptr, 0);
 }
 
 int result_open(aln_ctx *c, size_t words, DevResult *r) {

@@ -1188,8 +1188,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     ALN_TRY(check_launch("gb_reduce"));
     hipLaunchKernelGGL(k_gb_reduce_final, dim3(1), dim3(64), 0, c->stream, a, part, nb, o);
     ALN_TRY(check_launch("gb_reduce_final"));
-    ALN_HIP(hipStreamSynchronize(c->stream));
-    return ALN_OK;
+    return stream_wait(c);
   }
   if (total > 63) return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
   // LDS-cached aggregation kernel: at most 2048 blocks, of at least 4 rows per thread (450,000 rows
@@ -1229,8 +1228,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     ALN_TRY(gb_dense_groups(c, a, cnt, gcnt, ncodes, order, o, cap, h_ngroups, &gcode, &gslot));
     g = *h_ngroups;
     if (order != ALN_ORDER_HASH) {
-      ALN_HIP(hipStreamSynchronize(c->stream));
-      return ALN_OK;
+      return stream_wait(c);
     }
   } else {
     // many groups: global atomics (24 G/s) cost more than sorting the rows (12M rows of 12M
@@ -1316,8 +1314,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
                        gcode, gslot, g);
   }
   ALN_TRY(check_launch("gb_emit"));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  return stream_wait(c);
 }
 
 int aln_f64_order_keys(aln_ctx *c, const int64_t *d_in, uint64_t n, int64_t *d_out) {

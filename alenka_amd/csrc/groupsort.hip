@@ -456,16 +456,14 @@ int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int
     const size_t cur = c->cur, off = c->off;
     ALN_TRY(gs_run(c, a, n, total, kmax, true, seed, o, cap, h_ngroups, &clash));
     if (!clash) {
-      ALN_HIP(hipStreamSynchronize(c->stream));
-      return ALN_OK;
+      return stream_wait(c);
     }
     c->cur = cur;
     c->off = off;
   }
   ALN_TRY(gs_run(c, a, n, total, kmax, false, seed, o, cap, h_ngroups, &clash));
   if (order == ALN_ORDER_HASH) ALN_TRY(gs_by_hash(c, a, o, *h_ngroups, seed));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  return stream_wait(c);
 }
 
 }  // namespace aln

@@ -477,8 +477,7 @@ static int join_pairs(aln_ctx *c, uint32_t *d_probe_idx, uint32_t *d_build_idx, 
                          m.toff, d_probe_idx, d_build_idx);
   }
   ALN_TRY(check_launch("join_write"));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  return stream_wait(c);
 }
 
 // The dense path; *taken = false (and nothing else done) when the build keys repeat.
@@ -761,6 +760,5 @@ extern "C" int aln_join_rows(aln_ctx *c, const uint32_t *d_idx, uint64_t nidx, u
   hipLaunchKernelGGL(k_rows_write, dim3((unsigned)nblocks), dim3(JR_BLOCK), 0, c->stream, (const uint32_t *)bm,
                      nrows, anti ? 1 : 0, (const uint64_t *)off, d_rows);
   ALN_TRY(check_launch("join_rows_write"));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  return stream_wait(c);
 }

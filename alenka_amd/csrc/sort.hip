@@ -1640,8 +1640,7 @@ int aln_sort_keys(aln_ctx *c, const int64_t *const *d_keys, const int32_t *desc,
   ALN_REQUIRE(c && d_keys && (n == 0 || d_perm), "aln_sort_keys: bad arguments");
   ws_reset(c);
   ALN_TRY(sort_keys_impl(c, d_keys, desc, nkeys, n, d_perm));
-  ALN_HIP(hipStreamSynchronize(c->stream));
-  return ALN_OK;
+  return stream_wait(c);
 }
 
 int aln_topk(aln_ctx *c, const int64_t *const *d_keys, const int32_t *desc, int nkeys, uint64_t n,
