@@ -126,8 +126,10 @@ __device__ __forceinline__ void vm_binary(int op, int cmp, const int64_t (&l)[U]
 template <int U, typename Load>
 __device__ __forceinline__ void vm_eval(const VProg &p, Load load, int64_t *stk, int64_t (&t)[U]) {
   int sp = 0;  // rows of the LDS stack in use
+  VInsn next = p.ins[0];
   for (int i = 0; i < p.n; ++i) {
-    const VInsn &in = p.ins[i];
+    const VInsn in = next;  // the one after it is fetched while this one runs
+    next = p.ins[i + 1 < p.n ? i + 1 : i];
     switch (in.kind) {
       case V_COL:
       case V_CONST: {
