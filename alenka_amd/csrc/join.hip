@@ -644,31 +644,69 @@ namespace aln {
 // thread per 32-row word, 8192 rows per block.
 constexpr int JR_BLOCK = 256;
 
-// Each thread takes 8 consecutive indices: a join's pairs come in probe-row order, so they
-// are mostly rows of one bitmap word, ORed locally and set with one atomic per word.
+// A block takes 2048 consecutive indices.  A join's pairs come in probe-row order, so they mostly
+// fall into few words of the bitmap: those are ORed in an LDS window and reach the bitmap with
+// one atomic per word, side by side (9.6M pairs: 49 us with an atomic per word and thread, at
+// 24 G/s, 21 us now).  Indices spread wider set their bits directly, a thread merging its own.
+constexpr uint32_t JR_WINDOW = 2048;  // words
 __global__ void __launch_bounds__(256) k_rows_mark(const uint32_t *__restrict__ idx, uint64_t n,
                                                    uint64_t nrows, uint32_t *bm) {
-  const uint64_t nchunks = (n + 7) / 8;
-  for (uint64_t t = (uint64_t)blockIdx.x * 256 + threadIdx.x; t < nchunks; t += (uint64_t)gridDim.x * 256) {
-    uint32_t r[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const uint64_t i = t * 8 + u;
-      r[u] = 0xFFFFFFFFu;
-      if (i < n) r[u] = idx[i];
+  __shared__ uint32_t win[JR_WINDOW];
+  __shared__ uint32_t s_lo, s_hi;
+  for (uint64_t b0 = (uint64_t)blockIdx.x * 2048; b0 < n; b0 += (uint64_t)gridDim.x * 2048) {
+    if (threadIdx.x == 0) {
+      s_lo = 0xFFFFFFFFu;
+      s_hi = 0;
     }
-    uint32_t cw = 0xFFFFFFFFu, cb = 0;
+    uint32_t r[8], lo = 0xFFFFFFFFu, hi = 0;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      if (r[u] >= nrows) continue;  // past the end, or not a row
+      const uint64_t i = b0 + threadIdx.x * 8 + u;
+      r[u] = i < n ? idx[i] : 0xFFFFFFFFu;
+      if (r[u] < nrows) {  // (nrows < 2^32 - 1: past the end, or not a row, is larger)
+        lo = min(lo, r[u]);
+        hi = max(hi, r[u]);
+      }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+      lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 64));
+      hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 64));
+    }
+    __syncthreads();
+    if (__lane_id() == 0 && lo <= hi) {
+      atomicMin(&s_lo, lo);
+      atomicMax(&s_hi, hi);
+    }
+    __syncthreads();
+    const uint32_t wlo = s_lo >> 5, whi = s_hi >> 5;
+    const bool any = s_lo != 0xFFFFFFFFu || s_hi != 0;
+    const bool window = any && whi - wlo < JR_WINDOW;  // (uniform)
+    const uint32_t span = window ? whi - wlo + 1 : 0;
+    for (uint32_t w = threadIdx.x; w < span; w += 256) win[w] = 0;
+    __syncthreads();
+    uint32_t cw = 0xFFFFFFFFu, cb = 0;
+    auto flush = [&]() {
+      if (!cb) return;
+      if (window)
+        atomicOr(&win[cw - wlo], cb);
+      else
+        atomicOr(&bm[cw], cb);
+    };
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      if (r[u] >= nrows) continue;
       if ((r[u] >> 5) != cw) {
-        if (cb) atomicOr(&bm[cw], cb);
+        flush();
         cw = r[u] >> 5;
         cb = 0;
       }
       cb |= 1u << (r[u] & 31);
     }
-    if (cb) atomicOr(&bm[cw], cb);
+    flush();
+    __syncthreads();
+    for (uint32_t w = threadIdx.x; w < span; w += 256)
+      if (win[w]) atomicOr(&bm[wlo + w], win[w]);
+    __syncthreads();
   }
 }
 
@@ -704,7 +742,7 @@ __global__ void __launch_bounds__(JR_BLOCK) k_rows_write(const uint32_t *__restr
                                                          uint32_t *__restrict__ out) {
   __shared__ uint32_t wsum[JR_BLOCK / 64];
   const uint64_t w = (uint64_t)blockIdx.x * JR_BLOCK + threadIdx.x;
-  uint32_t x = kept_rows(bm, w, nrows, anti);
+  const uint32_t x = kept_rows(bm, w, nrows, anti);
   const uint32_t n = __popc(x);
   const unsigned lane = __lane_id(), wid = threadIdx.x / 64;
   uint32_t incl = n;
@@ -716,10 +754,16 @@ __global__ void __launch_bounds__(JR_BLOCK) k_rows_write(const uint32_t *__restr
   __syncthreads();
   uint32_t before = 0;
   for (unsigned k = 0; k < wid; ++k) before += wsum[k];
-  uint64_t pos = off[blockIdx.x] + before + incl - n;
-  while (x) {
-    out[pos++] = (uint32_t)((w << 5) + (uint32_t)(__ffs(x) - 1));
-    x &= x - 1;
+  // each wave writes the rows of its 64 words, 64 rows (two words) per store (9.6M marks: 9 us; a
+  // thread writing its own word row by row took 23)
+  uint32_t *dst = out + off[blockIdx.x] + before;
+  const uint32_t excl = incl - n, row0 = (uint32_t)(((uint64_t)blockIdx.x * JR_BLOCK + wid * 64) << 5) + lane;
+#pragma unroll 8
+  for (int k = 0; k < 32; ++k) {
+    const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)x, 2 * k + 1) << 32 |
+                       (uint32_t)__builtin_amdgcn_readlane((int)x, 2 * k);
+    const uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)excl, 2 * k);
+    if (m >> lane & 1) dst[at + below_count(m)] = row0 + 64u * (uint32_t)k;
   }
 }
 
@@ -742,7 +786,7 @@ extern "C" int aln_join_rows(aln_ctx *c, const uint32_t *d_idx, uint64_t nidx, u
   ALN_TRY(ws(c, nblocks, &off));
   ALN_TRY(fill_u32(c, bm, nw, 0));
   if (nidx) {
-    hipLaunchKernelGGL(k_rows_mark, dim3(grid_for((nidx + 7) / 8, 256, 65536)), dim3(256), 0, c->stream, d_idx,
+    hipLaunchKernelGGL(k_rows_mark, dim3(grid_for(nidx, 2048, 65536)), dim3(256), 0, c->stream, d_idx,
                        nidx, nrows, bm);
     ALN_TRY(check_launch("join_rows_mark"));
   }

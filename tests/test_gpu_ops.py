@@ -703,6 +703,27 @@ def test_join_rows(ctx, nrows, nidx):
         assert e.value.code == L.ALN_E_CAPACITY
 
 
+@pytest.mark.parametrize("nrows,nidx", [(1, 1), (8192, 2048), (8193, 2049), (70000, 5000), (1 << 22, 30000)])
+@pytest.mark.parametrize("order", ["sorted", "shuffled", "mixed"])
+def test_join_rows_windows(ctx, nrows, nidx, order):
+    """Row marks through the LDS window (indices in order, duplicates, both ends of the table),
+    directly (indices all over it), and both in one call; entries that are no row are left out."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(nrows + nidx)
+    idx = np.sort(r.integers(0, nrows, nidx)).astype(np.int64)
+    idx[0], idx[-1] = 0, nrows - 1
+    if order == "shuffled":
+        idx = r.permutation(idx)
+    elif order == "mixed" and nidx > 3000:
+        idx[2048:] = r.permutation(idx[2048:])
+        idx[100:110] = nrows  # not a row
+    t = torch.as_tensor(idx.astype(np.uint32).view(np.int32)).to(ctx.device)
+    semi = np.unique(idx[idx < nrows])
+    assert np.array_equal(host(D.join_rows(ctx, t, nrows, False)), semi)
+    assert np.array_equal(host(D.join_rows(ctx, t, nrows, True)), np.setdiff1d(np.arange(nrows), semi))
+
+
 # ---- sort / top-k ------------------------------------------------------------------------
 @pytest.mark.parametrize("wide", [False, True])
 def test_sort_and_topk(ctx, wide):
