@@ -447,10 +447,13 @@ constexpr uint32_t GP_LOW = 3;
 constexpr int GP_BLOCK = 512;
 constexpr int GP_ITEMS = 8;
 constexpr uint32_t GP_TILE = GP_BLOCK * GP_ITEMS;
-constexpr uint32_t GP_PARTS_MIN = 64, GP_PARTS_MAX = 2048;
+constexpr uint32_t GP_PARTS_MIN = 64, GP_PARTS_FEW = 256, GP_PARTS_MAX = 2048;
 constexpr uint32_t GP_SUB = 8;           // tiles a count block counts
 constexpr uint32_t GP_XCDS = 8;
-constexpr uint64_t GP_ROWS_MIN = 1ull << 20;
+constexpr uint64_t GP_ROWS_MIN = 3ull << 16;
+// (fewer rows: the atomics of k_gb_agg, in one launch instead of five.  150000 rows: 78 and 92 us
+// uniform and Zipf against 77 and 98; 250000: 87 and 104 against 78 and 84; 1M: 152 and 219
+// against 85 and 89.)
 constexpr uint64_t GP_BYTES_MAX = 16ull << 30;  // moved rows
 constexpr size_t GP_LDS = 65536, GP_LDS_MAX = 131072;
 
@@ -463,7 +466,7 @@ struct GpArgs {
   int32_t col_of[ALN_MAX_AGGS + 1];
   uint32_t *code;          // moved codes
   uint64_t n;
-  uint32_t ntiles, nsuper, lp, ncodes, chunk;  // nsuper: count blocks, of GP_SUB tiles
+  uint32_t ntiles, nsub, nsuper, lp, ncodes, chunk;  // nsuper: count blocks, of nsub tiles
   uint32_t *cnts, *excl, *tot;   // [part][count block], [count block][part], [part]
   uint16_t *sub;                 // [tile][part]: the part's rows in the count block's earlier tiles
   uint32_t *start, *work;        // [parts + 1]: first row, first work item of a part
@@ -497,8 +500,8 @@ __global__ void __launch_bounds__(GP_BLOCK) k_gp_count(GpArgs a) {
   uint32_t run[PER];  // of parts thread, thread + GP_BLOCK, ..
 #pragma unroll
   for (uint32_t q = 0; q < PER; ++q) run[q] = 0;
-  for (uint32_t s = 0; s < GP_SUB; ++s) {
-    const uint64_t tile = (uint64_t)blockIdx.x * GP_SUB + s, i0 = tile * GP_TILE;
+  for (uint32_t s = 0; s < a.nsub; ++s) {
+    const uint64_t tile = (uint64_t)blockIdx.x * a.nsub + s, i0 = tile * GP_TILE;
     if (i0 >= a.n) break;
 #pragma unroll
     for (uint32_t q = 0; q < PER; ++q) h[threadIdx.x + GP_BLOCK * q] = 0;
@@ -615,7 +618,7 @@ __global__ void __launch_bounds__(GP_BLOCK) k_gp_move(GpArgs a) {
 #pragma unroll
   for (uint32_t q = 0; q < PER; ++q) {  // the tile's first positions in parts t, t + GP_BLOCK, ..
     const uint32_t p = t + GP_BLOCK * q;
-    off[q] = p < parts ? a.start[p] + a.excl[(uint64_t)(tile / GP_SUB) * parts + p] + a.sub[(uint64_t)tile * parts + p]
+    off[q] = p < parts ? a.start[p] + a.excl[(uint64_t)(tile / a.nsub) * parts + p] + a.sub[(uint64_t)tile * parts + p]
                        : 0;
     h[t + GP_BLOCK * q] = 0;
   }
@@ -958,6 +961,10 @@ static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, 
   // as many blocks as the LDS holds on 256 CUs (5 or 2 per CU), fewer for few rows
   uint32_t nb = lds <= GL_COPIES ? 1280 : 512;
   nb = grid_for(n, 256 * GL_U, nb);
+  // a block clears and stores its accumulators, so it has at least as many rows (1M rows, 4096
+  // codes, two aggregates: 111 us with 488 blocks, 78 with 128)
+  const uint64_t most = std::max<uint64_t>(128, n / nacc);
+  if (nb > most) nb = (uint32_t)most;
   if ((uint64_t)nb * nacc > GL_PART) nb = (uint32_t)(GL_PART / nacc);
   int64_t *part, *tab;
   uint32_t *bad;
@@ -1052,18 +1059,24 @@ static int gb_parts(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int *cnt,
     g.cnt = g.g.nv++;
     g.g.aggs[g.cnt] = ALN_AGG_COUNT;
   }
-  // as few parts as leave two blocks per CU their accumulators; beyond 512 parts one block
+  // as few parts as leave two blocks per CU their accumulators (beyond 512 parts one block), but
+  // a block for each CU where the codes allow it (30M rows, 60000 codes: 537 us with 64 parts,
+  // 431 with 256)
   const uint64_t bytes = 8ull * g.ncodes * g.g.nv;
   uint32_t parts = GP_PARTS_MIN;
+  while (parts < GP_PARTS_FEW && parts < g.ncodes >> GP_LOW) parts *= 2;
   while (parts < 512 && bytes / parts > GP_LDS) parts *= 2;
   while (parts < GP_PARTS_MAX && bytes / parts > GP_LDS_MAX) parts *= 2;
   if (bytes / parts > GP_LDS_MAX || parts > g.ncodes >> GP_LOW) return ALN_OK;
   g.lp = 31 - __builtin_clz(parts);
   if (n * (4 + 8ull * g.ncol) > GP_BYTES_MAX) return ALN_OK;
   g.ntiles = (uint32_t)((n + GP_TILE - 1) / GP_TILE);
-  g.nsuper = (g.ntiles + GP_SUB - 1) / GP_SUB;
-  const uint64_t chunk = 2 * n / parts;
-  g.chunk = (uint32_t)(chunk < 32768 ? 32768 : chunk);
+  g.nsub = g.ntiles < 256 * GP_SUB ? 1 : GP_SUB;  // (fewer tiles: a block each, to fill the chip)
+  g.nsuper = (g.ntiles + g.nsub - 1) / g.nsub;
+  // a part of even shares stays whole, the part of a hot key is split among blocks (30M Zipf
+  // keys: 507 us with chunks of 2n / parts and at least 32768 rows, 446 now)
+  const uint64_t chunk = 5 * n / (4 * parts);
+  g.chunk = (uint32_t)(chunk < 8192 ? 8192 : chunk);
   const size_t cur = c->cur, off = c->off;
   int r = ws(c, n, &g.code);
   for (int k = 0; k < g.ncol && r == ALN_OK; ++k) r = ws(c, n, &g.moved[k]);

@@ -439,11 +439,12 @@ def test_groupby_few_groups(ctx, n, widths):
         assert e.value.code == L.ALN_E_CAPACITY
 
 
-@pytest.mark.parametrize("n", [1 << 20, (1 << 20) + 4097])
-@pytest.mark.parametrize("case", ["2keys", "wide", "skewed", "hot", "edge"])
+@pytest.mark.parametrize("n,case", [(n, c) for n in (196607, 196608, 1 << 20, (1 << 20) + 4097)
+                                    for c in ("2keys", "wide", "skewed", "hot", "edge")]
+                         + [(2047 * 4096, "2keys"), (2047 * 4096 + 1, "hot")])
 def test_groupby_parts(ctx, n, case):
-    """Rows moved into parts of the code range (from 2^20 rows on): a few thousand codes of two
-    keys, 2^21 codes, a skewed column (parts of several blocks), one key almost everywhere, and
+    """Rows moved into parts of the code range (from 196608 rows on; from 2048 tiles of 4096 rows on
+    eight tiles are counted per block): a few thousand codes of two keys, 2^21 codes, a skewed column (parts of several blocks), one key almost everywhere, and
     the smallest code range; all aggregates over one and several value columns, with and without
     a COUNT, in both orders."""
     from alenka_amd import device as D
