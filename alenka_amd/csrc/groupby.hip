@@ -41,9 +41,9 @@ constexpr uint32_t GB_DENSE_BITS = 26;
 // aggregated again in a table of 2n slots.
 constexpr uint64_t GB_HASH_START = 1ull << 20;
 constexpr uint64_t GB_FIRST_PROBES = 64;
-// Rows from which wide codes of many groups are sorted instead (fewer sort in eight passes of
-// their own launches, which the hash table's atomics still beat).
-constexpr uint64_t GB_SORT_MIN = 1ull << 20;
+// Rows from which wide codes of many groups may be sorted instead, and from which a sample of
+// 8192 rows is taken instead of 2048.
+constexpr uint64_t GB_SORT_MIN = 1ull << 17, GB_SORT_LOW = 1ull << 20;
 
 __global__ void __launch_bounds__(256) k_gb_init(uint64_t *tkey, GbArgs a, uint64_t cap) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < cap;
@@ -402,27 +402,31 @@ __global__ void __launch_bounds__(1024) k_gl_sample(GbArgs a, uint64_t n, DevRes
   if (threadIdx.x == 0) result_done(r);
 }
 
-// Distinct key codes among GB_SAMPLE rows spread over the table (n >= GB_SAMPLE), by 32-bit
-// fingerprints in an LDS set, one block.
-constexpr uint32_t GB_SAMPLE = 8192;
+// Distinct key codes among 1024 J rows spread over the table (n >= 1024 J), by 32-bit
+// fingerprints in an LDS set, one block: latency only, so all rows are read at once.
+template <int J>
 __global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevResult r) {
-  __shared__ uint32_t set[2 * GB_SAMPLE];
+  constexpr uint32_t SET = 2048 * J;
+  __shared__ uint32_t set[SET];
   __shared__ uint32_t found;
-  for (uint32_t i = threadIdx.x; i < 2 * GB_SAMPLE; i += 1024) set[i] = 0;
+  const uint64_t step = (n - 1024) / (J - 1);
+  uint64_t code[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) code[j] = gb_code(a, step * j + threadIdx.x);
+  for (uint32_t i = threadIdx.x; i < SET; i += 1024) set[i] = 0;
   if (threadIdx.x == 0) found = 0;
   __syncthreads();
-  const uint64_t step = (n - 1024) / 7;
   uint32_t mine = 0;
-#pragma unroll 1
-  for (uint32_t j = 0; j < GB_SAMPLE / 1024; ++j) {
-    const uint64_t h = murmur64a_u64(gb_code(a, step * j + threadIdx.x), 0x9747b28cu);
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const uint64_t h = murmur64a_u64(code[j], 0x9747b28cu);
     const uint32_t f = (uint32_t)(h >> 32) | 1u;
-    uint32_t at = (uint32_t)h & (2 * GB_SAMPLE - 1);
+    uint32_t at = (uint32_t)h & (SET - 1);
     while (true) {  // at most half full
       const uint32_t old = atomicCAS(&set[at], 0u, f);
       mine += old == 0;
       if (old == 0 || old == f) break;
-      at = (at + 1) & (2 * GB_SAMPLE - 1);
+      at = (at + 1) & (SET - 1);
     }
   }
   atomicAdd(&found, mine);
@@ -1207,7 +1211,11 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   // LDS-cached aggregation kernel: at most 2048 blocks, of at least 4 rows per thread (450,000 rows
   // into 200,000 groups: 119 us in 55 blocks of 32 rows per thread, 50 us)
   const size_t lds = gb_lds_bytes(nvals);
+  // (wide keys: every block adds its LDS table to the global one, up to 1024 groups of it.  1.1M
+  // rows, 600 and 1500 groups: 297 and 403 us with 1024 blocks, 253 and 340 with 256; 12M rows:
+  // 748 and 978 with 256 blocks, 522 and 1000 with 512)
   const uint32_t nb = grid_for(n, 256 * 4, 2048);
+  const uint32_t nbh = std::min<uint32_t>(nb, n >> 12 < 256 ? 256 : n >> 12 < 512 ? n >> 12 : 512);
   if (lds > 65536) {
     ALN_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_gb_agg<true>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1244,16 +1252,25 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
       return stream_wait(c);
     }
   } else {
-    // many groups: global atomics (24 G/s) cost more than sorting the rows (12M rows of 12M
-    // groups: 1.1 against 12 ms, by a 6M-row call of 8.6 ms).  Half of a sample distinct means some 5000 groups or more.
+    // many groups: global atomics (24 G/s) cost more than sorting the rows (12M rows of 12M groups:
+    // 12 against 1.0 ms; 2.5M rows of 1500 groups 416 us against 520, of 2500 groups 579 against
+    // 412).  1900 of 8192 rows distinct means some 2000 groups or more.  Fewer rows are worth
+    // sorting for more groups, 25000 at 250000 rows and 6500 at 1M, as told by the repeats among
+    // 2048 rows (150000 rows, 10000 groups 215 us and sorted 252, 60000 groups 260 and 232; 450000
+    // rows, 10000 groups 276 and 284, 25000 groups 296 and 261; 1M rows, 10000 groups 379 and 304).
     if (n >= GB_SORT_MIN) {
       DevResult r;
       uint64_t found = 0;
+      const bool low = n >= GB_SORT_LOW;
       ALN_TRY(result_open(c, 1, &r));
-      hipLaunchKernelGGL(k_gb_distinct, dim3(1), dim3(1024), 0, c->stream, a, n, r);
+      if (low)
+        hipLaunchKernelGGL(k_gb_distinct<8>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
+      else
+        hipLaunchKernelGGL(k_gb_distinct<2>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
       ALN_TRY(check_launch("gb_distinct"));
       ALN_TRY(result_wait(c, r, &found, 8));
-      if (2 * found >= GB_SAMPLE) return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
+      if (low ? found >= 1900 : 2048 - found <= 2048 / 24 * std::max<uint64_t>(1, n >> 18))
+        return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
     }
     // open addressing: first a table for up to GB_HASH_START keys (half full at most); more
     // keys than that set the overflow flag and the rows are aggregated again in a table of
@@ -1274,7 +1291,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
       ALN_TRY(check_launch("gb_init"));
       {
         ProfScope p(c, "groupby_insert");
-        hipLaunchKernelGGL(k_gb_agg<false>, dim3(nb), dim3(256), lds, c->stream, a, n, tkey, tcap,
+        hipLaunchKernelGGL(k_gb_agg<false>, dim3(nbh), dim3(256), lds, c->stream, a, n, tkey, tcap,
                            (uint32_t *)nullptr, ctl + 1, glimit, ctl);
       }
       ALN_TRY(check_launch("gb_agg"));

@@ -489,12 +489,12 @@ def murmur_unstep(x):
     return (x ^ x >> 47) * inv & M64
 
 
-@pytest.mark.parametrize("n", [1, 64, 65, 1023, 1025, 4096, 5121, 70001, (1 << 20) + 77])
+@pytest.mark.parametrize("n", [1, 64, 65, 1023, 1025, 4096, 5121, 70001, (1 << 17) - 1, 1 << 17, 300007, (1 << 20) + 77])
 @pytest.mark.parametrize("case", ["unique", "pairs", "runs", "one", "wide_values"])
 def test_groupby_sorted(ctx, n, case):
     """GROUP BY by sorting: key tuples of more than 63 bits with every group one row, two rows,
     runs over several 64-row words and 1024-row waves, one group; every aggregate (f64 with NaN),
-    one to eight distinct value columns; key and hash order; and (from 2^20 rows) one key of 40 to
+    one to eight distinct value columns; key and hash order; and (from 2^17 rows) one key of 40 to
     62 bits with many groups, whose rows are sorted instead of hashed."""
     from alenka_amd import device as D
 
@@ -516,7 +516,7 @@ def test_groupby_sorted(ctx, n, case):
         cols = [r.integers(-1000, 1000, n).astype(np.int64) for _ in range(8)]
         _gb_check(ctx, keys, cols, [L.AGG_SUM] * 8)
         _gb_check(ctx, keys, cols[:5], [L.AGG_SUM] * 5, order=L.ORDER_HASH, bounds=bounds)
-    if n >= 1 << 20 and case != "one":
+    if n >= (1 << 17) - 1 and case != "one":
         one = [(gid * 0x1234567 + 5).astype(np.int64)]
         _gb_check(ctx, one, [v, w], [L.AGG_SUM, L.AGG_COUNT])
         _gb_check(ctx, one, [v, w], [L.AGG_SUM, L.AGG_MIN], order=L.ORDER_HASH, bounds=bounds)
