@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(256) k_decode(const uint32_t *__restrict__ wor
 // The rows of an expression or a gather: U rows of a thread, 256 apart, each row's segment by a
 // product with ceil(2^64 / seg_rows) (seg_mul; 0 for one-row segments).  Selected rows ascend,
 // so a wave's rows mostly share a segment: its descriptors are then read once, as scalars
-// (price * (100 - disc) of 30M of 60M rows 461 -> 122 us, 240 MB written and 340 MB read).
+// (price * (100 - disc) of 30M of 60M rows 461 -> 105 us, 240 MB written and 340 MB read).
 struct RowArgs {
   ColTable ct;
   uint32_t nsegs, seg_rows;
@@ -415,9 +415,12 @@ __device__ __forceinline__ void ranges_pass(const RangeSet &rs, const ColTable &
 // One tile of SC_TILE rows per block: its passing rows as one bit per row and their number
 // (OUT SCAN_MASK), the number alone (SCAN_COUNT), or their global row ids (SCAN_WRITE).  Each
 // predicate is decoded and evaluated once, U rows of a thread at a time; the row ids then come
-// from the masks (k_scan_expand).  Bound by the instructions of the decode and of the program:
-// 40M rows of (date < d AND disc != 5) OR price * (100 - disc) > x took two passes of 1.03 ms
-// each with one row per instruction and the predicate evaluated by the count and by the write.
+// from the masks (k_scan_expand).  Bound by a chain of latencies per tile, descriptors, column
+// loads, then the program's instructions one after another (columns staged in LDS, or fewer or
+// more rows at a time, were all slower): 40M rows of (date < d AND disc != 5) OR
+// price * (100 - disc) > x took two passes of 1.03 ms each with one row per instruction and the
+// predicate evaluated by the count and by the write, 186 + 25 us now; 60M rows of one interval
+// 62 + 35 us.
 enum { SCAN_MASK = 0, SCAN_COUNT = 1, SCAN_WRITE = 2 };
 template <int OUT, int U, typename Pred>
 __device__ __forceinline__ void scan_tile(const ScanArgs &a, uint64_t *__restrict__ masks,

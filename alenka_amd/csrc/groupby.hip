@@ -43,7 +43,7 @@ constexpr uint64_t GB_HASH_START = 1ull << 20;
 constexpr uint64_t GB_FIRST_PROBES = 64;
 // Rows from which wide codes of many groups may be sorted instead, and from which a sample of
 // 8192 rows is taken instead of 2048.
-constexpr uint64_t GB_SORT_MIN = 1ull << 17, GB_SORT_LOW = 1ull << 20;
+constexpr uint64_t GB_SORT_MIN = 1ull << 17, GB_SORT_LARGE = 1ull << 20;
 
 __global__ void __launch_bounds__(256) k_gb_init(uint64_t *tkey, GbArgs a, uint64_t cap) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < cap;
@@ -402,23 +402,26 @@ __global__ void __launch_bounds__(1024) k_gl_sample(GbArgs a, uint64_t n, DevRes
   if (threadIdx.x == 0) result_done(r);
 }
 
-// Distinct key codes among 1024 J rows spread over the table (n >= 1024 J), by 32-bit
-// fingerprints in an LDS set, one block: latency only, so all rows are read at once.
+// Distinct key codes among 1024 J rows, 16 J spread runs of 64 (n >= 1024 J), by 32-bit
+// fingerprints in an LDS set, and the rows whose code is that of the row before in their run; one
+// block: latency only, so all rows are read at once.
 template <int J>
 __global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevResult r) {
   constexpr uint32_t SET = 2048 * J;
   __shared__ uint32_t set[SET];
-  __shared__ uint32_t found;
-  const uint64_t step = (n - 1024) / (J - 1);
+  __shared__ uint32_t found, equal;
+  const uint64_t step = (n - 64) / (16 * J - 1);
   uint64_t code[J];
 #pragma unroll
-  for (int j = 0; j < J; ++j) code[j] = gb_code(a, step * j + threadIdx.x);
+  for (int j = 0; j < J; ++j) code[j] = gb_code(a, step * (16 * j + threadIdx.x / 64) + __lane_id());
   for (uint32_t i = threadIdx.x; i < SET; i += 1024) set[i] = 0;
-  if (threadIdx.x == 0) found = 0;
+  if (threadIdx.x == 0) found = equal = 0;
   __syncthreads();
-  uint32_t mine = 0;
+  uint32_t mine = 0, same = 0;
 #pragma unroll
   for (int j = 0; j < J; ++j) {
+    const uint64_t above = __shfl_up(code[j], 1, 64);
+    same += __lane_id() > 0 && above == code[j];
     const uint64_t h = murmur64a_u64(code[j], 0x9747b28cu);
     const uint32_t f = (uint32_t)(h >> 32) | 1u;
     uint32_t at = (uint32_t)h & (SET - 1);
@@ -430,9 +433,11 @@ __global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevR
     }
   }
   atomicAdd(&found, mine);
+  atomicAdd(&equal, same);
   __syncthreads();
   if (threadIdx.x == 0) {
     r.dst[0] = found;
+    r.dst[1] = equal;
     result_done(r);
   }
 }
@@ -446,7 +451,8 @@ __global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevR
 // that the table is written in whole 64-byte sectors; low in the code, they spread the hot keys
 // of a skewed column (small codes, mostly) over the parts.  A part of more than `chunk` rows is
 // added up by several blocks, which then add into the table with atomics.
-// Bounded by the moves: the key twice, each value column read, written and read again.
+// Bounded by the moves: the key twice, each value column read, written and read again (30M rows
+// of one key and one value column: count 62, move 163, add up 124 us).
 constexpr uint32_t GP_LOW = 3;
 constexpr int GP_BLOCK = 512;
 constexpr int GP_ITEMS = 8;
@@ -454,10 +460,10 @@ constexpr uint32_t GP_TILE = GP_BLOCK * GP_ITEMS;
 constexpr uint32_t GP_PARTS_MIN = 64, GP_PARTS_FEW = 256, GP_PARTS_MAX = 2048;
 constexpr uint32_t GP_SUB = 8;           // tiles a count block counts
 constexpr uint32_t GP_XCDS = 8;
+// Fewer rows go through the atomics of k_gb_agg, in one launch instead of five (60000 codes,
+// uniform and Zipf: 150000 rows 78 and 92 us against 77 and 98 in parts; 250000 rows 87 and 104
+// against 78 and 84; 1M rows 152 and 219 against 85 and 89).
 constexpr uint64_t GP_ROWS_MIN = 3ull << 16;
-// (fewer rows: the atomics of k_gb_agg, in one launch instead of five.  150000 rows: 78 and 92 us
-// uniform and Zipf against 77 and 98; 250000: 87 and 104 against 78 and 84; 1M: 152 and 219
-// against 85 and 89.)
 constexpr uint64_t GP_BYTES_MAX = 16ull << 30;  // moved rows
 constexpr size_t GP_LDS = 65536, GP_LDS_MAX = 131072;
 
@@ -1215,7 +1221,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   // rows, 600 and 1500 groups: 297 and 403 us with 1024 blocks, 253 and 340 with 256; 12M rows:
   // 748 and 978 with 256 blocks, 522 and 1000 with 512)
   const uint32_t nb = grid_for(n, 256 * 4, 2048);
-  const uint32_t nbh = std::min<uint32_t>(nb, n >> 12 < 256 ? 256 : n >> 12 < 512 ? n >> 12 : 512);
+  uint32_t nbh = std::min<uint32_t>(nb, n >> 12 < 256 ? 256 : n >> 12 < 512 ? n >> 12 : 512);
   if (lds > 65536) {
     ALN_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_gb_agg<true>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1260,16 +1266,26 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     // rows, 10000 groups 276 and 284, 25000 groups 296 and 261; 1M rows, 10000 groups 379 and 304).
     if (n >= GB_SORT_MIN) {
       DevResult r;
-      uint64_t found = 0;
-      const bool low = n >= GB_SORT_LOW;
-      ALN_TRY(result_open(c, 1, &r));
-      if (low)
+      uint64_t h[2] = {0, 0};
+      bool many = false;
+      const bool large = n >= GB_SORT_LARGE;
+      ALN_TRY(result_open(c, 2, &r));
+      if (large)
         hipLaunchKernelGGL(k_gb_distinct<8>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
       else
         hipLaunchKernelGGL(k_gb_distinct<2>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
       ALN_TRY(check_launch("gb_distinct"));
-      ALN_TRY(result_wait(c, r, &found, 8));
-      if (low ? found >= 1900 : 2048 - found <= 2048 / 24 * std::max<uint64_t>(1, n >> 18))
+      ALN_TRY(result_wait(c, r, h, 16));
+      const uint64_t found = h[0], pairs = large ? 128 * 63 : 32 * 63, starts = pairs - h[1];
+      // rows in the order of their keys, or clustered: a wave's atomics are few, and so are the
+      // distinct codes of the sample.  Runs of 1000 rows leave a block little but to read (12M rows
+      // of 4000 groups: 742 us with 512 blocks, 604 with 2048); more groups than the first table
+      // holds are sorted (12M sorted rows of 1M groups: 3.7 ms in two tables, 0.83 sorted).
+      const bool clustered = 2 * h[1] > pairs;
+      if (clustered && n / pairs * starts > GB_HASH_START / 2) many = true;
+      if (clustered && starts <= pairs / 512) nbh = nb;
+      if (large ? found >= 1900 : 2048 - found <= 2048 / 24 * std::max<uint64_t>(1, n >> 18)) many = true;
+      if (many)
         return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
     }
     // open addressing: first a table for up to GB_HASH_START keys (half full at most); more

@@ -11,7 +11,7 @@
 //     runs that cross waves are combined with atomics.
 // Two tuples of one hash would be neighbours with equal codes: the reduction compares their keys,
 // and the call starts again in key order with a sort of the groups by hash.
-// 12M rows of 12M groups of two sparse keys, three aggregates, hash order: 5.50 -> 1.10 ms
+// 12M rows of 12M groups of two sparse keys, three aggregates, hash order: 5.50 -> 0.96 ms
 // (two sorts of all rows, a gather per column, atomics per row and value, a permutation per
 // output before).
 #include <string.h>

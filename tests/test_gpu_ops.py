@@ -489,6 +489,17 @@ def murmur_unstep(x):
     return (x ^ x >> 47) * inv & M64
 
 
+@pytest.mark.parametrize("n,run", [(1 << 17, 2), (300007, 40), (1 << 20, 3), (1_800_001, 3), (1_800_001, 1200)])
+def test_groupby_clustered(ctx, n, run):
+    """Wide keys whose rows come in runs: few and many groups, and (600001 groups) more than the
+    first hash table takes."""
+    r = np.random.default_rng(n + run)
+    keys = [np.arange(n, dtype=np.int64) // run * 0x1234567ABCD1 - (1 << 61)]
+    v = r.integers(-(1 << 40), 1 << 40, n).astype(np.int64)
+    _gb_check(ctx, keys, [v, v], [L.AGG_SUM, L.AGG_COUNT])
+    _gb_check(ctx, keys, [v], [L.AGG_MAX], order=L.ORDER_HASH, bounds=[0, n // 2, n])
+
+
 @pytest.mark.parametrize("n", [1, 64, 65, 1023, 1025, 4096, 5121, 70001, (1 << 17) - 1, 1 << 17, 300007, (1 << 20) + 77])
 @pytest.mark.parametrize("case", ["unique", "pairs", "runs", "one", "wide_values"])
 def test_groupby_sorted(ctx, n, case):
