@@ -944,7 +944,7 @@ static uint32_t gb_layout(GbArgs &a, const int64_t *mn, const int64_t *mx) {
 }
 
 // The few-groups path for codes of `total` bits, if all accumulators fit in LDS: *taken, and
-// *outside when a key lay outside the layout (nothing is valid then).  With order KEYS or NONE
+// *outside when a key lay outside the layout (nothing is valid then, and a and *cnt are as before).  With order KEYS or NONE
 // the groups are written out and *done is set; else the tables stand in a.tab (a.tab[*cnt] the
 // row counts).
 static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, const GbOut &o, uint64_t cap,
@@ -1008,6 +1008,7 @@ static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, 
   uint32_t hb = 0;
   ALN_TRY(copy_to_host(c, &hb, bad, 4));
   *outside = hb != 0;
+  if (*outside) return ALN_OK;
   for (int v = 0; v < l.g.nv; ++v) a.tab[v] = l.g.tab[v];
   *cnt = l.cnt;
   return ALN_OK;

@@ -473,6 +473,26 @@ def test_groupby_parts(ctx, n, case):
         assert np.array_equal(host(got).view(np.float64), want)
 
 
+@pytest.mark.parametrize("n,outlier,nv", [((1 << 21) + 4099, (1 << 22) - 1, 8), ((1 << 20) + 5, 1 << 20, 2),
+                                          ((1 << 20) + 5, 1 << 27, 2), ((1 << 20) + 5, 1 << 62, 2), ((1 << 20) + 5, 900, 2)])
+@pytest.mark.parametrize("order", [L.ORDER_KEYS, L.ORDER_HASH])
+def test_groupby_sample_missed(ctx, n, outlier, nv, order):
+    """A key that the sample of a few-groups call misses, in each route the call then starts again
+    with: direct-indexed tables with atomics (2^22 codes of eight accumulators and the row count are
+    too many for parts), parts, the hash table (codes over 2^26 or 2n), sorting (tuples over 63
+    bits) and accumulators in LDS again; without a COUNT among the aggregates, whose table would
+    tell the groups, and with one."""
+    r = np.random.default_rng(n + outlier % 1000)
+    for keys in ([r.integers(0, 200, n)], [r.integers(0, 4, n), r.integers(0, 3, n)]):
+        keys = [k.astype(np.int64) for k in keys]
+        keys[0][[12345, n - 20000]] = outlier, outlier - 1  # in none of the sampled runs
+        cols = [r.integers(-(1 << 40), 1 << 40, n).astype(np.int64) for _ in range(nv)]
+        bounds = [0, n // 2, n] if order == L.ORDER_HASH else None
+        _gb_check(ctx, keys, cols, [L.AGG_SUM, L.AGG_MIN, L.AGG_MAX, L.AGG_SUM] * (nv // 4) or [L.AGG_SUM, L.AGG_MIN],
+                  order=order, bounds=bounds)
+        _gb_check(ctx, keys, cols[:1] * 2, [L.AGG_SUM, L.AGG_COUNT], order=order, bounds=bounds)
+
+
 M64 = (1 << 64) - 1
 MUR = 0xC6A4A7935BD1E995
 
