@@ -359,6 +359,8 @@ __global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uin
     base += all;
     __syncthreads();
   }
+  __threadfence_system();  // the call returns on the result: every wave's groups are written by then
+  __syncthreads();
   if (threadIdx.x == 0) {
     r.dst[0] = base;
     r.dst[1] = *bad;

@@ -571,6 +571,44 @@ def test_groupby_sorted(ctx, n, case):
             assert e.value.code == L.ALN_E_CAPACITY
 
 
+def test_results_complete_on_return(ctx):
+    """What a call returns is whole for every stream, not only the context's: groups of the
+    few-groups kernels (which hand the host their number themselves) read at once on another
+    stream, and a join counted on one stream whose pairs are written on another."""
+    import ctypes as C
+
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(3)
+    other = torch.cuda.Stream()
+    n = 3000
+    key, v = r.integers(0, 1000, n).astype(np.int64), r.integers(-1000, 1000, n).astype(np.int64)
+    uk, inv = np.unique(key, return_inverse=True)
+    want = [np.bincount(inv, weights=v).astype(np.int64), np.bincount(inv)]
+    build, probe = r.permutation(4000)[:2000].astype(np.int64), r.integers(0, 4000, 50000).astype(np.int64)
+    row = np.full(4000, -1)
+    row[build] = np.arange(2000)
+    dk, dv, db, dp = (dev(ctx, x) for x in (key, v, build, probe))
+    torch.cuda.synchronize()
+    for _ in range(20):
+        (gk,), gv = D.groupby(ctx, [dk], [dv, dv], [L.AGG_SUM, L.AGG_COUNT])
+        with torch.cuda.stream(other):
+            got = [x.clone() for x in (gk, *gv)]
+        cnt = C.c_uint64()
+        L.check(ctx.lib.aln_hash_join_count(ctx.h, D._p(db), 2000, D._p(dp), 50000, C.byref(cnt)))
+        pi, bi = ctx.empty(cnt.value, torch.int32), ctx.empty(cnt.value, torch.int32)
+        L.check(ctx.lib.aln_set_stream(ctx.h, C.c_void_p(other.cuda_stream)))
+        try:
+            L.check(ctx.lib.aln_hash_join_pairs(ctx.h, D._p(pi), D._p(bi), cnt.value, C.byref(cnt)))
+        finally:
+            L.check(ctx.lib.aln_set_stream(ctx.h, C.c_void_p(ctx.stream.cuda_stream)))
+        torch.cuda.synchronize()
+        for x, y in zip(got, [uk] + want):
+            assert np.array_equal(host(x), y)
+        hit = np.nonzero(row[probe] >= 0)[0]
+        assert np.array_equal(host(pi), hit) and np.array_equal(host(bi), row[probe[hit]])
+
+
 def test_groupby_hash_clash(ctx):
     """Key tuples made to share a MurmurHash64A stay groups of their own in hash order: by hash,
     then by key tuple."""
