@@ -333,15 +333,30 @@ __global__ void __launch_bounds__(256) k_gl_sum(GlArgs a, const int64_t *__restr
     a.g.tab[v][s - v * a.ncodes] = ag == ALN_AGG_FMIN || ag == ALN_AGG_FMAX ? f64_unorder_key(r) : r;
 }
 
-// The groups (codes with rows) in code order into the outputs, at most cap of them; the number
-// of groups and whether a key lay outside the code range to the host.
+// The groups (codes with rows) in code order into the outputs; the number of groups and whether a
+// key lay outside the code range to the host.  Nothing is written when one did or there are more
+// groups than cap: the call may start again, from inputs that the outputs may lie over.
 __global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uint64_t cap,
                                                   const uint32_t *__restrict__ bad, DevResult r) {
   __shared__ uint32_t wsum[16];
-  uint64_t base = 0;
+  static_assert(GL_MOST / 8 <= 32 * 1024, "a bit per tile of 1024 codes");
+  const uint32_t miss = *bad;
+  uint32_t mine = 0, n = 0;  // this thread's codes with rows, a bit per tile; the wave's number of them
   for (uint32_t c0 = 0; c0 < a.ncodes; c0 += 1024) {
     const uint32_t c = c0 + threadIdx.x;
     const bool f = c < a.ncodes && a.g.tab[a.cnt][c] != 0;
+    mine |= (f ? 1u : 0u) << (c0 / 1024);
+    n += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(f));
+  }
+  if (__lane_id() == 0) wsum[threadIdx.x / 64] = n;
+  __syncthreads();
+  uint32_t total = 0;
+  for (uint32_t w = 0; w < 16; ++w) total += wsum[w];
+  __syncthreads();
+  uint64_t base = 0;
+  for (uint32_t c0 = 0; c0 < a.ncodes && !miss && total <= cap; c0 += 1024) {
+    const uint32_t c = c0 + threadIdx.x;
+    const bool f = mine >> (c0 / 1024) & 1;
     const uint64_t bal = __builtin_amdgcn_ballot_w64(f);
     if (__lane_id() == 0) wsum[threadIdx.x / 64] = (uint32_t)__popcll(bal);
     __syncthreads();
@@ -351,7 +366,7 @@ __global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uin
       all += wsum[w];
     }
     const uint64_t pos = base + before + below_count(bal);
-    if (f && pos < cap) {
+    if (f) {
       for (int k = 0; k < a.g.nk; ++k)
         o.keys[k][pos] = (int64_t)((uint64_t)a.g.kmin[k] + ((c >> a.g.shift[k]) & a.g.fmask[k]));
       for (int v = 0; v < nv; ++v) o.vals[v][pos] = a.g.tab[v][c];
@@ -362,8 +377,8 @@ __global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uin
   __threadfence_system();  // the call returns on the result: every wave's groups are written by then
   __syncthreads();
   if (threadIdx.x == 0) {
-    r.dst[0] = base;
-    r.dst[1] = *bad;
+    r.dst[0] = total;
+    r.dst[1] = miss;
     result_done(r);
   }
 }
@@ -1016,6 +1031,21 @@ static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, 
   return ALN_OK;
 }
 
+// Whether an output (up to m values are written) lies over an input.
+static bool gb_in_place(const GbArgs &a, uint64_t n, const GbOut &o, uint64_t m) {
+  auto over = [&](const int64_t *in, const int64_t *out) {
+    return in && out && (uintptr_t)out < (uintptr_t)(in + n) && (uintptr_t)in < (uintptr_t)(out + m);
+  };
+  for (int i = 0; i < a.nk + a.nv; ++i) {
+    const int64_t *out = i < a.nk ? o.keys[i] : o.vals[i - a.nk];
+    for (int k = 0; k < a.nk; ++k)
+      if (over(a.keys[k], out)) return true;
+    for (int v = 0; v < a.nv; ++v)
+      if (a.aggs[v] != ALN_AGG_COUNT && over(a.vals[v], out)) return true;
+  }
+  return false;
+}
+
 // The groups of direct-indexed tables in code order (row counts in gcnt, or, gcnt NULL, in
 // a.tab[cv]): written out, or with order HASH their codes and slots.
 static int gb_dense_groups(aln_ctx *c, const GbArgs &a, int cv, const uint32_t *gcnt, uint64_t ncodes, int order,
@@ -1267,7 +1297,8 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     // sorting for more groups, 25000 at 250000 rows and 6500 at 1M, as told by the repeats among
     // 2048 rows (150000 rows, 10000 groups 215 us and sorted 252, 60000 groups 260 and 232; 450000
     // rows, 10000 groups 276 and 284, 25000 groups 296 and 261; 1M rows, 10000 groups 379 and 304).
-    if (n >= GB_SORT_MIN) {
+    // (In place, the tables: they have read every row before a group is written.)
+    if (n >= GB_SORT_MIN && !gb_in_place(a, n, o, std::min(n, cap))) {
       DevResult r;
       uint64_t h[2] = {0, 0};
       bool many = false;

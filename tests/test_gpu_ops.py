@@ -493,6 +493,51 @@ def test_groupby_sample_missed(ctx, n, outlier, nv, order):
         _gb_check(ctx, keys, cols[:1] * 2, [L.AGG_SUM, L.AGG_COUNT], order=order, bounds=bounds)
 
 
+def gb_raw(ctx, keys, vals, aggs, order, outk, outv, cap):
+    """aln_groupby into given output tensors: (status, number of groups)."""
+    import ctypes as C
+
+    p = lambda ts: (C.c_void_p * max(1, len(ts)))(*[t.data_ptr() for t in ts])  # noqa: E731
+    g = C.c_uint64()
+    rc = ctx.lib.aln_groupby(ctx.h, p(keys), len(keys), p(vals), (C.c_int32 * max(1, len(aggs)))(*aggs), len(vals),
+                             keys[0].numel(), order, 100, p(outk), p(outv), cap, C.byref(g))
+    return rc, g.value
+
+
+# sizes, key columns: the routes of key codes of at most 63 bits
+GB_ROUTES = {"few": (5000, lambda r, n: [r.integers(0, 7, n), r.integers(0, 30, n)]),
+             "sampled": ((1 << 20) + 5, lambda r, n: [r.integers(0, 7, n)]),
+             "missed": ((1 << 20) + 5, lambda r, n: [np.where(np.arange(n) == 12345, 5000, r.integers(0, 7, n))]),
+             "direct": (150000, lambda r, n: [r.integers(0, 30000, n)]),
+             "parts": (300000, lambda r, n: [r.integers(0, 30000, n)]),
+             "table": (150000, lambda r, n: [r.integers(0, 300, n) * 1000003]),
+             "sorted": (300007, lambda r, n: [r.integers(0, n // 2, n) * 1000003])}
+
+
+@pytest.mark.parametrize("order", [L.ORDER_KEYS, L.ORDER_HASH])
+@pytest.mark.parametrize("route", GB_ROUTES)
+def test_groupby_in_place_and_short(ctx, route, order):
+    """Outputs that lie over the inputs: every row is read before a group is written, also when the
+    call starts again; and with too short a capacity nothing is written, the number needed is
+    returned, and the inputs are still there for the next call."""
+    n, gen = GB_ROUTES[route]
+    r = np.random.default_rng(n)
+    keys = [k.astype(np.int64) for k in gen(r, n)]
+    v = r.integers(-(1 << 40), 1 << 40, n).astype(np.int64)
+    bounds = [0, n // 2, n] if order == L.ORDER_HASH else None
+    aggs = [L.AGG_SUM, L.AGG_MAX]
+    wk, wv = O.groupby(keys, [v, v], aggs, seg_bounds=bounds, seed=100)
+    g = len(wk[0])
+    dk, dv = [dev(ctx, k) for k in keys], [dev(ctx, v), dev(ctx, v)]
+    for cap in (0, 1, g - 1):
+        assert gb_raw(ctx, dk, dv, aggs, order, dk, dv, cap) == (L.ALN_E_CAPACITY, g)
+        for x, y in zip(dk + dv, keys + [v, v]):
+            assert np.array_equal(host(x), y)
+    assert gb_raw(ctx, dk, dv, aggs, order, dk, dv, g) == (L.ALN_OK, g)
+    for x, y in zip(dk + dv, list(wk) + list(wv)):
+        assert np.array_equal(host(x)[:g], y)
+
+
 M64 = (1 << 64) - 1
 MUR = 0xC6A4A7935BD1E995
 
