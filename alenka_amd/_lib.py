@@ -119,6 +119,7 @@ SIGNATURES = {
     "aln_destroy": (None, [P]),
     "aln_set_stream": (C.c_int, [P, P]),
     "aln_sync": (C.c_int, [P]),
+    "aln_set_workspace_limit": (C.c_int, [P, U64]),
     "aln_profile_enable": (C.c_int, [P, C.c_int]),
     "aln_profile_reset": (C.c_int, [P]),
     "aln_profile_get": (C.c_int, [P, C.c_char_p, C.POINTER(C.c_double), PU64]),

@@ -47,6 +47,7 @@ struct aln_ctx {
   };
   std::vector<Chunk> chunks;
   size_t cur = 0, off = 0;
+  uint64_t ws_limit = 0;  // most bytes the chunks may take together (0: no limit)
   // pinned host staging for readbacks
   void *pinned = nullptr;
   size_t pinned_size = 0;
@@ -90,6 +91,13 @@ namespace aln {
 // Workspace allocation (device, 256-byte aligned) valid until the next ws_reset().
 int ws_alloc(aln_ctx *c, size_t bytes, void **out);
 void ws_reset(aln_ctx *c);
+// Back to an earlier state of the workspace.  `release`: chunks taken since then are given back to
+// the device (a route that ran out of memory leaves them to the next one).
+struct WsMark {
+  size_t cur, off, nchunks;
+};
+inline WsMark ws_mark(const aln_ctx *c) { return {c->cur, c->off, c->chunks.size()}; }
+void ws_rewind(aln_ctx *c, const WsMark &m, bool release = false);
 template <typename T>
 int ws(aln_ctx *c, size_t n, T **out) {
   return ws_alloc(c, n * sizeof(T) + 16, reinterpret_cast<void **>(out));

@@ -46,6 +46,14 @@ int ws_alloc(aln_ctx *c, size_t bytes, void **out) {
   size_t want = bytes;
   if (!c->chunks.empty() && c->chunks.back().size * 2 > want) want = c->chunks.back().size * 2;
   if (want < ((size_t)64 << 20)) want = (size_t)64 << 20;
+  if (c->ws_limit) {
+    uint64_t held = 0;
+    for (const auto &ch : c->chunks) held += ch.size;
+    if (held + bytes > c->ws_limit)
+      return set_error(ALN_E_NOMEM, "workspace of %llu bytes: %zu more would pass its limit of %llu",
+                       (unsigned long long)held, bytes, (unsigned long long)c->ws_limit);
+    if (held + want > c->ws_limit) want = bytes;
+  }
   void *p = nullptr;
   if (hipMalloc(&p, want) != hipSuccess) {
     (void)hipGetLastError();
@@ -66,6 +74,15 @@ void ws_reset(aln_ctx *c) {
   c->join.valid = false;
   c->cur = 0;
   c->off = 0;
+}
+
+void ws_rewind(aln_ctx *c, const WsMark &m, bool release) {
+  c->cur = m.cur;
+  c->off = m.off;
+  while (release && c->chunks.size() > m.nchunks) {
+    (void)hipFree(c->chunks.back().ptr);  // waits for the kernels that use it
+    c->chunks.pop_back();
+  }
 }
 
 int pinned(aln_ctx *c, size_t bytes, void **out) {
@@ -720,6 +737,12 @@ int aln_set_stream(aln_ctx *c, void *stream) {
 int aln_sync(aln_ctx *c) {
   ALN_REQUIRE(c, "aln_sync: ctx is NULL");
   ALN_HIP(hipStreamSynchronize(c->stream));
+  return ALN_OK;
+}
+
+int aln_set_workspace_limit(aln_ctx *c, uint64_t bytes) {
+  ALN_REQUIRE(c, "aln_set_workspace_limit: ctx is NULL");
+  c->ws_limit = bytes;
   return ALN_OK;
 }
 

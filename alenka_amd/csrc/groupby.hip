@@ -1120,8 +1120,11 @@ static int gb_parts(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int *cnt,
   // keys: 507 us with chunks of 2n / parts and at least 32768 rows, 446 now)
   const uint64_t chunk = 5 * n / (4 * parts);
   g.chunk = (uint32_t)(chunk < 8192 ? 8192 : chunk);
-  const size_t cur = c->cur, off = c->off;
-  int r = ws(c, n, &g.code);
+  const WsMark mark = ws_mark(c);
+  int r = ALN_OK;
+  for (int v = 0; v < g.g.nv && r == ALN_OK; ++v) r = ws(c, g.ncodes, &g.g.tab[v]);
+  const WsMark kept = ws_mark(c);  // what follows is free again when the tables are written
+  if (r == ALN_OK) r = ws(c, n, &g.code);
   for (int k = 0; k < g.ncol && r == ALN_OK; ++k) r = ws(c, n, &g.moved[k]);
   if (r == ALN_OK) r = ws(c, (size_t)parts * g.nsuper, &g.cnts);
   if (r == ALN_OK) r = ws(c, (size_t)parts * g.nsuper, &g.excl);
@@ -1129,10 +1132,8 @@ static int gb_parts(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int *cnt,
   if (r == ALN_OK) r = ws(c, parts, &g.tot);
   if (r == ALN_OK) r = ws(c, parts + 1, &g.start);
   if (r == ALN_OK) r = ws(c, parts + 1, &g.work);
-  for (int v = 0; v < g.g.nv && r == ALN_OK; ++v) r = ws(c, g.ncodes, &g.g.tab[v]);
   if (r == ALN_E_NOMEM) {  // the atomics need less
-    c->cur = cur;
-    c->off = off;
+    ws_rewind(c, mark, true);
     return ALN_OK;
   }
   ALN_TRY(r);
@@ -1156,6 +1157,7 @@ static int gb_parts(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int *cnt,
     ProfScope p(c, "groupby_insert");
     hipLaunchKernelGGL(k_gp_agg, dim3(parts + (uint32_t)(n / g.chunk)), dim3(1024), lds, c->stream, g);
   }
+  ws_rewind(c, kept);
   return check_launch("gb_parts");
 }
 
@@ -1319,8 +1321,12 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
       if (clustered && n / pairs * starts > GB_HASH_START / 2) many = true;
       if (clustered && starts <= pairs / 512) nbh = nb;
       if (large ? found >= 1900 : 2048 - found <= 2048 / 24 * std::max<uint64_t>(1, n >> 18)) many = true;
-      if (many)
-        return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
+      if (many) {
+        const WsMark mark = ws_mark(c);
+        const int rc = gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
+        if (rc != ALN_E_NOMEM) return rc;
+        ws_rewind(c, mark, true);  // a table of few enough groups needs less (48 to 85 MB for 2^20)
+      }
     }
     // open addressing: first a table for up to GB_HASH_START keys (half full at most); more
     // keys than that set the overflow flag and the rows are aggregated again in a table of

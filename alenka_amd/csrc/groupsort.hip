@@ -333,9 +333,9 @@ static int gs_by_hash(aln_ctx *c, const GbArgs &a, const GbOut &o, uint64_t g, u
 }
 
 // One sort and reduction.  hashed: by the tuples' hashes (*clash: two tuples share one, and the
-// outputs are void); else in key order.
+// outputs are void); else in key order.  pack: with packed rows.
 static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, const int64_t *kmax, bool hashed,
-                  uint32_t seed, const GbOut &o, uint64_t cap, uint64_t *h_ngroups, bool *clash) {
+                  bool pack, uint32_t seed, const GbOut &o, uint64_t cap, uint64_t *h_ngroups, bool *clash) {
   *clash = false;
   GsArgs a;
   memset(&a, 0, sizeof(a));
@@ -353,7 +353,7 @@ static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, const
     a.col_of[v] = k;
   }
   a.stride = (a.nkw + a.ncol + 1) & ~1;
-  // codes, packed rows (if the workspace has room for them), order
+  // codes, packed rows, order
   const bool coded_sort = hashed || a.coded;
   uint64_t *code = nullptr;
   int64_t *row = nullptr;
@@ -362,17 +362,7 @@ static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, const
   if (coded_sort || a.coded) ALN_TRY(ws(c, n, &code));
   ALN_TRY(ws(c, n, &perm));
   ALN_TRY(ws(c, n, &heads));
-  {
-    const size_t cur = c->cur, off = c->off;
-    const int r = ws(c, n * a.stride, &row);
-    if (r == ALN_E_NOMEM) {
-      row = nullptr;
-      c->cur = cur;
-      c->off = off;
-    } else {
-      ALN_TRY(r);
-    }
-  }
+  if (pack) ALN_TRY(ws(c, n * a.stride, &row));
   const dim3 rows(grid_for(n, GS_BLOCK));
   if (code || row) {
     ProfScope p(c, "groupby_pack");
@@ -449,20 +439,33 @@ static int gs_run(aln_ctx *c, const GbArgs &g, uint64_t n, uint32_t total, const
   return ALN_OK;
 }
 
+// gs_run with packed rows where the workspace holds them beside the sort's buffers (53 bytes a row
+// for one value column), else without (37).
+static int gs_fit(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, bool hashed,
+                  uint32_t seed, const GbOut &o, uint64_t cap, uint64_t *h_ngroups, bool *clash) {
+  const WsMark mark = ws_mark(c);
+  const int r = gs_run(c, a, n, total, kmax, hashed, true, seed, o, cap, h_ngroups, clash);
+  if (r != ALN_E_NOMEM) return r;
+  ws_rewind(c, mark, true);
+  return gs_run(c, a, n, total, kmax, hashed, false, seed, o, cap, h_ngroups, clash);
+}
+
 int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, uint32_t seed,
               const GbOut &o, uint64_t cap, uint64_t *h_ngroups) {
   bool clash = false;
+  const WsMark mark = ws_mark(c);
   if (order == ALN_ORDER_HASH) {
-    const size_t cur = c->cur, off = c->off;
-    ALN_TRY(gs_run(c, a, n, total, kmax, true, seed, o, cap, h_ngroups, &clash));
+    ALN_TRY(gs_fit(c, a, n, total, kmax, true, seed, o, cap, h_ngroups, &clash));
     if (!clash) {
       return stream_wait(c);
     }
-    c->cur = cur;
-    c->off = off;
+    ws_rewind(c, mark);
   }
-  ALN_TRY(gs_run(c, a, n, total, kmax, false, seed, o, cap, h_ngroups, &clash));
-  if (order == ALN_ORDER_HASH) ALN_TRY(gs_by_hash(c, a, o, *h_ngroups, seed));
+  ALN_TRY(gs_fit(c, a, n, total, kmax, false, seed, o, cap, h_ngroups, &clash));
+  if (order == ALN_ORDER_HASH) {
+    ws_rewind(c, mark);  // the groups are in the outputs
+    ALN_TRY(gs_by_hash(c, a, o, *h_ngroups, seed));
+  }
   return stream_wait(c);
 }
 

@@ -54,6 +54,10 @@ int aln_create(int device, void *stream, aln_ctx **out);
 void aln_destroy(aln_ctx *ctx);
 int aln_set_stream(aln_ctx *ctx, void *stream);
 int aln_sync(aln_ctx *ctx);
+/* Most bytes of device memory the context's workspace may take from now on (0, the start: no
+ * limit; what it holds already stays).  A call that needs more takes a route that needs less
+ * where it has one, else returns ALN_E_NOMEM, as when the device's memory runs out. */
+int aln_set_workspace_limit(aln_ctx *ctx, uint64_t bytes);
 /* Per-kernel timing with HIP events recorded on the context stream around every launch
  * (off by default).  aln_profile_get returns the summed milliseconds and launch count of
  * one kernel name since the last aln_profile_reset. */

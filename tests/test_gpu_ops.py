@@ -538,6 +538,46 @@ def test_groupby_in_place_and_short(ctx, route, order):
         assert np.array_equal(host(x)[:g], y)
 
 
+@pytest.mark.parametrize("order", [L.ORDER_KEYS, L.ORDER_HASH])
+@pytest.mark.parametrize("case,n", [("tuples", 300007), ("codes", 3_000_017), ("parts", 400_003)])
+def test_groupby_workspace_limit(ctx, case, n, order):
+    """Routes of less workspace where the first choice does not fit: wide tuples sorted without
+    packed rows (half the bytes), wide codes of many groups in the table instead of sorted, the
+    direct tables without moved rows; the results are the same, and below what any route needs the
+    call fails, and a context that has failed goes on working."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n)
+    keys = {"tuples": lambda: [r.integers(0, n // 3, n) * 0x1234567ABCD1 - (1 << 62),
+                               r.integers(0, 2, n) * ((1 << 62) + 5)],
+            "codes": lambda: [r.integers(0, 30000, n) * 1_000_003],
+            "parts": lambda: [r.integers(0, 60000, n)]}[case]()
+    keys = [k.astype(np.int64) for k in keys]
+    v, w = r.integers(-(1 << 40), 1 << 40, n).astype(np.int64), r.integers(-1000, 1000, n).astype(np.int64)
+    vals, aggs = ([v, v, w, v], AGGS4) if case == "tuples" else ([v, v], [L.AGG_SUM, L.AGG_COUNT])
+    bounds = [0, n // 2, n] if order == L.ORDER_HASH else None
+    # all routes fit (with what the chunks of a small workspace leave unused); the second only
+    full, less = {"tuples": (100 * n, 58 * n), "codes": (80 * n, 110 << 20), "parts": (40 * n, (8 if order == L.ORDER_KEYS else 14) * n)}[case]
+    first, second = {"tuples": (("groupby_pack", 1), ("groupby_sorted_agg", 1)),
+                     "codes": (("groupby_sorted_agg", 1), ("groupby_insert", 1)),
+                     "parts": (("groupby_move", 1), ("groupby_move", 0))}[case]
+    for limit, seen in ((full, first), (less, second)):
+        c = D.Context(0)
+        L.check(c.lib.aln_set_workspace_limit(c.h, limit))
+        c.profile()
+        _gb_check(c, keys, vals, aggs, order=order, bounds=bounds)
+        assert c.profile_get(seen[0])[1] == seen[1], seen
+        c.close()
+    c = D.Context(0)
+    L.check(c.lib.aln_set_workspace_limit(c.h, 1 << 16))
+    with pytest.raises(L.AlnError) as e:
+        _gb_check(c, keys, vals, aggs, order=order, bounds=bounds)
+    assert e.value.code == L.ALN_E_NOMEM
+    L.check(c.lib.aln_set_workspace_limit(c.h, 0))
+    _gb_check(c, keys, vals, aggs, order=order, bounds=bounds)
+    c.close()
+
+
 M64 = (1 << 64) - 1
 MUR = 0xC6A4A7935BD1E995
 
