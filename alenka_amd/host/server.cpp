@@ -112,8 +112,13 @@ double ms_between(Clock::time_point a, Clock::time_point b) {
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Device bytes of a filter + GROUP BY run through the operators: row ids, two evaluated
-// columns, group-by workspace and outputs.
-size_t plain_mem(const Table &t, uint64_t g) { return (size_t)(4 + 8 + 8 + 48) * t.nrows + 24 * g + (16u << 20); }
+// columns, group-by workspace and outputs.  The workspace is the sorted route's, the largest per
+// row: code 8, permutation 4, head flag 1, packed key and value 16, the sort's buffers 24 and its
+// counts (the parts take 12 and at most 32 for their tables).
+constexpr size_t GROUPBY_ROW = 54;
+size_t plain_mem(const Table &t, uint64_t g) {
+  return (4 + 8 + 8 + GROUPBY_ROW) * t.nrows + 24 * g + (16u << 20);
+}
 
 // Device bytes a request holds while it runs (what admission charges against the budget):
 // plain, the operators' bytes; batched, dense group tables + compaction + outputs (a

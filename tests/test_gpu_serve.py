@@ -155,3 +155,43 @@ def test_served_budget_admission(ctx, tables):
         assert srv.stats()["mem_in_use"] == 0
     finally:
         srv.close()
+
+
+def test_served_plain_budget(ctx, tables):
+    """The plain form's charge covers the GROUP BY route that takes most workspace, the sorted one:
+    a budget of 53 bytes a row of it is too small, one of 54 is enough."""
+    from alenka_amd import device as D
+
+    h, cols = tables["flat"]
+    n, g = len(h[0]), int(h[4].max() - h[4].min()) + 1
+    q = dict(pred_col=1, key_col=4, x_col=2, y_col=3, lo=19920101, hi=19981231, key_div=1, **REV)
+    for row, ok in ((53, False), (54, True)):
+        srv = D.Server(streams=1, plain=True, budget_bytes=(20 + row) * n + 24 * g + (16 << 20))
+        try:
+            i = srv.submit(srv.add_table(cols), q)
+            r = srv.wait(i, check=False)
+            assert r.status == (L.ALN_OK if ok else L.ALN_E_NOMEM)
+            if ok:
+                for a, b in zip(srv.fetch(i), want(h, q)):
+                    assert np.array_equal(a, b)
+        finally:
+            srv.close()
+
+
+def test_sorted_route_row_bytes(ctx):
+    """What that charge rests on: the sorted route of one wide key, a SUM and a COUNT runs in 54
+    bytes a row of workspace and a few MB."""
+    from alenka_amd import device as D
+
+    n = 6_000_000
+    key = torch.randint(0, n, (n,), device=ctx.device) * 1_000_003
+    v = torch.ones(n, dtype=torch.int64, device=ctx.device)
+    c = D.Context(0)
+    try:
+        L.check(c.lib.aln_set_workspace_limit(c.h, 54 * n + (4 << 20)))
+        c.profile()
+        k, (s, cnt) = D.groupby(c, [key], [v, v], [L.AGG_SUM, L.AGG_COUNT])
+        assert c.profile_get("groupby_sorted_agg")[1] == 1
+        assert torch.equal(s, cnt) and int(cnt.sum().item()) == n and bool((k[0][1:] > k[0][:-1]).all())
+    finally:
+        c.close()
