@@ -203,10 +203,6 @@ struct DevCols {
   const aln_seg *segs[ALN_MAX_COLS];
   int n;
 };
-struct DevProg {
-  aln_insn ins[ALN_MAX_INSN];
-  int n;
-};
 
 }  // namespace aln
 

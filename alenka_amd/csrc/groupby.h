@@ -60,10 +60,14 @@ __device__ __forceinline__ void agg_atomic(int a, int64_t *t, int64_t x) {
   }
 }
 
+// MurmurHash64A of nk int64 values laid out contiguously (v holds ALN_MAX_KEYS, unrolled so that they
+// stay in registers): the merge order of every route.
 __device__ __forceinline__ uint64_t murmur64a_tuple(const int64_t *v, int nk, uint32_t seed) {
   const uint64_t m = 0xc6a4a7935bd1e995ULL;
   uint64_t h = (uint64_t)seed ^ ((uint64_t)(8 * nk) * m);
-  for (int i = 0; i < nk; ++i) {
+#pragma unroll
+  for (int i = 0; i < ALN_MAX_KEYS; ++i) {
+    if (i >= nk) break;
     uint64_t k = (uint64_t)v[i];
     k *= m;
     k ^= k >> 47;

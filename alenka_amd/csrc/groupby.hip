@@ -902,8 +902,9 @@ __global__ void k_gb_hash(GbArgs a, const uint64_t *gcode, uint64_t g, uint32_t 
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < g;
        i += (uint64_t)gridDim.x * 256) {
     int64_t kv[ALN_MAX_KEYS];
-    for (int k = 0; k < a.nk; ++k)
-      kv[k] = (int64_t)((uint64_t)a.kmin[k] + ((gcode[i] >> a.shift[k]) & a.fmask[k]));
+#pragma unroll
+    for (int k = 0; k < ALN_MAX_KEYS; ++k)
+      kv[k] = k < a.nk ? (int64_t)((uint64_t)a.kmin[k] + ((gcode[i] >> a.shift[k]) & a.fmask[k])) : 0;
     hash[i] = murmur64a_tuple(kv, a.nk, seed);
   }
 }
@@ -932,7 +933,8 @@ __global__ void k_hash_rows(GbArgs a, uint64_t n, uint32_t seed, uint64_t *out) 
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < n;
        i += (uint64_t)gridDim.x * 256) {
     int64_t kv[ALN_MAX_KEYS];
-    for (int k = 0; k < a.nk; ++k) kv[k] = a.keys[k][i];
+#pragma unroll
+    for (int k = 0; k < ALN_MAX_KEYS; ++k) kv[k] = k < a.nk ? a.keys[k][i] : 0;
     out[i] = murmur64a_tuple(kv, a.nk, seed);
   }
 }

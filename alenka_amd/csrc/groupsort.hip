@@ -42,25 +42,6 @@ struct GsArgs {
   uint32_t *clash;
 };
 
-__device__ __forceinline__ uint64_t gs_tuple_hash(const int64_t *v, int nk, uint32_t seed) {
-  const uint64_t m = 0xc6a4a7935bd1e995ULL;
-  uint64_t h = (uint64_t)seed ^ ((uint64_t)(8 * nk) * m);
-#pragma unroll
-  for (int i = 0; i < ALN_MAX_KEYS; ++i) {
-    if (i >= nk) break;
-    uint64_t k = (uint64_t)v[i];
-    k *= m;
-    k ^= k >> 47;
-    k *= m;
-    h ^= k;
-    h *= m;
-  }
-  h ^= h >> 47;
-  h *= m;
-  h ^= h >> 47;
-  return h;
-}
-
 // The code of every row (NULL: not wanted): the tuple's hash, or the packed key code; and the
 // packed rows (NULL: not wanted).
 __global__ void __launch_bounds__(GS_BLOCK) k_gs_pack(GsArgs a, int hashed, uint32_t seed, uint64_t *__restrict__ code,
@@ -74,7 +55,7 @@ __global__ void __launch_bounds__(GS_BLOCK) k_gs_pack(GsArgs a, int hashed, uint
     kv[k] = k < a.g.nk ? __builtin_nontemporal_load(a.g.keys[k] + i) : 0;
     if (k < a.g.nk) packed |= (((uint64_t)kv[k] - (uint64_t)a.g.kmin[k]) & a.g.fmask[k]) << a.g.shift[k];
   }
-  if (code) code[i] = hashed ? gs_tuple_hash(kv, a.g.nk, seed) : packed;
+  if (code) code[i] = hashed ? murmur64a_tuple(kv, a.g.nk, seed) : packed;
   if (!row) return;
   int64_t w[GS_MAX_WORDS];
 #pragma unroll
@@ -300,7 +281,7 @@ __global__ void __launch_bounds__(GS_BLOCK) k_gs_group_hash(GbOut o, int nk, uin
   int64_t kv[ALN_MAX_KEYS];
 #pragma unroll
   for (int k = 0; k < ALN_MAX_KEYS; ++k) kv[k] = k < nk ? o.keys[k][i] : 0;
-  hash[i] = gs_tuple_hash(kv, nk, seed);
+  hash[i] = murmur64a_tuple(kv, nk, seed);
 }
 __global__ void __launch_bounds__(GS_BLOCK) k_gs_permute(const int64_t *__restrict__ in,
                                                          const uint32_t *__restrict__ perm, uint64_t n,
