@@ -27,6 +27,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "groupby.h"
@@ -41,9 +42,11 @@ constexpr uint32_t GB_DENSE_BITS = 26;
 // aggregated again in a table of 2n slots.
 constexpr uint64_t GB_HASH_START = 1ull << 20;
 constexpr uint64_t GB_FIRST_PROBES = 64;
-// Rows from which wide codes of many groups may be sorted instead, and from which a sample of
-// 8192 rows is taken instead of 2048.
+// Rows from which wide codes of many groups may be sorted instead (gb_wide), and from which a sample
+// of 8192 rows is taken instead of 2048.
 constexpr uint64_t GB_SORT_MIN = 1ull << 17, GB_SORT_LARGE = 1ull << 20;
+// Codes that never index accumulators directly, but fit a word.
+__host__ __device__ constexpr bool gb_wide_bits(uint32_t bits) { return bits > GB_DENSE_BITS && bits <= 63; }
 
 __global__ void __launch_bounds__(256) k_gb_init(uint64_t *tkey, GbArgs a, uint64_t cap) {
   for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < cap;
@@ -383,10 +386,87 @@ __global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uin
   }
 }
 
-// Smallest and largest key values among 16 spread runs of 1024 rows (n >= 16384), one block.
+// What a sample of 1024 J rows, 16 J spread runs of 64 (n >= 1024 J), tells of wide keys.
+enum { GW_FOUND, GW_ONCE, GW_MOST, GW_EQUAL, GW_RISING, GW_WORDS };
+// By a block of 1024 threads: latency only, so all rows are read at once.  Rows are told apart by
+// their tuple's hash; those that start a run of equal tuples are counted in an LDS table of 18-bit
+// fingerprints and 14-bit counts, at most half full:
+//   FOUND  distinct tuples, ONCE those of one run, MOST the runs of the most frequent one;
+//   EQUAL  rows whose tuple is that of the row before (in their 64);
+//   RISING how many of the 16 J first rows have a first key not below the one before.
+template <int J>
+__device__ __forceinline__ void gb_wide_sample(const GbArgs &a, uint64_t n, uint64_t *__restrict__ out) {
+  constexpr uint32_t SET = 2048 * J;
+  __shared__ uint32_t set[SET];
+  __shared__ int64_t first[16 * J];
+  __shared__ uint32_t sum[GW_WORDS];
+  const uint64_t step = (n - 64) / (16 * J - 1);
+  int64_t kv[J][ALN_MAX_KEYS];
+#pragma unroll
+  for (int k = 0; k < ALN_MAX_KEYS; ++k)
+#pragma unroll
+    for (int j = 0; j < J; ++j)
+      kv[j][k] = k < a.nk ? a.keys[k][step * (16 * j + threadIdx.x / 64) + __lane_id()] : 0;
+  for (uint32_t i = threadIdx.x; i < SET; i += 1024) set[i] = 0;
+  if (threadIdx.x < GW_WORDS) sum[threadIdx.x] = 0;
+  __syncthreads();
+  uint32_t w[GW_WORDS] = {0, 0, 0, 0, 0};
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    const uint64_t h = murmur64a_tuple(kv[j], a.nk, 0x9747b28cu), above = __shfl_up(h, 1, 64);
+    if (__lane_id() == 0) first[16 * j + threadIdx.x / 64] = kv[j][0];
+    if (__lane_id() > 0 && above == h) {
+      ++w[GW_EQUAL];
+      continue;
+    }
+    const uint32_t f = (uint32_t)(h >> 46) | 1u;
+    uint32_t at = (uint32_t)h & (SET - 1);
+    while (true) {
+      const uint32_t old = atomicCAS(&set[at], 0u, f << 14 | 1u);
+      if (old != 0 && old >> 14 == f) atomicAdd(&set[at], 1u);
+      if (old == 0 || old >> 14 == f) break;
+      at = (at + 1) & (SET - 1);
+    }
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < SET; i += 1024) {
+    const uint32_t c = set[i] & 0x3FFFu;
+    w[GW_FOUND] += c != 0;
+    w[GW_ONCE] += c == 1;
+    w[GW_MOST] = c > w[GW_MOST] ? c : w[GW_MOST];
+  }
+  if (threadIdx.x > 0 && threadIdx.x < 16 * J) w[GW_RISING] = first[threadIdx.x] >= first[threadIdx.x - 1];
+#pragma unroll
+  for (int q = 0; q < GW_WORDS; ++q) {
+    for (int o = 32; o > 0; o >>= 1) {
+      const uint32_t x = (uint32_t)__shfl_xor((int)w[q], o, 64);
+      w[q] = q == GW_MOST ? (x > w[q] ? x : w[q]) : w[q] + x;
+    }
+    if (__lane_id() == 0) {
+      if (q == GW_MOST)
+        atomicMax(&sum[q], w[q]);
+      else
+        atomicAdd(&sum[q], w[q]);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int q = 0; q < GW_WORDS; ++q) out[q] = sum[q];
+}
+
+template <int J>
+__global__ void __launch_bounds__(1024) k_gb_sample(GbArgs a, uint64_t n, DevResult r) {
+  gb_wide_sample<J>(a, n, r.dst);
+  if (threadIdx.x == 0) result_done(r);
+}
+
+// Smallest and largest key values among 16 spread runs of 1024 rows (n >= 16384), one block; and,
+// when these ranges make wide codes already, what gb_wide asks of them (the same wait).
 __global__ void __launch_bounds__(1024) k_gl_sample(GbArgs a, uint64_t n, DevResult r) {
   __shared__ int64_t lo[16], hi[16];
+  __shared__ uint32_t bits;
   const uint64_t step = (n - 1024) / 15;
+  if (threadIdx.x == 0) bits = 0;
   for (int k = 0; k < a.nk; ++k) {
     int64_t x[16], mn = INT64_MAX, mx = INT64_MIN;
 #pragma unroll
@@ -413,50 +493,12 @@ __global__ void __launch_bounds__(1024) k_gl_sample(GbArgs a, uint64_t n, DevRes
       }
       r.dst[2 * k] = (uint64_t)mn;
       r.dst[2 * k + 1] = (uint64_t)mx;
+      bits += mx == mn ? 0 : 64 - (uint32_t)__builtin_clzll((uint64_t)mx - (uint64_t)mn);
     }
     __syncthreads();
   }
+  if (gb_wide_bits(bits)) gb_wide_sample<8>(a, n, r.dst + 2 * ALN_MAX_KEYS);
   if (threadIdx.x == 0) result_done(r);
-}
-
-// Distinct key codes among 1024 J rows, 16 J spread runs of 64 (n >= 1024 J), by 32-bit
-// fingerprints in an LDS set, and the rows whose code is that of the row before in their run; one
-// block: latency only, so all rows are read at once.
-template <int J>
-__global__ void __launch_bounds__(1024) k_gb_distinct(GbArgs a, uint64_t n, DevResult r) {
-  constexpr uint32_t SET = 2048 * J;
-  __shared__ uint32_t set[SET];
-  __shared__ uint32_t found, equal;
-  const uint64_t step = (n - 64) / (16 * J - 1);
-  uint64_t code[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) code[j] = gb_code(a, step * (16 * j + threadIdx.x / 64) + __lane_id());
-  for (uint32_t i = threadIdx.x; i < SET; i += 1024) set[i] = 0;
-  if (threadIdx.x == 0) found = equal = 0;
-  __syncthreads();
-  uint32_t mine = 0, same = 0;
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    const uint64_t above = __shfl_up(code[j], 1, 64);
-    same += __lane_id() > 0 && above == code[j];
-    const uint64_t h = murmur64a_u64(code[j], 0x9747b28cu);
-    const uint32_t f = (uint32_t)(h >> 32) | 1u;
-    uint32_t at = (uint32_t)h & (SET - 1);
-    while (true) {  // at most half full
-      const uint32_t old = atomicCAS(&set[at], 0u, f);
-      mine += old == 0;
-      if (old == 0 || old == f) break;
-      at = (at + 1) & (SET - 1);
-    }
-  }
-  atomicAdd(&found, mine);
-  atomicAdd(&equal, same);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    r.dst[0] = found;
-    r.dst[1] = equal;
-    result_done(r);
-  }
 }
 
 // ---- many codes: partitions of the code range ------------------------------------------------
@@ -1033,6 +1075,65 @@ static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, 
   return ALN_OK;
 }
 
+// The route of wide key codes: sorted, or through the table with nb blocks; and about how many
+// groups there are.
+struct GbWide {
+  bool sort;
+  uint32_t nb;
+  double groups;
+};
+
+// From a sample (k_gb_sample).  Sorting takes about 97 us per 1M rows whatever the keys.  The table's
+// time depends on the rows that miss the blocks' LDS tables: 64-way global atomics, about as dear for
+// a few lanes of a wave as for many of them, dearer the larger the table, and on 5 ns for every new
+// group (the count of groups is one address).  Codes come in three kinds:
+//   sorted   the sample's runs rise and do not return: every run of equal codes is a group;
+//   skewed   one code far more frequent than the mean: groups grow as a power of the rows, whose
+//            exponent is the share of the sample's codes seen once;
+//   even     from the repeats among the sample's runs.
+// The constants are fitted to both routes' times over 216 inputs of 140,000 to 40M rows of 50 to
+// 4M groups, uniform, Zipf 1.2 to 2.2, one hot key, sorted, and in blocks of 3, 16 and 100 rows
+// (sorted / table us, the one taken marked: 1.5M rows of 1500 groups 407 / 391*, of 4000 421* / 459;
+// 12M rows of 2500 groups 1460 / 1221*, of 20,000 1368* / 1623, Zipf 1.8 1749 / 842*, 600 groups in
+// blocks of 16 rows 1385 / 466*, 1M sorted groups 1395* / 3557; 40M rows 99 % of one key 5109 / 1990*).
+static GbWide gb_wide(uint64_t n, bool large, const uint64_t *s) {
+  const double rows = large ? 8192 : 2048, pairs = rows - rows / 64, m = (double)n;
+  const double starts = pairs - (double)s[GW_EQUAL], heads = rows - (double)s[GW_EQUAL];
+  const double found = (double)s[GW_FOUND], once = (double)s[GW_ONCE], runs = m * starts / pairs;
+  const bool sorted = s[GW_RISING] == (large ? 127u : 31u) && starts < pairs / 2 && found >= starts;
+  const bool skewed = !sorted && (double)s[GW_MOST] > 8 + 4 * heads / found;
+  GbWide p;
+  double cold = 1;  // share of the runs that miss the LDS tables
+  if (sorted) {
+    p.groups = runs;
+  } else if (skewed) {
+    p.groups = found * std::pow(std::max(runs, m / 64) / heads, once / found);
+    cold = once / heads;
+  } else {  // found = groups * (1 - exp(-heads / groups))
+    if (heads - found <= heads / 8) {
+      p.groups = heads * heads / 2 / std::max(heads - found, 0.5);
+    } else {
+      p.groups = found;
+      for (int i = 0; i < 60; ++i) p.groups = found / (1 - std::exp(-heads / p.groups));
+    }
+    p.groups = std::max(1.0, std::min(p.groups, runs));
+    cold = std::max(0.0, 1 - 1000 / p.groups);
+  }
+  p.groups = std::min(p.groups, m);
+  // blocks of 8192 rows (a block adds up to 1024 groups of its LDS table to the global one at its
+  // end); beyond 1024 of them only where few rows of a block miss that table, or repeat in it
+  const bool more = sorted ? starts <= pairs / 512 : skewed == (starts >= pairs / 2);
+  p.nb = (uint32_t)std::max<uint64_t>(256, std::min<uint64_t>(more ? 2048 : 1024, n >> 13));
+  const double lanes = 64 * (runs / m + 1.0 / 64) * cold, wave = lanes < 1 ? 6 * lanes : 6 + lanes * 58 / 64;
+  const double flush = p.nb * std::min(std::min(1000.0, p.groups), std::max(1.0, runs / p.nb));
+  const double adds = m / 64 * wave * (skewed ? 1.5 : 1) + flush;
+  const double scan = 27e-6 * m + (80e-6 + 20e-6 * std::min(1.0, 3e6 / m)) * adds * (1 + p.groups / 100e3);
+  const double fresh = 5e-3 * p.groups;
+  const double table = 200 + std::max(scan, fresh) + 0.8 * std::min(scan, fresh);
+  p.sort = p.groups > 0.85 * GB_HASH_START || 270 + 97e-6 * m <= table;
+  return p;
+}
+
 // Whether an output (up to m values are written) lies over an input.
 static bool gb_in_place(const GbArgs &a, uint64_t n, const GbOut &o, uint64_t m) {
   auto over = [&](const int64_t *in, const int64_t *out) {
@@ -1211,18 +1312,23 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   uint32_t total = 0;
   bool lds_taken = false, lds_done = false, outside = false;
   int cnt = -1;
+  uint64_t wide[GW_WORDS];
+  bool have_wide = false;
+  static_assert(GL_SAMPLE_MIN == GB_SORT_LARGE, "one sample for both");
   if (nkeys && n >= GL_SAMPLE_MIN) {
     DevResult r;
-    int64_t h[2 * ALN_MAX_KEYS];
-    ALN_TRY(result_open(c, 2 * ALN_MAX_KEYS, &r));
+    int64_t h[2 * ALN_MAX_KEYS + GW_WORDS];
+    ALN_TRY(result_open(c, 2 * ALN_MAX_KEYS + GW_WORDS, &r));
     hipLaunchKernelGGL(k_gl_sample, dim3(1), dim3(1024), 0, c->stream, a, n, r);
     ALN_TRY(check_launch("gb_sample"));
-    ALN_TRY(result_wait(c, r, h, 16 * (size_t)nkeys));
+    ALN_TRY(result_wait(c, r, h, sizeof(h)));
     for (int k = 0; k < nkeys; ++k) {
       mn[k] = h[2 * k];
       mx[k] = h[2 * k + 1];
     }
     total = gb_layout(a, mn, mx);
+    have_wide = gb_wide_bits(total);
+    memcpy(wide, h + 2 * ALN_MAX_KEYS, sizeof(wide));
     if (total > 0 && total <= GL_SAMPLE_BITS)
       ALN_TRY(gb_few(c, a, n, total, order, o, cap, h_ngroups, &cnt, &lds_taken, &lds_done, &outside));
     if (outside) lds_taken = lds_done = false;
@@ -1254,11 +1360,8 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
   // LDS-cached aggregation kernel: at most 2048 blocks, of at least 4 rows per thread (450,000 rows
   // into 200,000 groups: 119 us in 55 blocks of 32 rows per thread, 50 us)
   const size_t lds = gb_lds_bytes(nvals);
-  // (wide keys: every block adds its LDS table to the global one, up to 1024 groups of it.  1.1M
-  // rows, 600 and 1500 groups: 297 and 403 us with 1024 blocks, 253 and 340 with 256; 12M rows:
-  // 748 and 978 with 256 blocks, 522 and 1000 with 512)
   const uint32_t nb = grid_for(n, 256 * 4, 2048);
-  uint32_t nbh = std::min<uint32_t>(nb, n >> 12 < 256 ? 256 : n >> 12 < 512 ? n >> 12 : 512);
+  uint32_t nbh = std::min<uint32_t>(nb, 256);  // wide codes of few rows; more: gb_wide
   if (lds > 65536) {
     ALN_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_gb_agg<true>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1295,35 +1398,22 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
       return stream_wait(c);
     }
   } else {
-    // many groups: global atomics (24 G/s) cost more than sorting the rows (12M rows of 12M groups:
-    // 12 against 1.0 ms; 2.5M rows of 1500 groups 416 us against 520, of 2500 groups 579 against
-    // 412).  1900 of 8192 rows distinct means some 2000 groups or more.  Fewer rows are worth
-    // sorting for more groups, 25000 at 250000 rows and 6500 at 1M, as told by the repeats among
-    // 2048 rows (150000 rows, 10000 groups 215 us and sorted 252, 60000 groups 260 and 232; 450000
-    // rows, 10000 groups 276 and 284, 25000 groups 296 and 261; 1M rows, 10000 groups 379 and 304).
-    // (In place, the tables: they have read every row before a group is written.)
+    // (In place, the table: it has read every row before a group is written.)
     if (n >= GB_SORT_MIN && !gb_in_place(a, n, o, std::min(n, cap))) {
-      DevResult r;
-      uint64_t h[2] = {0, 0};
-      bool many = false;
       const bool large = n >= GB_SORT_LARGE;
-      ALN_TRY(result_open(c, 2, &r));
-      if (large)
-        hipLaunchKernelGGL(k_gb_distinct<8>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
-      else
-        hipLaunchKernelGGL(k_gb_distinct<2>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
-      ALN_TRY(check_launch("gb_distinct"));
-      ALN_TRY(result_wait(c, r, h, 16));
-      const uint64_t found = h[0], pairs = large ? 128 * 63 : 32 * 63, starts = pairs - h[1];
-      // rows in the order of their keys, or clustered: a wave's atomics are few, and so are the
-      // distinct codes of the sample.  Runs of 1000 rows leave a block little but to read (12M rows
-      // of 4000 groups: 742 us with 512 blocks, 604 with 2048); more groups than the first table
-      // holds are sorted (12M sorted rows of 1M groups: 3.7 ms in two tables, 0.83 sorted).
-      const bool clustered = 2 * h[1] > pairs;
-      if (clustered && n / pairs * starts > GB_HASH_START / 2) many = true;
-      if (clustered && starts <= pairs / 512) nbh = nb;
-      if (large ? found >= 1900 : 2048 - found <= 2048 / 24 * std::max<uint64_t>(1, n >> 18)) many = true;
-      if (many) {
+      if (!have_wide) {
+        DevResult r;
+        ALN_TRY(result_open(c, GW_WORDS, &r));
+        if (large)
+          hipLaunchKernelGGL(k_gb_sample<8>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
+        else
+          hipLaunchKernelGGL(k_gb_sample<2>, dim3(1), dim3(1024), 0, c->stream, a, n, r);
+        ALN_TRY(check_launch("gb_sample"));
+        ALN_TRY(result_wait(c, r, wide, sizeof(wide)));
+      }
+      const GbWide p = gb_wide(n, large, wide);
+      nbh = std::min(nb, p.nb);
+      if (p.sort) {
         const WsMark mark = ws_mark(c);
         const int rc = gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
         if (rc != ALN_E_NOMEM) return rc;

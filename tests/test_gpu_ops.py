@@ -493,6 +493,39 @@ def test_groupby_sample_missed(ctx, n, outlier, nv, order):
         _gb_check(ctx, keys, cols[:1] * 2, [L.AGG_SUM, L.AGG_COUNT], order=order, bounds=bounds)
 
 
+@pytest.mark.parametrize("kind,n,sort", [("blocks", 9_000_000, False), ("sorted", 9_000_000, False),
+                                         ("one_row_runs", 2_000_000, True), ("zipf", 2_000_000, False),
+                                         ("hot", 2_000_000, False), ("hot_tail", 2_000_000, True),
+                                         ("blocks", 200_000, False), ("one_row_runs", 200_000, True)])
+def test_groupby_wide_route(ctx, kind, n, sort):
+    """Wide keys whose rows come in blocks of a few repeated keys, in order, skewed, with one hot key
+    and few or many others, or all different: the groups, and the route a sample chooses for them
+    (few global additions: the table, however the rows are clustered; many: sorting)."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n + len(kind))
+    gid = {"blocks": lambda: np.repeat(r.integers(0, 600, n // 16 + 1), 16)[:n],
+           "sorted": lambda: np.sort(r.integers(0, 20000, n)),
+           "one_row_runs": lambda: r.integers(0, n, n),
+           "zipf": lambda: np.minimum(r.zipf(2.0, n), 1 << 20),
+           "hot": lambda: np.where(r.random(n) < 0.99, 0, r.integers(0, n, n)),
+           "hot_tail": lambda: np.where(r.random(n) < 0.5, 0, r.integers(0, n, n))}[kind]().astype(np.int64)
+    v = r.integers(-1000, 1000, n).astype(np.int64)
+    cnt = np.bincount(gid)
+    g = np.nonzero(cnt)[0]
+    want = [g * 1_000_003 + 5, np.bincount(gid, weights=v)[g].astype(np.int64), cnt[g]]
+    dk, dv = dev(ctx, gid * 1_000_003 + 5), dev(ctx, v)
+    ctx.profile()
+    ctx.profile_reset()
+    try:
+        k, out = D.groupby(ctx, [dk], [dv, dv], [L.AGG_SUM, L.AGG_COUNT])
+        assert ctx.profile_get("groupby_sorted_agg")[1] == int(sort)
+    finally:
+        ctx.profile(False)
+    for x, y in zip(k + out, want):
+        assert np.array_equal(host(x), y)
+
+
 def gb_raw(ctx, keys, vals, aggs, order, outk, outv, cap):
     """aln_groupby into given output tensors: (status, number of groups)."""
     import ctypes as C
