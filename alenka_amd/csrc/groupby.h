@@ -88,8 +88,9 @@ struct GbOut {
 
 // Groups by sorting the rows (groupsort.hip): packed codes of `total` bits, or, above 63 bits, key
 // tuples.  Writes the groups in the order asked for.
-// kmax: the keys' largest values (the smallest are in a).
-int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, uint32_t seed,
-              const GbOut &o, uint64_t cap, uint64_t *h_ngroups);
+// kmax: the keys' largest values (the smallest are in a).  by_key: for hash order, sort the rows by
+// key all the same and then the groups by hash.
+int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, bool by_key,
+              uint32_t seed, const GbOut &o, uint64_t cap, uint64_t *h_ngroups);
 
 }  // namespace aln

@@ -1075,10 +1075,13 @@ static int gb_few(aln_ctx *c, GbArgs &a, uint64_t n, uint32_t total, int order, 
   return ALN_OK;
 }
 
-// The route of wide key codes: sorted, or through the table with nb blocks; and about how many
-// groups there are.
+// The route of wide key codes: sorted (by_key: for hash order all the same), or through the table
+// with nb blocks; and about how many groups there are.  Rows of groups of 32 rows and more share all
+// 64 bits of the hash, which the sort's buckets do not hold, and eight digit passes would follow
+// instead of the code's four or five (12M rows of 4000 groups 1.96 ms by hash, 1.47 by key, of
+// 250,000 groups 1.53 and 1.63).
 struct GbWide {
-  bool sort;
+  bool sort, by_key;
   uint32_t nb;
   double groups;
 };
@@ -1096,7 +1099,7 @@ struct GbWide {
 // (sorted / table us, the one taken marked: 1.5M rows of 1500 groups 407 / 391*, of 4000 421* / 459;
 // 12M rows of 2500 groups 1460 / 1221*, of 20,000 1368* / 1623, Zipf 1.8 1749 / 842*, 600 groups in
 // blocks of 16 rows 1385 / 466*, 1M sorted groups 1395* / 3557; 40M rows 99 % of one key 5109 / 1990*).
-static GbWide gb_wide(uint64_t n, bool large, const uint64_t *s) {
+static GbWide gb_wide(uint64_t n, bool large, int order, const uint64_t *s) {
   const double rows = large ? 8192 : 2048, pairs = rows - rows / 64, m = (double)n;
   const double starts = pairs - (double)s[GW_EQUAL], heads = rows - (double)s[GW_EQUAL];
   const double found = (double)s[GW_FOUND], once = (double)s[GW_ONCE], runs = m * starts / pairs;
@@ -1130,7 +1133,9 @@ static GbWide gb_wide(uint64_t n, bool large, const uint64_t *s) {
   const double scan = 27e-6 * m + (80e-6 + 20e-6 * std::min(1.0, 3e6 / m)) * adds * (1 + p.groups / 100e3);
   const double fresh = 5e-3 * p.groups;
   const double table = 200 + std::max(scan, fresh) + 0.8 * std::min(scan, fresh);
-  p.sort = p.groups > 0.85 * GB_HASH_START || 270 + 97e-6 * m <= table;
+  // (hash order: the table's groups are sorted by hash anyway, the sorted ones as an extra step)
+  p.by_key = order == ALN_ORDER_HASH && 32 * p.groups < m;
+  p.sort = p.groups > 0.85 * GB_HASH_START || 270 + (p.by_key ? 70 : 0) + 97e-6 * m <= table;
   return p;
 }
 
@@ -1356,7 +1361,7 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
     ALN_TRY(check_launch("gb_reduce_final"));
     return stream_wait(c);
   }
-  if (total > 63) return gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
+  if (total > 63) return gb_sorted(c, a, n, total, mx, order, false, seed, o, cap, h_ngroups);
   // LDS-cached aggregation kernel: at most 2048 blocks, of at least 4 rows per thread (450,000 rows
   // into 200,000 groups: 119 us in 55 blocks of 32 rows per thread, 50 us)
   const size_t lds = gb_lds_bytes(nvals);
@@ -1411,11 +1416,11 @@ int aln_groupby(aln_ctx *c, const int64_t *const *d_keys, int nkeys, const int64
         ALN_TRY(check_launch("gb_sample"));
         ALN_TRY(result_wait(c, r, wide, sizeof(wide)));
       }
-      const GbWide p = gb_wide(n, large, wide);
+      const GbWide p = gb_wide(n, large, order, wide);
       nbh = std::min(nb, p.nb);
       if (p.sort) {
         const WsMark mark = ws_mark(c);
-        const int rc = gb_sorted(c, a, n, total, mx, order, seed, o, cap, h_ngroups);
+        const int rc = gb_sorted(c, a, n, total, mx, order, p.by_key, seed, o, cap, h_ngroups);
         if (rc != ALN_E_NOMEM) return rc;
         ws_rewind(c, mark, true);  // a table of few enough groups needs less (48 to 85 MB for 2^20)
       }

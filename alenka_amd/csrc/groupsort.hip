@@ -5,7 +5,8 @@
 //     (50 G/s): one read per row instead of one per column;
 //   * the rows are ordered by one 64-bit code: the packed key code (key order), or the tuple's
 //     MurmurHash64A (the multi-segment merge order, merge.cu:138-203, which needs no second sort
-//     then), or, for key tuples wider than 63 bits in key order, by the keys themselves;
+//     then; codes of 63 bits of few groups are sorted by key and the groups by hash), or, for key
+//     tuples wider than 63 bits in key order, by the keys themselves;
 //   * a wave takes 1024 sorted rows, 64 at a time, combines the runs with a segmented scan,
 //     carries the open run to the next 64 rows and stores each group when its run ends; only
 //     runs that cross waves are combined with atomics.
@@ -431,11 +432,11 @@ static int gs_fit(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const
   return gs_run(c, a, n, total, kmax, hashed, false, seed, o, cap, h_ngroups, clash);
 }
 
-int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, uint32_t seed,
-              const GbOut &o, uint64_t cap, uint64_t *h_ngroups) {
+int gb_sorted(aln_ctx *c, const GbArgs &a, uint64_t n, uint32_t total, const int64_t *kmax, int order, bool by_key,
+              uint32_t seed, const GbOut &o, uint64_t cap, uint64_t *h_ngroups) {
   bool clash = false;
   const WsMark mark = ws_mark(c);
-  if (order == ALN_ORDER_HASH) {
+  if (order == ALN_ORDER_HASH && !by_key) {
     ALN_TRY(gs_fit(c, a, n, total, kmax, true, seed, o, cap, h_ngroups, &clash));
     if (!clash) {
       return stream_wait(c);

@@ -526,6 +526,17 @@ def test_groupby_wide_route(ctx, kind, n, sort):
         assert np.array_equal(host(x), y)
 
 
+@pytest.mark.parametrize("n,groups", [(1 << 20, 30000), (1_100_000, 34000), (1_100_000, 40000), (300_007, 9000)])
+def test_groupby_hash_order_by_key(ctx, n, groups):
+    """Hash order of sorted wide keys around 32 rows a group, from where the rows are sorted by key
+    and the groups by hash, against the oracle; two keys and one, several aggregates."""
+    r = np.random.default_rng(n + groups)
+    gid = r.integers(0, groups, n)
+    v, w = r.integers(-(1 << 40), 1 << 40, n).astype(np.int64), r.integers(-1000, 1000, n).astype(np.int64)
+    for keys in ([gid * 0x12345677 + 5], [gid * 1_000_003 - 77, gid % 5 * 10_000_019]):
+        _gb_check(ctx, [k.astype(np.int64) for k in keys], [v, v, w, v], AGGS4, order=L.ORDER_HASH, bounds=[0, n // 2, n])
+
+
 def gb_raw(ctx, keys, vals, aggs, order, outk, outv, cap):
     """aln_groupby into given output tensors: (status, number of groups)."""
     import ctypes as C
