@@ -1354,12 +1354,14 @@ int topk_codes(aln_ctx *c, uint64_t *code, uint32_t *idx, uint64_t n, uint32_t k
 //   k_tk_collect  the rows within the bound, read again only in chunks that have one
 //   k_tk_final    one block sorts up to tf_max candidates by all keys and row number
 // With one key, equal codes are ordered by row, so the bound is a (code, chunk) pair and rows
-// of the bound's code count only up to its chunk: at most k chunks of candidates whatever the
-// values.  With more keys every row that ties on the first is a candidate; when those are too
-// many (a flag), the keys' codes are written out and bounded as one key.  Candidates too many
-// for k_tk_final go through the tile sort.
+// of the bound's code count only up to its chunk: at most k * ceil(chunks / TK_GROUPS) chunks of
+// candidates whatever the values.  With more keys every row that ties on the first is a candidate.
+// Candidates too many for k_tk_final go through the tile sort, or, when most rows tie, the keys'
+// codes are written out and bounded as one key; more than TK_CAND candidates leave the call to the
+// tile sort of all rows, also with one key.
 constexpr uint32_t TK_GROUPS = 4096;
 constexpr uint32_t TK_CAND = 1u << 20;
+constexpr uint64_t TK_ALL = 1ull << 20;
 constexpr int TF_BLOCK = 1024;
 
 // Order-preserving unsigned code of a key value over the whole int64 range; of a code (desc
@@ -1590,6 +1592,12 @@ static int topk_bounded(aln_ctx *c, const TfArgs &a, uint64_t n, uint32_t k, uin
     return ALN_OK;
   }
   if (m > TK_CAND) return ALN_OK;
+  // Rows in order leave k chunks of candidates, an eighth of all rows at most: more are ties of
+  // the first key, and the codes of all rows spread again where the candidates' tile sort is a
+  // gather and ranges of every key and several launches (100,000 rows of 5 first values, first 100:
+  // 190 us by the tile sort, 145 by all rows' codes, of one value, first 500, 339 and 165; 2M rows, first
+  // 500 504 and 312, but first 100 241 and 247, first 10 207 and 241).
+  if (a.nk > 1 && m > n / 8 && 4 * m > 320ull * u * k && (n <= TK_ALL || k >= 256)) return ALN_OK;
   // the tile sort of the candidates' codes
   const unsigned gm = grid_for(m, 256, 65536);
   uint64_t *code;
