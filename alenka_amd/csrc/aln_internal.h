@@ -122,7 +122,7 @@ int copy_to_host(aln_ctx *c, void *h, const void *d, size_t bytes);  // synchron
 int copy_to_device(aln_ctx *c, void *d, const void *h, size_t bytes);
 
 // Results a kernel hands to the host itself: it writes them to dst and calls result_done after
-// its last write (one thread, after a fence by any other that wrote).  dst is coherent host
+// its last write (one thread, after block_stores_done or a fence by any other that wrote).  dst is coherent host
 // memory whose flag word the host polls, or (flag NULL) a device buffer that is copied.  One
 // at a time per context, and no copy_to_host between open and wait.
 struct DevResult {
@@ -209,6 +209,13 @@ struct DevCols {
 // ---- device helpers ---------------------------------------------------------------------
 namespace aln {
 
+// Barrier after which every wave's stores are in the block's L2: the system-scope fence of the one
+// thread that calls result_done then publishes them too (a fence in each wave would write the L2 back
+// once per wave: 2 to 3 us a call).
+__device__ __forceinline__ void block_stores_done() {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
 __device__ __forceinline__ void result_done(const DevResult &r) {
   if (!r.flag) return;
   __threadfence_system();

@@ -421,8 +421,7 @@ __global__ void __launch_bounds__(64 * SCAN_ONE_WAVES) k_scan_one(const T *__res
     const uint32_t i = base + (uint32_t)j * 64;
     if ((uint32_t)j < rows && i < n) out[i] = off + v[j];
   }
-  __threadfence();  // the scan is complete, for every stream, when the host has the total
-  __syncthreads();
+  block_stores_done();  // the scan is complete, for every stream, when the host has the total
   if (threadIdx.x == 0) {
     r.dst[0] = total;
     result_done(r);

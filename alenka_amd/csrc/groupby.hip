@@ -377,8 +377,7 @@ __global__ void __launch_bounds__(1024) k_gl_emit(GlArgs a, GbOut o, int nv, uin
     base += all;
     __syncthreads();
   }
-  __threadfence_system();  // the call returns on the result: every wave's groups are written by then
-  __syncthreads();
+  block_stores_done();  // the call returns on the result: every wave's groups are written by then
   if (threadIdx.x == 0) {
     r.dst[0] = total;
     r.dst[1] = miss;
