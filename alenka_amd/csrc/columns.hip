@@ -144,10 +144,13 @@ __global__ void __launch_bounds__(256) k_pack(const int64_t *__restrict__ v, uin
 
 // Rows outside the column (a segment past nsegs, or past a short last segment) read as 0.
 //
-// Consecutive rows [r0, r0 + n): a block's 2048 rows mostly lie in one segment, whose
-// descriptor is then scalar and whose codes are unpacked with 32-bit bit positions (HBM-bound:
-// 50M 24-bit codes 260 -> 94 us; a descriptor, a division and 64-bit positions per row before).
-constexpr int DEC_ROWS = 8;
+// Consecutive rows [r0, r0 + n): a block's rows mostly lie in one segment, whose descriptor is then
+// scalar and whose codes are unpacked with 32-bit bit positions (HBM-bound: 50M 24-bit codes 260 ->
+// 94 us; a descriptor, a division and 64-bit positions per row before).  Eight rows per thread, or one
+// where many blocks of 2048 rows would cross segments (1M rows in segments of 1000 rows: 11.2 us a
+// call with eight, 9.7 with one).
+constexpr uint32_t DEC_SEG_ROWS = 8192;
+template <int DEC_ROWS>
 __global__ void __launch_bounds__(256) k_decode(const uint32_t *__restrict__ words,
                                                 const aln_seg *__restrict__ segs, uint32_t nsegs,
                                                 uint32_t seg_rows, uint64_t r0, uint64_t n,
@@ -157,8 +160,8 @@ __global__ void __launch_bounds__(256) k_decode(const uint32_t *__restrict__ wor
   const uint64_t seg = (r0 + b0) / seg_rows;
   const uint32_t l0 = (uint32_t)(r0 + b0 - seg * seg_rows);
   out += b0;
-  if (seg < nsegs && (uint64_t)l0 + m <= segs[seg].nrows) {
-    const aln_seg sg = segs[seg];
+  const aln_seg sg = segs[seg < nsegs ? seg : 0];
+  if (seg < nsegs && (uint64_t)l0 + m <= sg.nrows) {
     const uint64_t bit = (uint64_t)l0 * sg.bits;
     uint32_t idx[DEC_ROWS];
     uint64_t c[DEC_ROWS];
@@ -748,6 +751,22 @@ __global__ void __launch_bounds__(256) k_row_segments(const uint32_t *__restrict
   }
 }
 
+template <int DEC_ROWS>
+static int launch_decode_rows(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_begin, uint64_t n,
+                              int64_t *d_out) {
+  const uint64_t nb = (n + 256 * DEC_ROWS - 1) / (256 * DEC_ROWS);
+  ALN_REQUIRE(nb < (1ull << 31), "decode: grid too large");
+  hipLaunchKernelGGL(k_decode<DEC_ROWS>, dim3((unsigned)nb), dim3(256), 0, c->stream, col->words, col->segs,
+                     col->nsegs, seg_rows, row_begin, n, d_out);
+  return check_launch("decode");
+}
+static int launch_decode(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_begin, uint64_t n,
+                         int64_t *d_out) {
+  if (seg_rows < DEC_SEG_ROWS && n < (1ull << 38))  // (blocks of 256 rows: the grid's limit)
+    return launch_decode_rows<1>(c, col, seg_rows, row_begin, n, d_out);
+  return launch_decode_rows<8>(c, col, seg_rows, row_begin, n, d_out);
+}
+
 // ---- fixed scratch of the allocation-free scan -----------------------------------------------
 // aln_scan_filter_noalloc keeps its temporaries in this array instead of the context's
 // workspace: the per-segment zone-map verdicts it uploads, the per-tile counts, their exclusive
@@ -821,15 +840,17 @@ int aln_encode_plan(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t 
   if (nsegs == 0) return ALN_OK;
   const uint32_t bps = (uint32_t)grid_for(seg_rows, 256 * 16, 256);
   int64_t *part, *mm;
-  ALN_TRY(ws(c, 2 * (size_t)nsegs * bps, &part));
   ALN_TRY(ws(c, 2 * (size_t)nsegs, &mm));
+  part = mm;  // (one block per segment: its partials are the ranges)
+  if (bps > 1) ALN_TRY(ws(c, 2 * (size_t)nsegs * bps, &part));
   {
     ProfScope p(c, "seg_minmax");
     int64_t *pmax = part + (size_t)nsegs * bps;
     hipLaunchKernelGGL(k_seg_minmax, dim3(nsegs * bps), dim3(256), 0, c->stream, d_vals, nrows,
                        seg_rows, bps, part, pmax);
-    hipLaunchKernelGGL(k_seg_minmax_final, dim3(nsegs), dim3(64), 0, c->stream, (const int64_t *)part,
-                       (const int64_t *)pmax, bps, nsegs, mm);
+    if (bps > 1)
+      hipLaunchKernelGGL(k_seg_minmax_final, dim3(nsegs), dim3(64), 0, c->stream, (const int64_t *)part,
+                         (const int64_t *)pmax, bps, nsegs, mm);
   }
   ALN_TRY(check_launch("seg_minmax"));
   std::vector<int64_t> range(2 * (size_t)nsegs);
@@ -907,15 +928,6 @@ int aln_plain_col(aln_ctx *c, const int64_t *d_vals, uint64_t nrows, uint32_t se
   out->nsegs = nsegs;
   out->decimals = decimals;
   return ALN_OK;
-}
-
-static int launch_decode(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_begin, uint64_t n,
-                         int64_t *d_out) {
-  const uint64_t nb = (n + 256 * DEC_ROWS - 1) / (256 * DEC_ROWS);
-  ALN_REQUIRE(nb < (1ull << 31), "decode: grid too large");
-  hipLaunchKernelGGL(k_decode, dim3((unsigned)nb), dim3(256), 0, c->stream, col->words, col->segs, col->nsegs,
-                     seg_rows, row_begin, n, d_out);
-  return check_launch("decode");
 }
 
 int aln_decode(aln_ctx *c, const aln_col *col, uint32_t seg_rows, uint64_t row_begin,

@@ -222,7 +222,6 @@ def hash_join(ctx, build_keys, probe_keys, cap=None):
     if cap is None:
         L.check(ctx.lib.aln_hash_join_count(ctx.h, _p(build_keys), nb, _p(probe_keys), npb, C.byref(cnt)),
                 "aln_hash_join_count")
-        cap = cnt.value
         rc = L.ALN_E_CAPACITY
     else:
         pi, bi = ctx.empty(cap, torch.int32), ctx.empty(cap, torch.int32)

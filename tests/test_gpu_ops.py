@@ -71,7 +71,8 @@ def test_encode_decode(ctx, name, gen, n, seg_rows):
     assert np.array_equal(host(got), v[rows])
 
 
-@pytest.mark.parametrize("n,seg_rows", [(7, 7), (2047, 5000), (2049, 2049), (4129, 4096), (6200, 3000)])
+@pytest.mark.parametrize("n,seg_rows", [(7, 7), (2047, 5000), (2049, 2049), (4129, 4096), (6200, 3000),
+                                        (2049, 8191), (2049, 8192), (20481, 8192), (18433, 8200)])
 def test_codec_every_width(ctx, n, seg_rows):
     """Every code width, natural and forced, at the edges of the 2048-row tiles the codes are
     packed and unpacked in: the words are the oracle's and decode to the values."""
