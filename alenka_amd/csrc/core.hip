@@ -173,8 +173,8 @@ static int readback_small(aln_ctx *c, void *h, const void *d, size_t bytes) {
 
 __global__ void k_flag(DevResult r) { result_done(r); }
 
-// The work enqueued so far is done when a kernel after it has set the flag: the host's wake-up
-// from a stream synchronisation is what this spares (about 8 us a call).
+// The work enqueued so far is done when a kernel after it has set the flag: what a stream
+// synchronisation (which polls as well) costs beyond that is spared, 4 to 12 us a call.
 int stream_wait(aln_ctx *c) {
   if (!readback_ready(c)) {
     ALN_HIP(hipStreamSynchronize(c->stream));

@@ -390,14 +390,23 @@ __global__ void __launch_bounds__(RS_BLOCK) k_rs_scatter(RsPass a) {
 // codes in input order, so the result is the same).
 constexpr uint32_t RL_W = RS_TILE / 2;  // the smallest window, half of a block's positions
 constexpr uint32_t RL_RUN = 32;
-constexpr uint32_t RL_OVERFLOW = 1, RL_REDO = 2;  // bits of *overflow
+// Bits of ctl[0]; ctl[1] counts the windows k_rs_bins left to k_rs_local.  RL_CROWDED: so many of them
+// that the windows not begun yet go there at once.
+constexpr uint32_t RL_OVERFLOW = 1, RL_REDO = 2, RL_CROWDED = 4;
+__device__ __forceinline__ uint32_t rl_peek(const uint32_t *p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Sets a bit once: thousands of atomics on one address take 6 ns each.
+__device__ __forceinline__ void rl_set(uint32_t *ctl, uint32_t bit) {
+  if (!(rl_peek(ctl) & bit)) atomicOr(ctl, bit);
+}
 
 struct RsLocal {
   const uint64_t *keys;
   const uint32_t *vals;
   uint32_t *vout;
   uint8_t *heads;  // may be NULL: 1 where a position's code differs from the one before
-  uint32_t *overflow;
+  uint32_t *ctl;
   uint8_t *redo;  // per window: left by k_rs_bins to k_rs_local
   uint64_t n;
   uint32_t w;     // window: positions whose buckets a block owns (a multiple of 64)
@@ -415,6 +424,8 @@ struct RsLocal {
 // the load to the placing; LDS holds the bins, then the placed codes with their positions (below
 // nextshift a code's bits and 12 bits of position fit 64), then the permutation.
 constexpr uint32_t RB_BINS = 8192;  // 16-bit counters, two to a word: as large as sv
+constexpr uint32_t RB_RESIDENT = 768;  // three blocks on each of 256 CUs
+constexpr uint32_t RB_WIDE = 2 * RB_RESIDENT;
 __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6, 6))) k_rs_bins(RsLocal a) {
   __shared__ uint64_t sk[RS_TILE];
   __shared__ uint32_t sv[RS_TILE];
@@ -426,6 +437,17 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   const uint32_t q = a.nblk / RS_XCDS, rm = a.nblk % RS_XCDS, x = blockIdx.x % RS_XCDS;
   const uint32_t win = x * q + min(x, rm) + blockIdx.x / RS_XCDS;
   const uint64_t n = a.n, w0 = (uint64_t)win * a.w;
+  // blocks after the first that fill the chip: nothing to do once a bucket has overflowed; once half
+  // of the windows were crowded the rest only look for an overflow (64 rows of every code, 16M rows:
+  // 1.17 ms by k_rs_local alone, 1.37 with every window tried, 1.28 now)
+  uint32_t state = 0;
+  if (blockIdx.x >= RB_RESIDENT) {
+    if (t == 0) s_long = rl_peek(a.ctl);
+    __syncthreads();
+    state = s_long;
+    if (state & RL_OVERFLOW) return;
+    __syncthreads();
+  }
   uint64_t key[RS_ITEMS];
   uint32_t val[RS_ITEMS], hi16[RS_ITEMS];
   // positions w0 + i, i = wave * 512 + row * 64 + lane
@@ -433,7 +455,7 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   for (int j = 0; j < RS_ITEMS; ++j) {
     const uint32_t i = wid * RS_WAVE_ITEMS + j * 64 + lane;
     key[j] = w0 + i < n ? __builtin_nontemporal_load(a.keys + w0 + i) : ~0ull;
-    val[j] = w0 + i < n ? __builtin_nontemporal_load(a.vals + w0 + i) : 0u;
+    val[j] = w0 + i < n && !(state & RL_CROWDED) ? __builtin_nontemporal_load(a.vals + w0 + i) : 0u;
   }
   const uint64_t before = w0 > 0 ? a.keys[w0 - 1] : 0;
   auto top = [&](uint64_t k) { return ((uint32_t)(k >> a.hish) & a.himask) << RS_BITS | ((uint32_t)(k >> a.topshift) & 0xFFu); };
@@ -486,10 +508,14 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   if (lo == 0xFFFFFFFFu) return;  // no bucket starts here (uniform across the block)
   if (hi == 0xFFFFFFFFu) {
     if (w0 + RS_TILE < n) {  // the last bucket runs past the block's capacity
-      if (t == 0) atomicOr(a.overflow, RL_OVERFLOW);
+      if (t == 0) rl_set(a.ctl, RL_OVERFLOW);
       return;
     }
     hi = (uint32_t)(n - w0);
+  }
+  if (state & RL_CROWDED) {
+    if (t == 0) a.redo[win] = 1;
+    return;
   }
   const uint32_t m = hi - lo;
   // bins: the bucket's ordinal and as many code bits below as leave RB_BINS of them
@@ -530,7 +556,8 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
     if (s_long) {
       if (t == 0) {
         a.redo[win] = 1;
-        atomicOr(a.overflow, RL_REDO);
+        rl_set(a.ctl, RL_REDO);
+        if (2 * atomicAdd(a.ctl + 1, 1u) >= blockIdx.x && blockIdx.x >= RB_RESIDENT) rl_set(a.ctl, RL_CROWDED);
       }
       return;
     }
@@ -633,7 +660,7 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   uint32_t hi = s_hi;
   if (hi == 0xFFFFFFFFu) {
     if (w0 + RS_TILE < n) {  // the last bucket runs past the block's capacity
-      if (t == 0) atomicOr(a.overflow, RL_OVERFLOW);
+      if (t == 0) rl_set(a.ctl, RL_OVERFLOW);
       return;
     }
     hi = (uint32_t)(n - w0);
@@ -894,14 +921,16 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
     uint32_t pb = bits - RS_BITS * p < RS_BITS ? bits - RS_BITS * p : RS_BITS;
     return (1u << pb) - 1;
   };
-  uint32_t *ovf;
-  ALN_TRY(ws(c, 1, &ovf));
+  uint32_t *ctl;
+  ALN_TRY(ws(c, 2, &ctl));
   // the wide window: room for a bucket of 1.25 x the mean (over the codes that the top two
   // digits' varying bits make) and 256 rows more
   const int top_bits = __builtin_popcountll(vary >> (RS_BITS * run[nrun - 1]) & pass_mask(run[nrun - 1])) +
                        __builtin_popcountll(vary >> (RS_BITS * run[nrun - 2]) & pass_mask(run[nrun - 2]));
   const uint64_t tail = (n >> top_bits) + (n >> top_bits) / 4 + 256;
-  const uint32_t wide = tail < RS_TILE - RL_W ? (uint32_t)(RS_TILE - tail) & ~63u : RL_W;
+  // (a sort whose windows are all resident at once gains little by fewer of them, and loses a second
+  // try where a bucket does not fit)
+  const uint32_t wide = tail < RS_TILE - RL_W && n > (uint64_t)RL_W * RB_WIDE ? (uint32_t)(RS_TILE - tail) & ~63u : RL_W;
   // two passes: the second most significant varying digit, then the most significant
   for (uint32_t r = 0; r < 2; ++r) {
     const uint32_t p = run[nrun - 2 + r];
@@ -946,7 +975,7 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
   l.vals = vt[1];
   l.vout = alias ? vt[0] : vout;
   l.heads = heads;
-  l.overflow = ovf;
+  l.ctl = ctl;
   l.n = n;
   l.topshift = RS_BITS * run[nrun - 2];
   l.hish = RS_BITS * run[nrun - 1];
@@ -964,14 +993,15 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
   for (uint32_t w = wide; o & RL_OVERFLOW; w = RL_W) {
     l.w = w;
     l.nblk = (uint32_t)((n + w - 1) / w);
-    ALN_TRY(fill_u32(c, ovf, 1, 0));
+    ALN_TRY(fill_u32(c, ctl, 2, 0));
     ALN_TRY(fill_u32(c, reinterpret_cast<uint32_t *>(l.redo), (l.nblk + 3) / 4, 0));
     {
       ProfScope ps(c, "radix_local");
       hipLaunchKernelGGL(k_rs_bins, dim3(l.nblk), dim3(RS_BLOCK), 0, c->stream, l);
     }
     ALN_TRY(check_launch("radix_bins"));
-    ALN_TRY(copy_to_host(c, &o, ovf, 4));
+    ALN_TRY(copy_to_host(c, &o, ctl, 4));
+    o &= RL_OVERFLOW | RL_REDO;
     if (w == RL_W) break;
   }
   if (o == RL_REDO) {
@@ -980,7 +1010,7 @@ static int rs_hybrid(aln_ctx *c, const RsIn &in, bool from_keys, uint64_t n, uin
       hipLaunchKernelGGL(k_rs_local, dim3(l.nblk), dim3(RS_BLOCK), 0, c->stream, l);
     }
     ALN_TRY(check_launch("radix_local"));
-    ALN_TRY(copy_to_host(c, &o, ovf, 4));
+    ALN_TRY(copy_to_host(c, &o, ctl, 4));
     o &= RL_OVERFLOW;
   }
   *done = o == 0;

@@ -970,6 +970,37 @@ def test_topk_candidates(ctx, n, k, kind):
         assert np.array_equal(got, want), (len(keys), desc)
 
 
+@pytest.mark.parametrize("n", [1_600_000, 3_145_728, 3_145_729, 4_000_003])
+@pytest.mark.parametrize("kind", ["copies64", "half", "long", "few_long", "heavy_low"])
+def test_sort_crowded_windows(ctx, n, kind):
+    """ORDER BY of codes that crowd the bucket path's bins (64 copies of every code, of half of
+    them), or overflow its windows (one code of 5000 rows, several, a crowd of codes in one bucket),
+    with more windows than are resident at once and at the sizes where wide windows begin; the
+    permutation is the stable one, also in the GROUP BY that sorts by codes."""
+    from alenka_amd import device as D
+
+    r = np.random.default_rng(n + len(kind))
+    spread = lambda ids: ids * np.int64(0x1234567ABCDEF)  # noqa: E731  (wraps)
+    with np.errstate(over="ignore"):
+        key = spread(r.integers(0, n * 4, n))
+        if kind == "copies64":
+            key = spread(r.integers(0, n // 64, n))
+        elif kind == "half":
+            key[: n // 2] = spread(r.integers(0, n // 128, n // 2))
+        elif kind == "long":
+            key[r.choice(n, 5000, replace=False)] = key[7]
+        elif kind == "few_long":
+            for i in range(20):
+                key[r.choice(n, 3000, replace=False)] = key[i]
+        else:
+            key[r.choice(n, 30000, replace=False)] = key[7] + r.integers(0, 1000, 30000)
+    got = host(D.sort_keys(ctx, [dev(ctx, key)], [0]))
+    assert np.array_equal(got, np.argsort(key, kind="stable"))
+    ucode, cnt = np.unique(key, return_counts=True)
+    (k,), (c,) = D.groupby(ctx, [dev(ctx, key)], [None], [L.AGG_COUNT])
+    assert np.array_equal(host(k), ucode) and np.array_equal(host(c), cnt)
+
+
 def test_radix_sort_pairs(ctx):
     from alenka_amd import device as D
 
