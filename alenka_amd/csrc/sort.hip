@@ -431,7 +431,7 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   __shared__ uint32_t sv[RS_TILE];
   __shared__ uint32_t wlast[RS_WAVES], wfirst[RS_WAVES], wnext[RS_WAVES], wstarts[RS_WAVES], winside[RS_WAVES];
   __shared__ uint32_t wsum[RS_WAVES];
-  __shared__ uint32_t s_long;
+  __shared__ uint32_t s_long, s_state;
   static_assert(RB_BINS == 2 * RS_TILE && RS_TILE == 4096, "bins alias sv; 12 bits of position");
   const unsigned t = threadIdx.x, lane = __lane_id(), wid = t / 64;
   const uint32_t q = a.nblk / RS_XCDS, rm = a.nblk % RS_XCDS, x = blockIdx.x % RS_XCDS;
@@ -442,11 +442,10 @@ __global__ void __launch_bounds__(RS_BLOCK) __attribute__((amdgpu_waves_per_eu(6
   // 1.17 ms by k_rs_local alone, 1.37 with every window tried, 1.28 now)
   uint32_t state = 0;
   if (blockIdx.x >= RB_RESIDENT) {
-    if (t == 0) s_long = rl_peek(a.ctl);
+    if (t == 0) s_state = rl_peek(a.ctl);
     __syncthreads();
-    state = s_long;
+    state = s_state;
     if (state & RL_OVERFLOW) return;
-    __syncthreads();
   }
   uint64_t key[RS_ITEMS];
   uint32_t val[RS_ITEMS], hi16[RS_ITEMS];
