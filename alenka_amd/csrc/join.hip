@@ -6,8 +6,8 @@
 // (operators.cu:1239-1284).  Here each probe row is looked up directly in a structure over
 // the build side:
 //   * unique build keys whose range is at most 64 per build row (the primary-key case): a
-//     table with one 8-byte entry per 32 keys (bits present, rank base) and the build rows
-//     in key order;
+//     table with one 32-byte group per 224 keys (seven words of bits present, the rank base) and
+//     the build rows in key order;
 //   * other keys: an open-addressing table keyed by MurmurHash64A (linear probing) of 16-byte
 //     entries, so that a probe step is one load: the key and the build row, or, when build
 //     keys repeat, the bounds of the key's run in the build rows sorted by table slot (a
